@@ -62,36 +62,110 @@ constexpr uint64_t kCsrMagic = 0x7472686970637372ull;  // "trhipcsr"
 
 // ------------------------------------------------------------ reductions
 
+// Lane exchanges without the LDS crossbar.  A butterfly of __shfl_xor costs
+// two ds_bpermute round trips per step (a wave_sum about 0.35 us, measured
+// in the chain kernel's phases); these are VALU moves.
+// (a, b) -> the pair whose sum is, in each lane, lo(self) + lo(partner) in
+// the lanes with bit O clear and hi(self) + hi(partner) in the others
+// (partner = lane ^ O), O = 32 or 16.
+template <int O>
+__device__ __forceinline__ double swap_sum(double lo, double hi)
+{
+    static_assert(O == 32 || O == 16, "half-wave or 16-lane rows");
+    union U {
+        double d;
+        unsigned u[2];
+    } a, b, x, y;
+    a.d = lo;
+    b.d = hi;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        if constexpr (O == 32) {
+            const auto r = __builtin_amdgcn_permlane32_swap(a.u[i], b.u[i], false, false);
+            x.u[i] = r[0];
+            y.u[i] = r[1];
+        } else {
+            const auto r = __builtin_amdgcn_permlane16_swap(a.u[i], b.u[i], false, false);
+            x.u[i] = r[0];
+            y.u[i] = r[1];
+        }
+    }
+    return x.d + y.d;
+}
+
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v)
+{
+    union U {
+        double d;
+        int i[2];
+    } a;
+    a.d = v;
+    a.i[0] = __builtin_amdgcn_update_dpp(0, a.i[0], CTRL, 0xf, 0xf, true);
+    a.i[1] = __builtin_amdgcn_update_dpp(0, a.i[1], CTRL, 0xf, 0xf, true);
+    return a.d;
+}
+
+// v of lane ^ O within a 16-lane row, O = 8, 4, 2 or 1.
+template <int O>
+__device__ __forceinline__ double row_xor(double v)
+{
+    static_assert(O == 8 || O == 4 || O == 2 || O == 1, "inside a 16-lane row");
+    if constexpr (O == 8) return dpp<0x128>(v);              // row_ror:8
+    if constexpr (O == 4) return dpp<0x1B>(dpp<0x141>(v));   // half mirror (^7), then quad_perm ^3
+    if constexpr (O == 2) return dpp<0x4E>(v);               // quad_perm [2,3,0,1]
+    return dpp<0xB1>(v);                                     // quad_perm [1,0,3,2]
+}
+
+// Wave total, the same in every lane: a butterfly over lane ^ 32, 16, ..., 1.
 __device__ __forceinline__ double wave_sum(double v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    v = swap_sum<32>(v, v);
+    v = swap_sum<16>(v, v);
+    v += row_xor<8>(v);
+    v += row_xor<4>(v);
+    v += row_xor<2>(v);
+    v += row_xor<1>(v);
     return v;
 }
 
+template <int O, int CNT, int N>
+__device__ __forceinline__ void transpose_step(double (&v)[N], int lane)
+{
+    if constexpr (CNT > 1) {
+        if constexpr (O >= 16) {
+#pragma unroll
+            for (int i = 0; i < CNT / 2; ++i) v[i] = swap_sum<O>(v[i], v[i + CNT / 2]);
+        } else {
+            const bool hi = (lane & O) != 0;
+#pragma unroll
+            for (int i = 0; i < CNT / 2; ++i) {
+                // select values, not array elements: a conditional lvalue
+                // would become a dynamically indexed (scratch) array access
+                const double lo_v = v[i], hi_v = v[i + CNT / 2];
+                const double send = hi ? lo_v : hi_v;
+                const double keep = hi ? hi_v : lo_v;
+                v[i] = keep + row_xor<O>(send);
+            }
+        }
+        transpose_step<O / 2, CNT / 2, N>(v, lane);
+    } else if constexpr (O >= 1) {
+        if constexpr (O >= 16)
+            v[0] = swap_sum<O>(v[0], v[0]);
+        else
+            v[0] += row_xor<O>(v[0]);
+        transpose_step<O / 2, 1, N>(v, lane);
+    }
+}
+
 // Transpose-reduce N per-lane values across the 64 lanes of a wave:
-// afterwards lane l holds the wave total of value index l / (64 / N).
-// Costs N-1+log2(64/N) shuffles instead of N*6.
+// afterwards lane l holds the wave total of value index l / (64 / N), with
+// wave_sum's bits.  N-1+log2(64/N) exchanges instead of N*6.
 template <int N>
 __device__ __forceinline__ double wave_transpose_sum(double (&v)[N], int lane)
 {
     static_assert(N >= 1 && N <= 64 && (N & (N - 1)) == 0, "N power of 2");
-    int o = 32;
-#pragma unroll
-    for (int cnt = N; cnt > 1; cnt >>= 1, o >>= 1) {
-        const bool hi = (lane & o) != 0;
-#pragma unroll
-        for (int i = 0; i < cnt / 2; ++i) {
-            // select values, not array elements: a conditional lvalue
-            // would become a dynamically indexed (scratch) array access
-            const double lo_v = v[i], hi_v = v[i + cnt / 2];
-            const double send = hi ? lo_v : hi_v;
-            const double keep = hi ? hi_v : lo_v;
-            v[i] = keep + __shfl_xor(send, o);
-        }
-    }
-#pragma unroll
-    for (; o > 0; o >>= 1) v[0] += __shfl_xor(v[0], o);
+    transpose_step<32, N, N>(v, lane);
     return v[0];
 }
 
