@@ -111,7 +111,7 @@ typedef struct {
     int *iwrk;                              /* 4 maxlan, index map leftovers */
     double *hx, *hy;                        /* host staging for host ops */
     const float *dstart;                    /* device FP32 start vector (batch jobs), or NULL */
-    int chain;                              /* batched real solve: most steps per round (0: 1) */
+    int chain;                              /* real device operator: most steps per chain (0: 1) */
     uint64_t rng;
     int rot_n;                              /* order of rot */
 } lz_t;
@@ -1161,9 +1161,10 @@ static void lz_iterate(lz_t *z, double *eval, double *evec, int lde, double *wrk
                 info->stat = -1111;
                 return;
             }
-            /* batched: the steps up to the next convergence test or the
-             * end of the cycle may run in this round, as long as the device
-             * sees each accepted as the solver will (trlhip_step_chain) */
+            /* the steps up to the next convergence test or the end of the
+             * cycle may run with this one (one kernel, or one round of a
+             * batch), as long as the device sees each accepted as the solver
+             * will (trlhip_step_chain) */
             if (z->chain && !z->uo && info->verbose <= 6) {
                 const int left = DMIN(DMIN(z->chain, info->klan - jnd + 1),
                                       DMAX(1, next_test - info->matvec));
@@ -1459,13 +1460,16 @@ static int lz_setup(lz_t *z, trl_matvec op, ztrl_matvec zop, trl_uo user_ortho, 
         __atomic_add_fetch(&g_ns_alloc, ta1 - ta0, __ATOMIC_RELAXED);
         __atomic_add_fetch(&g_ns_ctx, lz_ns() - ta1, __ATOMIC_RELAXED);
     }
-    /* batched real solves chain up to 8 inner steps per round (measured
+    /* a single real solve's inner steps run as chains in one kernel each
+     * where the operator allows (trlhip_step_cgs), up to the next
+     * convergence test or the end of the cycle;
+     * batched real solves chain up to 8 inner steps per round (measured
      * on the batched 2D Anderson workload: 4 steps 8,344, 6: 8,560,
      * 8: 8,667, 12: 8,408, 16: 8,445 eigenpairs/s; longer chains make the
      * host/device overlap coarser); TRLHIP_BATCH_CHAIN=k: at most k, 0 or
      * 1: one step per round */
     const char *ec = getenv("TRLHIP_BATCH_CHAIN");
-    z->chain = (b != NULL && z->A != NULL && !cplx) ? (ec ? atoi(ec) : 8) : 0;
+    z->chain = (z->A != NULL && !cplx) ? (b == NULL ? 32 : ec ? atoi(ec) : 8) : 0;
     if (z->chain < 2) z->chain = 0;
     return 1;
 }

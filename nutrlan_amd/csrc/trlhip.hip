@@ -51,6 +51,9 @@ constexpr int kRowsBlk = kBlock;       // rows per SpMV row block (at most)
 constexpr int kMinRowsUpd = 4 * kBlock;
 constexpr int kMinSpmvRowBlocks = 1;
 constexpr int kChainMax = 32;  // Lanczos steps one batched context may record per round
+// chain kernels (trl_chain.h): workgroups at most (their flags), basis
+// columns at most, the gate words after the flags, 32-bit words in all
+constexpr int kChainMaxWG = 256, kChainMaxCols = 192, kChainGate = 512, kChainSync = 640;
 constexpr uint64_t kCsrMagic = 0x7472686970637372ull;  // "trhipcsr"
 
 
@@ -1104,6 +1107,13 @@ __global__ __launch_bounds__(kBlock) void k_proj(
     proj_body<VS, RS, E, CB, RU>(n, V, ld, c0, m, r, part, gx, gy, blockIdx.x, gridDim.x);
 }
 
+// Sum of four squares, the order fixed (the kernels that form a row block's
+// norm in different code agree bit for bit).
+__device__ __forceinline__ double sumsq4(const double r[4])
+{
+    return fma(r[3], r[3], fma(r[2], r[2], fma(r[0], r[0], r[1] * r[1])));
+}
+
 // Rows row + j*kBlock (j < R) of rout = rin - Vc hs; returns the sum of
 // their |rout|^2.  Per row the products are summed into four interleaved
 // partial sums (column c into sum c mod 4 within each group of 8 columns,
@@ -1138,17 +1148,13 @@ __device__ __forceinline__ double update_rows4(int row, const VS *__restrict__ V
     }
     double ri[4], ro[4];
     load4(rin + row, ri);
-    double nrm = 0.0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        ro[j] = (double)(RS)(ri[j] - ((s[j][0] + s[j][1]) + (s[j][2] + s[j][3])));
-        nrm += ro[j] * ro[j];
-    }
+    for (int j = 0; j < 4; ++j) ro[j] = (double)(RS)(ri[j] - ((s[j][0] + s[j][1]) + (s[j][2] + s[j][3])));
     store4(rout + row, ro);
     if (ro_out)
 #pragma unroll
         for (int j = 0; j < 4; ++j) ro_out[j] = ro[j];
-    return nrm;
+    return sumsq4(ro);
 }
 
 // One complex basis entry; NT streams it (the recurrence's columns).
@@ -1650,6 +1656,7 @@ struct trlhip_csr {
     int E;          // doubles per value (complex 2)
     int nb;         // SpMV row blocks (CSR-stream kernel)
     int lpr;        // lanes per row of the vector-CSR kernel in use; 0: CSR-stream
+    int max_blk_nnz; // nonzeros of the largest row block (a longer row has a block of its own)
     int lpr_vec;    // the vector kernel's lanes per row for this matrix (0: unsuitable)
     int vgrid;      // blocks of the vector-CSR kernel
     int *rb;        // nb + 1 row-block starts
@@ -1718,6 +1725,12 @@ struct trlhip_ctx {
     // followers recorded with the last step
     int ch_budget, ch_kept, ch_ntot;  // hint: steps the solver allows (<= 1: none)
     int ch_n, ch_next;                // steps in the chain; next follower to hand out (0: none)
+    // chain kernels of a single solve (k_chain): its flags and gate words
+    // (after dscal's scalars), the flag value used so far, the gate word in
+    // turn, and whether a gate has closed (the ordinary kernels from then on)
+    unsigned *sync;
+    unsigned sync_base;
+    int gate_parity, chain_off;
     int ch_copy_ok;                   // that follower's fused normalisation was claimed
     int ch_qa[kChainMax], ch_qb[kChainMax], ch_rcol[kChainMax], ch_jnd[kChainMax];
 };
@@ -1967,8 +1980,10 @@ size_t hres_chain(int ncols) { return 8 + 3 * (size_t)(ncols + 1); }
 constexpr int kHresNorm = 4;  // a batched column norm (OP_NORM)
 // host-coherent results: a step's 4 scalars, 3 per refined pair from index
 // 8, then 7 per chain follower from hres_chain (alpha, ||r||^2, ||h||^2,
-// ||r - V h||^2, go, 1/beta, beta)
-size_t hres_count(int ncols) { return hres_chain(ncols) + 7 * (size_t)kChainMax; }
+// ||r - V h||^2, go, 1/beta, beta), then a chain kernel's recurrence
+// coefficients from hres_coef
+size_t hres_coef(int ncols) { return hres_chain(ncols) + 7 * (size_t)kChainMax; }
+size_t hres_count(int ncols) { return hres_coef(ncols) + (size_t)ncols + 2; }
 size_t part_need(int E, int ncols)
 {
     return (size_t)kSpmvGrid + 2 * (size_t)kMaxGrid + (size_t)kProjGrid * E * (ncols + 1) + 64;
@@ -2021,6 +2036,34 @@ int spmv_grid(const trlhip_csr *A)
 bool recproj_ok(const trlhip_ctx *c)
 {
     return c->E == 1 && (long)c->n <= (long)kMaxGrid * kMinRowsUpd;
+}
+
+// Row waves (256 rows each) per workgroup of a chain kernel.  The stencil
+// kernels take 4 above 32,768 rows: a barrier among 64 workgroups costs 2.7
+// us against 1.6 among 32, which outweighs the shorter phases of smaller
+// workgroups (181^2 sites, mixed: 9.2 ms a solve with 4, 9.9 with 2; 100^2
+// sites: 6.5 with 4, 6.4 with 2).  The CSR kinds keep 2: with 4, their
+// prefetched nonzeros no longer fit the 128 registers a thread of 16 waves
+// has (n = 50,001, 17 nonzeros a row: the product takes 30 us against 16).
+int chain_rw(const trlhip_csr *A) { return spmv_kind(A) <= -2 && A->n > 32768 ? 4 : 2; }
+int chain_wgs(const trlhip_csr *A) { return (A->n + 256 * chain_rw(A) - 1) / (256 * chain_rw(A)); }
+
+// Whether a step of a single solve runs as a chain kernel: real solves with
+// a stencil or CSR-stream operator whose workgroups fit kChainMaxWG (n <=
+// 262,144 for stencils, 131,072 else) and, for CSR, at most kChainCsrIter
+// row blocks a thread group (denser operators keep the wider SpMV kernel).
+// Against the single-step kernels, per solve: n = 1,000 9.3 -> 5.1 ms, n =
+// 10,000 (2D) 11.7 -> 6.4, n = 62,500 16.7 -> 9.9, n = 262,144 24.9 -> 23.3;
+// random rows n = 50,001 69 -> 48 ms.
+constexpr int kChainCsrIter = 4;
+bool chain_fits(const trlhip_ctx *c, const trlhip_csr *A, int jnd)
+{
+    if (!A || c->batch || c->E != 1 || c->chain_off || A->lpr || A->pn_on || jnd > kChainMaxCols) return false;
+    const int g = chain_wgs(A);
+    if (g > kChainMaxWG || A->nb > kSpmvGrid) return false;
+    if (spmv_kind(A) <= -2) return true;
+    const int groups = g * chain_rw(A);
+    return A->max_blk_nnz <= kNnzBlk && (A->nb + groups - 1) / groups <= kChainCsrIter;
 }
 
 // Workgroups of the stencil SpMV: kStRB row blocks each (one alpha partial
@@ -2631,6 +2674,8 @@ __device__ __forceinline__ bool chain_go(double alpha, double rr2, double hh, do
     if (rnrm <= DBL_EPSILON * fabs(alpha)) return false;
     return true;
 }
+
+#include "trl_chain.h"
 
 // Both norms of a step (before and after its speculative Gram-Schmidt
 // pass), in one block per request: the same fixed-order sums k_sum2 forms,
@@ -3638,6 +3683,8 @@ int trlhip_csr_create(trlhip_csr **out, int n, long nnz, const int *row_ptr, con
     A->E = vtype == TRLHIP_C128 ? 2 : 1;
     const std::vector<int> rb = row_blocks(n, row_ptr);
     A->nb = (int)rb.size() - 1;
+    for (int b = 0; b < A->nb; ++b)
+        A->max_blk_nnz = std::max(A->max_blk_nnz, row_ptr[rb[b + 1]] - row_ptr[rb[b]]);
     choose_spmv(A, row_ptr);
     const size_t nz1 = (size_t)(nnz > 0 ? nnz : 1);
     int rc = 0;
@@ -3985,7 +4032,9 @@ int trlhip_ctx_create_batched(trlhip_ctx **out, int n, int ncols, int vtype, trl
         rc = TRLHIP_ENOMEM;
     if (!rc && c->V32 && hipMemsetAsync(c->V32, 0, sbytes, c->s) != hipSuccess) rc = TRLHIP_EHIP;
     if (!rc) rc = ensure_part(c, part_need(c->E, ncols));
-    if (!rc && hipMalloc((void **)&c->dscal, sizeof(double) * 16) != hipSuccess) rc = TRLHIP_ENOMEM;
+    const size_t scbytes = sizeof(double) * 16 + sizeof(unsigned) * kChainSync;
+    if (!rc && hipMalloc((void **)&c->dscal, scbytes) != hipSuccess) rc = TRLHIP_ENOMEM;
+    if (!rc) c->sync = reinterpret_cast<unsigned *>(c->dscal + 16);
     if (!rc && hipMalloc((void **)&c->dcoef, sizeof(double) * ncoef) != hipSuccess) rc = TRLHIP_ENOMEM;
     if (!rc && hipMalloc((void **)&c->dh, sizeof(double) * ncoef) != hipSuccess) rc = TRLHIP_ENOMEM;
     if (!rc && hipHostMalloc((void **)&c->hbuf, sizeof(double) * c->hcap, 0) != hipSuccess) rc = TRLHIP_ENOMEM;
@@ -3994,7 +4043,7 @@ int trlhip_ctx_create_batched(trlhip_ctx **out, int n, int ncols, int vtype, trl
         rc = TRLHIP_ENOMEM;
     if (!rc && hipHostGetDevicePointer((void **)&c->dres, c->hres, 0) != hipSuccess) rc = TRLHIP_EHIP;
     if (!rc && hipMemsetAsync(c->V, 0, vbytes, c->s) != hipSuccess) rc = TRLHIP_EHIP;
-    if (!rc && hipMemsetAsync(c->dscal, 0, sizeof(double) * 16, c->s) != hipSuccess) rc = TRLHIP_EHIP;
+    if (!rc && hipMemsetAsync(c->dscal, 0, scbytes, c->s) != hipSuccess) rc = TRLHIP_EHIP;
     if (!rc && hipStreamSynchronize(c->s) != hipSuccess) rc = TRLHIP_EHIP;
     if (rc) {
         trlhip_ctx_destroy(c);
@@ -4243,6 +4292,115 @@ int trlhip_restart_step(trlhip_ctx *c, const trlhip_csr *A, int qa, const double
     return 0;
 }
 
+// Runs a step and up to K - 1 followers of a single real solve as one
+// kernel (k_chain); sets the followers up as a batch's recorded chain does.
+// Returns 1 when the step ran, 0 when it must run as ordinary kernels (the
+// gate closed: the device is filled by other work, so the context keeps to
+// them from then on), or an error.
+static int run_chain(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int qb, double beta_prev,
+                     const double *beta, int jnd, int rcol, int K)
+{
+    ChainArgs q{};
+    const int rw = chain_rw(A);
+    q.n = c->n;
+    q.g = chain_wgs(A);
+    q.steps = K;
+    q.first = first;
+    q.qa = qa;
+    q.qb = first ? -1 : qb;
+    q.rcol = rcol;
+    q.jnd = jnd;
+    q.kept = c->ch_kept;
+    q.ntot = c->ch_ntot;
+    q.kind = spmv_kind(A);
+    q.nb = A->nb;
+    q.L = A->st_L;
+    q.off = A->st_off;
+    q.ld = c->ld;
+    q.beta_prev = beta_prev;
+    q.eps = c->V32 ? (double)FLT_EPSILON : DBL_EPSILON;
+    if (c->pend_dst == qa && rcol != c->pend_src) {
+        q.x = colp<double>(c, c->pend_src);
+        q.xscale = c->pend_s;
+        q.store_q = 1;
+    } else {
+        if (int rc = settle(c)) return rc;
+        q.x = colp<double>(c, qa);
+        q.xscale = 1.0;
+    }
+    q.V = colp<double>(c, 0);
+    q.V32 = c->V32;
+    q.scratch = colp<double>(c, c->ncols);
+    q.dg = A->dg;
+    q.val = A->val;
+    q.tab = A->tab;
+    q.rb = A->rb;
+    q.rp = A->rp;
+    q.ci = A->ci;
+    q.pk = A->pk;
+    q.part_alpha = part_alpha(c);
+    q.part_recur = part_recur(c);
+    q.part_update = part_update(c);
+    q.part_proj = part_proj(c);
+    if (first) memcpy(c->hres + hres_coef(c->ncols), beta, sizeof(double) * (size_t)(jnd - 1));
+    q.coef = c->dres + hres_coef(c->ncols);
+    q.hm = c->dres;
+    q.hchain = c->dres + hres_chain(c->ncols);
+    q.sync = c->sync;
+    q.base = c->sync_base;
+    q.parity = c->gate_parity;
+    c->hres[6] = 0.0;
+    for (int k = 1; k < K; ++k) c->hres[hres_chain(c->ncols) + 7 * (size_t)(k - 1) + 4] = 0.0;
+    {
+        // the chain's bytes if every step runs
+        double bytes = 0.0;
+        for (int k = 0; k < K; ++k)
+            bytes += spmv_bytes(A, 1, 8, 8) + ((c->V32 ? 8.0 : 16.0) * (jnd + k) + 40.0) * c->n;
+        Timed t(TRLHIP_K_MISC, c->s, bytes);
+#define CHAIN_LAUNCH(RW, KIND)                                                                 \
+    do {                                                                                       \
+        if (c->V32)                                                                            \
+            KLAUNCH((k_chain<RW, KIND, float>), dim3(q.g), dim3(256 * RW), 0, c->s, q);         \
+        else                                                                                   \
+            KLAUNCH((k_chain<RW, KIND, double>), dim3(q.g), dim3(256 * RW), 0, c->s, q);        \
+    } while (0)
+        switch (q.kind) {
+        case -3:
+            if (rw == 4) CHAIN_LAUNCH(4, -3);
+            else CHAIN_LAUNCH(2, -3);
+            break;
+        case -2:
+            if (rw == 4) CHAIN_LAUNCH(4, -2);
+            else CHAIN_LAUNCH(2, -2);
+            break;
+        case -1: CHAIN_LAUNCH(2, -1); break;
+        default: CHAIN_LAUNCH(2, 0); break;
+        }
+#undef CHAIN_LAUNCH
+        if (hipGetLastError() != hipSuccess) return TRLHIP_EHIP;
+    }
+    c->sync_base += 3u * (unsigned)K + 1u;
+    c->gate_parity ^= 1;
+    if (int rc = ctx_wait(c)) return rc;
+    const double status = *(const volatile double *)(c->hres + 6);
+    if (status == 2.0) {
+        c->chain_off = 1;
+        return 0;
+    }
+    if (status != 1.0) return TRLHIP_EHIP;
+    if (q.store_q) c->pend_dst = -1;
+    for (int k = 1; k < K; ++k) {
+        c->ch_qa[k] = rcol + k - 1;
+        c->ch_qb[k] = k >= 2 ? rcol + k - 2 : qa;
+        c->ch_rcol[k] = rcol + k;
+        c->ch_jnd[k] = jnd + k;
+    }
+    c->ch_n = K;
+    c->ch_next = K > 1 ? 1 : 0;
+    c->ch_copy_ok = 0;
+    return 1;
+}
+
 int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int qb,
                     double beta_prev, const double *beta, int jnd, int rcol, double out[4])
 {
@@ -4325,6 +4483,22 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
         return 0;
     }
     if (int rc = batch_drain(c)) return rc;
+    int K = first ? 1 : std::max(1, std::min(c->ch_budget, kChainMax));
+    c->ch_budget = 0;
+    if (chain_fits(c, A, jnd)) {
+        while (K > 1 && (!valid_col(c, rcol + K - 1) || jnd + K - 1 > c->ncols || jnd + K - 1 > kChainMaxCols))
+            --K;
+        const int ran = run_chain(c, A, first, qa, qb, beta_prev, beta, jnd, rcol, K);
+        if (ran < 0) return ran;
+        if (ran) {
+            const volatile double *hr = c->hres;
+            out[0] = hr[S_ALPHA];
+            out[1] = hr[S_RR2];
+            out[2] = hr[S_HH];
+            out[3] = hr[S_RR2B];
+            return 0;
+        }
+    }
     int rc;
     if (recproj_ok(c)) {
         // SpMV, then the recurrence fused with the first projection
@@ -4388,7 +4562,7 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
 int trlhip_step_chain(trlhip_ctx *c, int steps, int kept, int ntot)
 {
     if (!c) return TRLHIP_EINVAL;
-    if (!c->batch || c->E != 1) return 0;  // chains are a batched-step device layout
+    if (c->E != 1) return 0;
     c->ch_budget = steps;
     c->ch_kept = kept;
     c->ch_ntot = ntot;
