@@ -15,6 +15,16 @@
 // MFMA f32 16x16x32 bf16 operand layout (lane l): A row l%16 with K
 // elements 8*(l/16) .. +7, B column l%16 with the same K elements, result
 // D[4*(l/16) + i][l%16] in accumulator element i.
+//
+// A wave takes a strip of 16 pixels of one image row and walks down kRows
+// rows: each input row is loaded once (three column shifts) and feeds the
+// three output rows that use it, the layer's weights stay in registers, and
+// the weights are the A operand, so a lane holds four consecutive channels
+// of one pixel and stores them together.  What bounds the forward is the
+// activations' HBM traffic; with nine loads a pixel, weights re-read per 16
+// pixels and two-byte stores a 32 -> 32 layer took 0.89 ms for 7.3 M pixels
+// (256 lattices, sides 64-256; 0.94 GB, 0.19 ms at copy rate), now 0.37; the
+// first and last layers 0.54 and 0.44, now 0.18 each.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -33,7 +43,8 @@ namespace {
 constexpr int C = 32;          // hidden channels
 constexpr int T = 9;           // 3x3 taps
 constexpr int NB = 256;        // threads per block
-constexpr int PIX_BLK = 64;    // pixels per block (4 waves x 16)
+constexpr int kStrip = 16;     // pixels of a row per wave
+constexpr int kRows = 8;       // rows a wave walks
 
 // parameter offsets in the flat FP32 vector
 constexpr int OW1 = 0, OB1 = OW1 + C * T;             // W1[co][t]
@@ -69,37 +80,6 @@ struct Geo {
     long np;  // pixels
 };
 
-// pixel p shifted by tap t (dy = t/3 - 1, dx = t%3 - 1; sign -1 inverts), periodic
-__device__ inline long nbr(const Geo &g, long p, int t, int sign)
-{
-    const int dy = sign * (t / 3 - 1), dx = sign * (t % 3 - 1);
-    const long hw = (long)g.h * g.w;
-    const long img = p / hw;
-    const int r = (int)(p - img * hw);
-    int y = r / g.w + dy, x = r % g.w + dx;
-    y = y < 0 ? y + g.h : (y >= g.h ? y - g.h : y);
-    x = x < 0 ? x + g.w : (x >= g.w ? x - g.w : x);
-    return img * hw + (long)y * g.w + x;
-}
-
-// The 9 neighbours of pixel p (tap t = (dy+1)*3 + dx+1, periodic), with
-// one division per pixel instead of one per tap: nb[t] equals nbr(g, p, t, 1).
-__device__ inline void nbr9(const Geo &g, long p, long nb[9])
-{
-    const long hw = (long)g.h * g.w;
-    const long img = p / hw;
-    const int r = (int)(p - img * hw);
-    const int y = r / g.w, x = r - y * g.w;
-    const int ym = y == 0 ? g.h - 1 : y - 1, yp = y == g.h - 1 ? 0 : y + 1;
-    const int xm = x == 0 ? g.w - 1 : x - 1, xp = x == g.w - 1 ? 0 : x + 1;
-    const long base = img * hw;
-    const int ys[3] = {ym, y, yp}, xs[3] = {xm, x, xp};
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int b = 0; b < 3; ++b) nb[a * 3 + b] = base + (long)ys[a] * g.w + xs[b];
-}
-
 __device__ inline bf16x8 load8(const bf16_t *p)
 {
     const uint4 v = *reinterpret_cast<const uint4 *>(p);
@@ -108,41 +88,101 @@ __device__ inline bf16x8 load8(const bf16_t *p)
 
 __device__ inline bf16x8 zero8() { return __builtin_bit_cast(bf16x8, uint4{0, 0, 0, 0}); }
 
+// Wave tasks of a convolution: strips x row segments of every image.
+__host__ __device__ inline int strips_of(int w) { return (w + kStrip - 1) / kStrip; }
+__host__ __device__ inline int segs_of(int h) { return (h + kRows - 1) / kRows; }
+__host__ __device__ inline long conv_tasks(const Geo &g) { return (long)g.nimg * strips_of(g.w) * segs_of(g.h); }
+inline long conv_blocks(const Geo &g) { return (conv_tasks(g) + NB / 64 - 1) / (NB / 64); }
+
+// A wave's strip: its image's first pixel, columns, rows [y0, y1).
+struct Strip {
+    long base;
+    int x, xc[3], y0, y1;  // the lane's column, its neighbours' (periodic), the rows
+    bool ok;               // the lane's column exists (others repeat the last one)
+};
+
+__device__ __forceinline__ bool strip_of(const Geo &g, long task, Strip &s)
+{
+    if (task >= conv_tasks(g)) return false;
+    const int ns = strips_of(g.w), per = ns * segs_of(g.h);
+    const int img = (int)(task / per), r = (int)(task - (long)img * per);
+    const int seg = r / ns, strip = r - seg * ns;
+    const int x = strip * kStrip + (int)(threadIdx.x & 15);
+    s.ok = x < g.w;
+    s.x = s.ok ? x : g.w - 1;
+    s.xc[0] = s.x == 0 ? g.w - 1 : s.x - 1;
+    s.xc[1] = s.x;
+    s.xc[2] = s.x == g.w - 1 ? 0 : s.x + 1;
+    s.base = (long)img * g.h * g.w;
+    s.y0 = seg * kRows;
+    s.y1 = s.y0 + kRows < g.h ? s.y0 + kRows : g.h;
+    return true;
+}
+
+__device__ __forceinline__ int wrap(int y, int h) { return y < 0 ? y + h : (y >= h ? y - h : y); }
+
+__device__ __forceinline__ uint2 pack4(const float v[4])
+{
+    return uint2{(uint32_t)f2bf(v[0]) | (uint32_t)f2bf(v[1]) << 16,
+                 (uint32_t)f2bf(v[2]) | (uint32_t)f2bf(v[3]) << 16};
+}
+
 // ---------------------------------------------------------------- forward
 
 // Layer 1: one input channel (FP32 potential, rounded to BF16), K = the 9
-// taps padded to 32.  out = relu(W1 * x + b1), BF16, 32 channels.
+// taps padded to 32.  out = relu(W1 * x + b1), BF16, 32 channels.  The
+// wave's three input rows slide down in registers.
 __device__ __forceinline__ void fwd1_body(const Geo &g, long bid, const float *__restrict__ x,
                                           const bf16_t *__restrict__ w1, const float *__restrict__ b1,
                                           bf16_t *__restrict__ out)
 {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const long p0 = (bid * 4 + wv) * 16;
-    if (p0 >= g.np) return;
+    const int lane = threadIdx.x & 63;
+    Strip s;
+    if (!strip_of(g, bid * (NB / 64) + (threadIdx.x >> 6), s)) return;
     const int m = lane & 15, kq = lane >> 4;
-    const long p = p0 + m;
-    bf16x8 a = zero8();
-    if (p < g.np) {
-        long nb[9];
-        nbr9(g, p, nb);
+    bf16x8 wt[2];
+    float bs[2][4];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int t = 8 * kq + j;
-            if (t < T) a[j] = as_bf(f2bf(x[nb[t]]));
-        }
-    }
     for (int nt = 0; nt < 2; ++nt) {
-        const int co = 16 * nt + m;
-        bf16x8 b = zero8();
-        for (int j = 0; j < 8; ++j) {
-            const int t = 8 * kq + j;
-            if (t < T) b[j] = as_bf(w1[co * T + t]);
+        wt[nt] = zero8();
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (8 * kq + j < T) wt[nt][j] = as_bf(w1[(16 * nt + m) * T + 8 * kq + j]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bs[nt][i] = b1[16 * nt + 4 * kq + i];
+    }
+    const float *xi = x + s.base;
+    auto row = [&](int y, __bf16 r[3]) {
+        const float *p = xi + (long)wrap(y, g.h) * g.w;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) r[d] = as_bf(f2bf(p[s.xc[d]]));
+    };
+    __bf16 r0[3], r1[3], r2[3];
+    row(s.y0 - 1, r0);
+    row(s.y0, r1);
+    const __bf16 z = as_bf(0);
+    for (int y = s.y0; y < s.y1; ++y) {
+        row(y + 1, r2);
+        // taps 0..7 in the lanes of K 0..7, tap 8 in those of K 8..15
+        bf16x8 a = zero8();
+        const __bf16 t8[8] = {r0[0], r0[1], r0[2], r1[0], r1[1], r1[2], r2[0], r2[1]};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[j] = kq == 0 ? t8[j] : z;
+        if (kq == 1) a[0] = r2[2];
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            f4 acc = {0.f, 0.f, 0.f, 0.f};
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[nt], a, acc, 0, 0, 0);
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = fmaxf(acc[i] + bs[nt][i], 0.f);
+            if (s.ok)
+                *reinterpret_cast<uint2 *>(out + (s.base + (long)y * g.w + s.x) * C + 16 * nt + 4 * kq) = pack4(v);
         }
-        f4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-        for (int i = 0; i < 4; ++i) {
-            const long q = p0 + 4 * kq + i;
-            if (q < g.np) out[q * C + co] = f2bf(fmaxf(acc[i] + b1[co], 0.f));
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            r0[d] = r1[d];
+            r1[d] = r2[d];
         }
     }
 }
@@ -154,34 +194,81 @@ __global__ __launch_bounds__(NB) void k_fwd1(Geo g, const float *__restrict__ x,
     fwd1_body(g, blockIdx.x, x, w1, b1, out);
 }
 
-// Layers 2 and 3: 32 -> 32 channels, K = 9 taps x 32 channels.
-__device__ __forceinline__ void fwd32_body(const Geo &g, long bid, const bf16_t *__restrict__ in,
-                                           const bf16_t *__restrict__ w, const float *__restrict__ bias,
-                                           bf16_t *__restrict__ out)
+// A 32 -> 32 channel 3x3 convolution over a wave's strip, K = 9 taps x 32
+// channels: forward (BWD = false: out = relu(W * in + bias)) or the data
+// gradient (BWD: out = relu'(act) * W^T * in, taps mirrored, w transposed).
+// Rows are walked so that each output row receives its taps in order 0..8:
+// downwards, or upwards for the mirrored taps.  Input row r is the first
+// tap row of the output row after it, the middle of its own and the last of
+// the one before, so three rows of accumulators are open at a time.
+template <bool BWD>
+__device__ __forceinline__ void conv32_body(const Geo &g, long bid, const bf16_t *__restrict__ in,
+                                            const bf16_t *__restrict__ w, const float *__restrict__ bias,
+                                            const bf16_t *__restrict__ act, bf16_t *__restrict__ out)
 {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const long p0 = (bid * 4 + wv) * 16;
-    if (p0 >= g.np) return;
+    const int lane = threadIdx.x & 63;
+    Strip s;
+    if (!strip_of(g, bid * (NB / 64) + (threadIdx.x >> 6), s)) return;
     const int m = lane & 15, kq = lane >> 4;
-    const long p = p0 + m;
-    f4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    long nb[9];
-    if (p < g.np) nbr9(g, p, nb);
+    bf16x8 wt[T][2];
 #pragma unroll
-    for (int t = 0; t < T; ++t) {
-        const bf16x8 a = p < g.np ? load8(in + nb[t] * C + 8 * kq) : zero8();
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) wt[t][nt] = load8(w + ((long)(16 * nt + m) * T + t) * C + 8 * kq);
+    float bs[2][4];
+    if constexpr (!BWD)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bs[nt][i] = bias[16 * nt + 4 * kq + i];
+    const bf16_t *pi = in + s.base * C + 8 * kq;
+    const int nr = s.y1 - s.y0;
+    // step k loads input row y0 - 1 + k, or y1 - k
+    auto row = [&](int k) { return BWD ? s.y1 - k : s.y0 - 1 + k; };
+    auto load = [&](int k, bf16x8 a[3]) {
+        const bf16_t *p = pi + (long)wrap(row(k), g.h) * g.w * C;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) a[d] = load8(p + s.xc[BWD ? 2 - d : d] * C);
+    };
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+    f4 mid[2] = {zero, zero}, last[2] = {zero, zero};  // output rows k - 1 (middle taps next), k - 2
+    bf16x8 a[3], nx[3];
+    load(0, a);
+    for (int k = 0; k < nr + 2; ++k) {
+        if (k + 1 < nr + 2) load(k + 1, nx);
+        f4 first[2] = {zero, zero};
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                first[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[d][nt], a[d], first[nt], 0, 0, 0);
+                mid[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[3 + d][nt], a[d], mid[nt], 0, 0, 0);
+                last[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[6 + d][nt], a[d], last[nt], 0, 0, 0);
+            }
+        if (k >= 2 && s.ok) {
+            const long q = (s.base + (long)(BWD ? row(k) + 1 : row(k) - 1) * g.w + s.x) * C + 4 * kq;
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt) {
+                float v[4];
+                if constexpr (BWD) {
+                    const uint2 av = *reinterpret_cast<const uint2 *>(act + q + 16 * nt);
+                    const uint32_t h[4] = {av.x & 0xFFFFu, av.x >> 16, av.y & 0xFFFFu, av.y >> 16};
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[i] = last[nt][i] * (bf2f((bf16_t)h[i]) > 0.f ? 1.f : 0.f);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[i] = fmaxf(last[nt][i] + bs[nt][i], 0.f);
+                }
+                *reinterpret_cast<uint2 *>(out + q + 16 * nt) = pack4(v);
+            }
+        }
+#pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
-            const int co = 16 * nt + m;
-            const bf16x8 b = load8(w + ((long)co * T + t) * C + 8 * kq);
-            acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[nt], 0, 0, 0);
+            last[nt] = mid[nt];
+            mid[nt] = first[nt];
         }
-    }
-    for (int nt = 0; nt < 2; ++nt) {
-        const int co = 16 * nt + m;
-        for (int i = 0; i < 4; ++i) {
-            const long q = p0 + 4 * kq + i;
-            if (q < g.np) out[q * C + co] = f2bf(fmaxf(acc[nt][i] + bias[co], 0.f));
-        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) a[d] = nx[d];
     }
 }
 
@@ -189,33 +276,49 @@ __global__ __launch_bounds__(NB) void k_fwd32(Geo g, const bf16_t *__restrict__ 
                                               const bf16_t *__restrict__ w, const float *__restrict__ bias,
                                               bf16_t *__restrict__ out)
 {
-    fwd32_body(g, blockIdx.x, in, w, bias, out);
+    conv32_body<false>(g, blockIdx.x, in, w, bias, nullptr, out);
 }
 
-// Layer 4: 32 -> 1 channel (N padded to 16, column 0 real), FP32 output.
+// Layer 4: 32 -> 1 channel (M padded to 16, row 0 real), FP32 output; rows
+// walked as in conv32_body.
 __device__ __forceinline__ void fwd4_body(const Geo &g, long bid, const bf16_t *__restrict__ in,
                                           const bf16_t *__restrict__ w4, const float *__restrict__ b4,
                                           float *__restrict__ out)
 {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const long p0 = (bid * 4 + wv) * 16;
-    if (p0 >= g.np) return;
+    const int lane = threadIdx.x & 63;
+    Strip s;
+    if (!strip_of(g, bid * (NB / 64) + (threadIdx.x >> 6), s)) return;
     const int m = lane & 15, kq = lane >> 4;
-    const long p = p0 + m;
-    f4 acc = {0.f, 0.f, 0.f, 0.f};
-    long nb[9];
-    if (p < g.np) nbr9(g, p, nb);
+    bf16x8 wt[T];
 #pragma unroll
-    for (int t = 0; t < T; ++t) {
-        const bf16x8 a = p < g.np ? load8(in + nb[t] * C + 8 * kq) : zero8();
-        const bf16x8 b = m == 0 ? load8(w4 + (long)t * C + 8 * kq) : zero8();
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-    }
-    if (m == 0)
-        for (int i = 0; i < 4; ++i) {
-            const long q = p0 + 4 * kq + i;
-            if (q < g.np) out[q] = acc[i] + b4[0];
+    for (int t = 0; t < T; ++t) wt[t] = m == 0 ? load8(w4 + (long)t * C + 8 * kq) : zero8();
+    const float bias = b4[0];
+    const bf16_t *pi = in + s.base * C + 8 * kq;
+    const int nr = s.y1 - s.y0;
+    auto load = [&](int k, bf16x8 a[3]) {
+        const bf16_t *p = pi + (long)wrap(s.y0 - 1 + k, g.h) * g.w * C;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) a[d] = load8(p + s.xc[d] * C);
+    };
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+    f4 mid = zero, last = zero;
+    bf16x8 a[3], nx[3];
+    load(0, a);
+    for (int k = 0; k < nr + 2; ++k) {
+        if (k + 1 < nr + 2) load(k + 1, nx);
+        f4 first = zero;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            first = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[d], a[d], first, 0, 0, 0);
+            mid = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[3 + d], a[d], mid, 0, 0, 0);
+            last = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[6 + d], a[d], last, 0, 0, 0);
         }
+        if (k >= 2 && s.ok && kq == 0) out[s.base + (long)(s.y0 + k - 2) * g.w + s.x] = last[0] + bias;
+        last = mid;
+        mid = first;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) a[d] = nx[d];
+    }
 }
 
 __global__ __launch_bounds__(NB) void k_fwd4(Geo g, const bf16_t *__restrict__ in,
@@ -266,7 +369,7 @@ __global__ __launch_bounds__(NB) void k_fwd32_many(const GroupGeo *__restrict__ 
 {
     const int i = group_of(pre, ng, blockIdx.x);
     const GroupGeo q = gg[i];
-    fwd32_body(q.g, blockIdx.x - pre[i], in + q.off * C, w, bias, out + q.off * C);
+    conv32_body<false>(q.g, blockIdx.x - pre[i], in + q.off * C, w, bias, nullptr, out + q.off * C);
 }
 
 __global__ __launch_bounds__(NB) void k_fwd4_many(const GroupGeo *__restrict__ gg, const int *__restrict__ pre,
@@ -316,36 +419,59 @@ __global__ __launch_bounds__(NB) void k_loss(Geo g, const float *__restrict__ o,
 }
 
 // dX for layer 4's input: dA3[p][ci] = relu'(a3[p][ci]) * sum_t dO[nbr(p,-t)] W4[t][ci].
-// K = the 9 taps padded to 32 (one output channel), N = 32 input channels.
+// K = the 9 taps padded to 32 (one output channel), M = 32 input channels;
+// the three rows of dO slide down in registers (tap 0 reads the row below).
 __global__ __launch_bounds__(NB) void k_bwd4(Geo g, const float *__restrict__ dout,
                                              const bf16_t *__restrict__ w4, const bf16_t *__restrict__ a3,
                                              bf16_t *__restrict__ da3)
 {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const long p0 = ((long)blockIdx.x * 4 + wv) * 16;
-    if (p0 >= g.np) return;
+    const int lane = threadIdx.x & 63;
+    Strip s;
+    if (!strip_of(g, (long)blockIdx.x * (NB / 64) + (threadIdx.x >> 6), s)) return;
     const int m = lane & 15, kq = lane >> 4;
-    const long p = p0 + m;
-    bf16x8 a = zero8();
-    for (int j = 0; j < 8; ++j) {
-        const int t = 8 * kq + j;
-        if (t < T && p < g.np) a[j] = as_bf(f2bf(dout[nbr(g, p, t, -1)]));
-    }
+    bf16x8 wt[2];
+#pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
-        const int ci = 16 * nt + m;
-        bf16x8 b = zero8();
-        for (int j = 0; j < 8; ++j) {
-            const int t = 8 * kq + j;
-            if (t < T) b[j] = as_bf(w4[t * C + ci]);
-        }
-        f4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-        for (int i = 0; i < 4; ++i) {
-            const long q = p0 + 4 * kq + i;
-            if (q < g.np) {
-                const float mask = bf2f(a3[q * C + ci]) > 0.f ? 1.f : 0.f;
-                da3[q * C + ci] = f2bf(acc[i] * mask);
+        wt[nt] = zero8();
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (8 * kq + j < T) wt[nt][j] = as_bf(w4[(8 * kq + j) * C + 16 * nt + m]);
+    }
+    const float *di = dout + s.base;
+    auto row = [&](int y, __bf16 r[3]) {
+        const float *p = di + (long)wrap(y, g.h) * g.w;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) r[d] = as_bf(f2bf(p[s.xc[2 - d]]));
+    };
+    __bf16 r0[3], r1[3], r2[3];  // rows y + 1, y, y - 1: taps 0..2, 3..5, 6..8
+    row(s.y0 - 1, r2);
+    row(s.y0, r1);
+    const __bf16 z = as_bf(0);
+    for (int y = s.y0; y < s.y1; ++y) {
+        row(y + 1, r0);
+        bf16x8 a = zero8();
+        const __bf16 t8[8] = {r0[0], r0[1], r0[2], r1[0], r1[1], r1[2], r2[0], r2[1]};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[j] = kq == 0 ? t8[j] : z;
+        if (kq == 1) a[0] = r2[2];
+        const long q = (s.base + (long)y * g.w + s.x) * C + 4 * kq;
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            f4 acc = {0.f, 0.f, 0.f, 0.f};
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[nt], a, acc, 0, 0, 0);
+            if (s.ok) {
+                const uint2 av = *reinterpret_cast<const uint2 *>(a3 + q + 16 * nt);
+                const uint32_t h[4] = {av.x & 0xFFFFu, av.x >> 16, av.y & 0xFFFFu, av.y >> 16};
+                float v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = acc[i] * (bf2f((bf16_t)h[i]) > 0.f ? 1.f : 0.f);
+                *reinterpret_cast<uint2 *>(da3 + q + 16 * nt) = pack4(v);
             }
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            r2[d] = r1[d];
+            r1[d] = r0[d];
         }
     }
 }
@@ -356,84 +482,190 @@ __global__ __launch_bounds__(NB) void k_bwd32(Geo g, const bf16_t *__restrict__ 
                                               const bf16_t *__restrict__ wt, const bf16_t *__restrict__ a,
                                               bf16_t *__restrict__ da)
 {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const long p0 = ((long)blockIdx.x * 4 + wv) * 16;
-    if (p0 >= g.np) return;
-    const int m = lane & 15, kq = lane >> 4;
-    const long p = p0 + m;
-    f4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    for (int t = 0; t < T; ++t) {
-        const bf16x8 av = p < g.np ? load8(dy + nbr(g, p, t, -1) * C + 8 * kq) : zero8();
-        for (int nt = 0; nt < 2; ++nt) {
-            const int ci = 16 * nt + m;
-            const bf16x8 b = load8(wt + ((long)ci * T + t) * C + 8 * kq);
-            acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, b, acc[nt], 0, 0, 0);
-        }
-    }
-    for (int nt = 0; nt < 2; ++nt) {
-        const int ci = 16 * nt + m;
-        for (int i = 0; i < 4; ++i) {
-            const long q = p0 + 4 * kq + i;
-            if (q < g.np) {
-                const float mask = bf2f(a[q * C + ci]) > 0.f ? 1.f : 0.f;
-                da[q * C + ci] = f2bf(acc[nt][i] * mask);
-            }
-        }
+    conv32_body<true>(g, blockIdx.x, dy, wt, nullptr, a, da);
+}
+
+// ------------------------------------------------------- weight gradients
+//
+// K = pixels, so both operands are needed pixel-contiguous per channel while
+// the activations are channel-last.  Each wave transposes its own pixels
+// through LDS: 32 pixels of a row x 32 channels are loaded with 16-byte
+// loads, two pixels' channels interleaved by v_perm into dwords [channel]
+// [pixel pair], and read back 8 pixels a lane.  Rows of kTr = 18 dwords put
+// the writes of a wave on 64 different banks.  A wave walks down a strip of
+// 32 x kDwRows pixels and keeps its accumulators over all its strips.
+// Gathering the operands two bytes at a time with a division per pixel and
+// tap, the two layers took 330 us each at 64 images of 64 x 64 (now 19), and
+// the first and last layers, one thread per weight over a serial pixel loop,
+// 650 us each (now 17).
+constexpr int kDwW = 32, kDwRows = 8;
+constexpr int kTr = 18;               // dwords per channel: 36 pixels
+constexpr int kDwBlocks = 256;        // blocks (4 waves each, a partial per wave)
+
+__host__ __device__ inline long dw_tasks(const Geo &g)
+{
+    return (long)g.nimg * ((g.w + kDwW - 1) / kDwW) * ((g.h + kDwRows - 1) / kDwRows);
+}
+
+struct DwStrip {
+    long base;
+    int x0, y0, y1;
+};
+
+__device__ __forceinline__ DwStrip dw_strip(const Geo &g, long task)
+{
+    const int ns = (g.w + kDwW - 1) / kDwW, per = ns * ((g.h + kDwRows - 1) / kDwRows);
+    const int img = (int)(task / per), r = (int)(task - (long)img * per);
+    const int seg = r / ns;
+    DwStrip s;
+    s.base = (long)img * g.h * g.w;
+    s.x0 = (r - seg * ns) * kDwW;
+    s.y0 = seg * kDwRows;
+    s.y1 = s.y0 + kDwRows < g.h ? s.y0 + kDwRows : g.h;
+    return s;
+}
+
+// Column x0 + p of a row of w, periodic one pixel beyond either end; further
+// out (a ragged strip's unused pixels) any column.
+__device__ __forceinline__ int dw_col(int x, int w)
+{
+    x = x < 0 ? x + w : (x >= w ? x - w : x);
+    return x < w ? x : 0;
+}
+
+// The lane's two pixels (2 pp, 2 pp + 1 after `x`) of row `row`, 8 channels.
+struct Pair {
+    uint4 a, b;
+};
+
+// Two pixels' 8 channels as 8 dwords [pixel 1 | pixel 0], to rows 8 cg + c.
+__device__ __forceinline__ void put_pair(uint32_t *tr, int cg, int dw, const Pair &v)
+{
+    const uint32_t a[4] = {v.a.x, v.a.y, v.a.z, v.a.w}, b[4] = {v.b.x, v.b.y, v.b.z, v.b.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        tr[(8 * cg + 2 * i) * kTr + dw] = __builtin_amdgcn_perm(b[i], a[i], 0x05040100u);
+        tr[(8 * cg + 2 * i + 1) * kTr + dw] = __builtin_amdgcn_perm(b[i], a[i], 0x07060302u);
     }
 }
 
-// Weight gradient dW[co][t][ci] = sum_p dY[p][co] X[nbr(p,t)][ci] for a
-// 32 -> 32 layer, K = pixels in chunks of 32 (8 per lane group), M = co,
-// N = ci.  Block b takes pixel chunks b, b + nblk, ...; its 4 waves take
-// alternate chunks; the block's partial (co, t, ci) and bias partial sums
-// go to part[b][.] and are reduced by k_reduce in block order.
+__device__ __forceinline__ bf16x8 frag(const uint32_t d[4])
+{
+    return __builtin_bit_cast(bf16x8, uint4{d[0], d[1], d[2], d[3]});
+}
+
+// Weight gradient dW[co][t][ci] = sum_p dY[p][co] X[nbr(p,t)][ci] of a
+// 32 -> 32 layer: M = co, N = ci.  Three rows of X stay in LDS (a row
+// serves the dY rows above, at and below it); a lane reads 12 pixels of a
+// channel and shifts them by one for the left and right taps.  The wave's
+// partial (co, t, ci) and bias sums (a product with ones) go to
+// part[4 blockIdx + wave].
 __global__ __launch_bounds__(NB) void k_dw32(Geo g, const bf16_t *__restrict__ dy,
                                              const bf16_t *__restrict__ x, float *__restrict__ part)
 {
     constexpr int NW = C * T * C;
+    __shared__ __align__(16) uint32_t lds[NB / 64][4][C * kTr];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int m = lane & 15, kq = lane >> 4;
-    f4 acc[T][2][2];
+    const int pp = lane >> 2, cg = lane & 3;
+    uint32_t *ty = lds[wv][3];
+    f4 acc[T][2][2], bacc[2];
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < T; ++t)
+    for (int mt = 0; mt < 2; ++mt) {
+        bacc[mt] = zero;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[t][i][j] = f4{0.f, 0.f, 0.f, 0.f};
-    float bsum[2] = {0.f, 0.f};
-    const long nchunk = (g.np + 31) / 32;
-    for (long ch = (long)blockIdx.x * 4 + wv; ch < nchunk; ch += (long)gridDim.x * 4) {
-        const long pc = ch * 32 + 8 * kq;
-        bf16x8 av[2];
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-            const int co = 16 * mt + m;
-            av[mt] = zero8();
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (pc + j < g.np) {
-                    const bf16_t h = dy[(pc + j) * C + co];
-                    av[mt][j] = as_bf(h);
-                    bsum[mt] += bf2f(h);
-                }
-        }
-#pragma unroll
-        for (int t = 0; t < T; ++t)
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                const int ci = 16 * nt + m;
-                bf16x8 bv = zero8();
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (pc + j < g.np) bv[j] = as_bf(x[nbr(g, pc + j, t, 1) * C + ci]);
-#pragma unroll
-                for (int mt = 0; mt < 2; ++mt)
-                    acc[t][mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[mt], bv, acc[t][mt][nt], 0, 0, 0);
-            }
+        for (int t = 0; t < T; ++t) acc[t][mt][0] = acc[t][mt][1] = zero;
     }
-    // combine the 4 waves through the partial buffer rows (wave w writes
-    // slot 4*b + w; the reduce kernel sums all slots in order)
-    float *out = part + ((long)blockIdx.x * 4 + wv) * (NW + C);
+    bf16x8 ones;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ones[j] = as_bf(0x3F80);
+    const uint4 z4 = {0, 0, 0, 0};
+    const long nt_ = dw_tasks(g);
+    for (long task = (long)blockIdx.x * (NB / 64) + wv; task < nt_; task += (long)gridDim.x * (NB / 64)) {
+        const DwStrip s = dw_strip(g, task);
+        const int nr = s.y1 - s.y0;
+        const int c0 = dw_col(s.x0 + 2 * pp, g.w), c1 = dw_col(s.x0 + 2 * pp + 1, g.w);
+        // the pixels just left and right of the strip, lanes 0..7
+        const int ch = dw_col(pp == 0 ? s.x0 - 1 : s.x0 + kDwW, g.w);
+        const bool y0ok = s.x0 + 2 * pp < g.w, y1ok = s.x0 + 2 * pp + 1 < g.w;
+        auto ldx = [&](int y, Pair &v, uint4 &h) {
+            const bf16_t *p = x + (s.base + (long)wrap(y, g.h) * g.w) * C + 8 * cg;
+            v.a = *reinterpret_cast<const uint4 *>(p + (long)c0 * C);
+            v.b = *reinterpret_cast<const uint4 *>(p + (long)c1 * C);
+            h = lane < 8 ? *reinterpret_cast<const uint4 *>(p + (long)ch * C) : z4;
+        };
+        auto ldy = [&](int y, Pair &v) {
+            const bf16_t *p = dy + (s.base + (long)y * g.w) * C + 8 * cg;
+            v.a = y0ok ? *reinterpret_cast<const uint4 *>(p + (long)c0 * C) : z4;
+            v.b = y1ok ? *reinterpret_cast<const uint4 *>(p + (long)c1 * C) : z4;
+        };
+        // pixel p of the strip at half-word p + 2 of a channel's row
+        auto putx = [&](int slot, const Pair &v, const uint4 &h) {
+            uint32_t *tr = lds[wv][slot];
+            put_pair(tr, cg, pp + 1, v);
+            if (lane < 8) {
+                Pair e;
+                e.a = pp == 0 ? z4 : h;
+                e.b = pp == 0 ? h : z4;
+                put_pair(tr, cg, pp == 0 ? 0 : kDwW / 2 + 1, e);
+            }
+        };
+        Pair vx, vy;
+        uint4 hx;
+        ldx(s.y0 - 1, vx, hx);
+        putx(0, vx, hx);
+        ldx(s.y0, vx, hx);
+        putx(1, vx, hx);
+        ldx(s.y0 + 1, vx, hx);
+        ldy(s.y0, vy);
+        for (int r = 0; r < nr; ++r) {
+            putx((r + 2) % 3, vx, hx);
+            put_pair(ty, cg, pp, vy);
+            if (r + 1 < nr) {
+                ldx(s.y0 + r + 2, vx, hx);
+                ldy(s.y0 + r + 1, vy);
+            }
+            __builtin_amdgcn_wave_barrier();
+            bf16x8 av[2];
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt) {
+                const uint32_t *p = ty + (16 * mt + m) * kTr + 4 * kq;
+                const uint2 lo = *reinterpret_cast<const uint2 *>(p), hi = *reinterpret_cast<const uint2 *>(p + 2);
+                const uint32_t d[4] = {lo.x, lo.y, hi.x, hi.y};
+                av[mt] = frag(d);
+                bacc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[mt], ones, bacc[mt], 0, 0, 0);
+            }
+#pragma unroll
+            for (int dyi = 0; dyi < 3; ++dyi) {
+                const uint32_t *tr = lds[wv][(r + dyi) % 3];
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt) {
+                    const uint32_t *p = tr + (16 * nt + m) * kTr + 4 * kq;
+                    const uint2 q0 = *reinterpret_cast<const uint2 *>(p);
+                    const uint2 q1 = *reinterpret_cast<const uint2 *>(p + 2);
+                    const uint2 q2 = *reinterpret_cast<const uint2 *>(p + 4);
+                    const uint32_t e[6] = {q0.x, q0.y, q1.x, q1.y, q2.x, q2.y};
+                    uint32_t l[4], c[4], rr[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        l[i] = __builtin_amdgcn_alignbit(e[i + 1], e[i], 16);
+                        c[i] = e[i + 1];
+                        rr[i] = __builtin_amdgcn_alignbit(e[i + 2], e[i + 1], 16);
+                    }
+                    const bf16x8 b[3] = {frag(l), frag(c), frag(rr)};
+#pragma unroll
+                    for (int d = 0; d < 3; ++d)
+#pragma unroll
+                        for (int mt = 0; mt < 2; ++mt)
+                            acc[3 * dyi + d][mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                av[mt], b[d], acc[3 * dyi + d][mt][nt], 0, 0, 0);
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    float *out = part + ((long)blockIdx.x * (NB / 64) + wv) * (NW + C);
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
@@ -445,58 +677,127 @@ __global__ __launch_bounds__(NB) void k_dw32(Geo g, const bf16_t *__restrict__ d
                     const int co = 16 * mt + 4 * kq + i, ci = 16 * nt + m;
                     out[((long)co * T + t) * C + ci] = acc[t][mt][nt][i];
                 }
-    // bias: lanes of one co (same m) across the 4 lane groups
-    for (int mt = 0; mt < 2; ++mt) {
-        float v = bsum[mt];
-        v += __shfl_xor(v, 16);
-        v += __shfl_xor(v, 32);
-        if (kq == 0) out[NW + 16 * mt + m] = v;
-    }
+    if (m == 0)
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) out[NW + 16 * mt + 4 * kq + i] = bacc[mt][i];
 }
 
-// Weight gradients of layer 1 (x: FP32 potential) and layer 4 (dy: FP32
-// output gradient, x = a3): plain FP32 reductions (288 + 32 values each).
-// Layer 1: dW1[co][t] = sum_p dA1[p][co] x[nbr(p,t)], db1[co] = sum_p dA1[p][co].
-// Layer 4: dW4[t][ci] = sum_p dO[p] a3[nbr(p,t)][ci], db4 = sum_p dO[p].
-// Thread j < 320 of each block owns one output value over the block's
-// pixel range; partials part[b][320] reduced by k_reduce.
-__global__ __launch_bounds__(NB) void k_dw_small(Geo g, int layer, const bf16_t *__restrict__ dy32,
-                                                 const float *__restrict__ x1, const float *__restrict__ dy1,
-                                                 const bf16_t *__restrict__ x32, float *__restrict__ part)
+// Weight gradients of the layers with a one-channel side: M = the 32
+// channels of v, N = the 9 taps of the FP32 one-channel u (rounded to BF16),
+// K = pixels.
+// Layer 1 (LAST = false): v = dA1, u = the potential x:
+//   dW1[co][t] = sum_p dA1[p][co] x[nbr(p,t)], db1[co] = sum_p dA1[p][co]
+//   (column 9: ones).
+// Layer 4 (LAST): v = a3, u = dO:
+//   dW4[t][ci] = sum_p a3[p][ci] dO[nbr(p,-t)], db4 = sum_p dO[p] in FP32.
+// The wave's partial goes to part[4 blockIdx + wave], C T + C values in the
+// parameters' order.
+template <bool LAST>
+__global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict__ v,
+                                                const float *__restrict__ u, float *__restrict__ part)
 {
-    constexpr int NV = C * T + C;  // 320
-    const long per = (g.np + gridDim.x - 1) / gridDim.x;
-    const long pa = (long)blockIdx.x * per, pb = pa + per < g.np ? pa + per : g.np;
-    for (int j = threadIdx.x; j < NV; j += NB) {
-        float s = 0.f;
-        if (layer == 1) {
-            if (j < C * T) {
-                const int co = j / T, t = j % T;
-                for (long p = pa; p < pb; ++p) s += bf2f(dy32[p * C + co]) * bf2f(f2bf(x1[nbr(g, p, t, 1)]));
-            } else {
-                const int co = j - C * T;
-                for (long p = pa; p < pb; ++p) s += bf2f(dy32[p * C + co]);
-            }
-        } else {
-            if (j < C * T) {
-                const int t = j / C, ci = j % C;
-                for (long p = pa; p < pb; ++p) s += bf2f(f2bf(dy1[p])) * bf2f(x32[nbr(g, p, t, 1) * C + ci]);
-            } else if (j == C * T) {
-                for (long p = pa; p < pb; ++p) s += dy1[p];
-            }
+    constexpr int NV = C * T + C;
+    __shared__ __align__(16) uint32_t lds[NB / 64][C * kTr];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int m = lane & 15, kq = lane >> 4;
+    const int pp = lane >> 2, cg = lane & 3;
+    const int sgn = LAST ? -1 : 1;
+    const int ody = sgn * (m / 3 - 1), odx = sgn * (m % 3 - 1);  // the tap of column m < 9
+    uint32_t *tv = lds[wv];
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+    f4 acc[2] = {zero, zero};
+    float bsum = 0.f;
+    const uint4 z4 = {0, 0, 0, 0};
+    const long nt_ = dw_tasks(g);
+    for (long task = (long)blockIdx.x * (NB / 64) + wv; task < nt_; task += (long)gridDim.x * (NB / 64)) {
+        const DwStrip s = dw_strip(g, task);
+        const int c0 = dw_col(s.x0 + 2 * pp, g.w), c1 = dw_col(s.x0 + 2 * pp + 1, g.w);
+        const bool ok0 = s.x0 + 2 * pp < g.w, ok1 = s.x0 + 2 * pp + 1 < g.w;
+        int uc[8];
+        bool uok[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            uok[j] = s.x0 + 8 * kq + j < g.w;
+            uc[j] = dw_col(s.x0 + 8 * kq + j + odx, g.w);
         }
-        part[(long)blockIdx.x * NV + j] = s;
+        auto ldv = [&](int y, Pair &p) {
+            const bf16_t *b = v + (s.base + (long)y * g.w) * C + 8 * cg;
+            p.a = ok0 ? *reinterpret_cast<const uint4 *>(b + (long)c0 * C) : z4;
+            p.b = ok1 ? *reinterpret_cast<const uint4 *>(b + (long)c1 * C) : z4;
+        };
+        auto ldu = [&](int y, float f[8]) {
+            const float *b = u + s.base + (long)wrap(y + ody, g.h) * g.w;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) f[j] = m < T ? b[uc[j]] : 1.f;
+        };
+        Pair pv;
+        float f[8];
+        ldv(s.y0, pv);
+        ldu(s.y0, f);
+        for (int y = s.y0; y < s.y1; ++y) {
+            put_pair(tv, cg, pp, pv);
+            bf16x8 b;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                b[j] = as_bf(m <= T ? f2bf(f[j]) : (bf16_t)0);
+                if (LAST && m == 4 && uok[j]) bsum += f[j];  // the centre tap's pixels
+            }
+            if (y + 1 < s.y1) {
+                ldv(y + 1, pv);
+                ldu(y + 1, f);
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt) {
+                const uint32_t *p = tv + (16 * mt + m) * kTr + 4 * kq;
+                const uint2 lo = *reinterpret_cast<const uint2 *>(p), hi = *reinterpret_cast<const uint2 *>(p + 2);
+                const uint32_t d[4] = {lo.x, lo.y, hi.x, hi.y};
+                acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(d), b, acc[mt], 0, 0, 0);
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    float *out = part + ((long)blockIdx.x * (NB / 64) + wv) * NV;
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int ch = 16 * mt + 4 * kq + i;
+            if (m < T) out[LAST ? m * C + ch : ch * T + m] = acc[mt][i];
+            if (!LAST && m == T) out[C * T + ch] = acc[mt][i];
+        }
+    if (LAST) {
+        bsum += __shfl_xor(bsum, 16);
+        bsum += __shfl_xor(bsum, 32);
+        if (lane == 4) out[C * T] = bsum;
     }
 }
 
-// out[j] = sum_b part[b][j] over nb rows of stride len, in row order.
-__global__ __launch_bounds__(NB) void k_reduce(const float *__restrict__ part, int nb, int len,
-                                               float *__restrict__ out)
+// out[j] = sum_b part[b][j] over nb rows of stride len, in FP64: a block
+// takes 64 columns, its 16 groups of 64 threads every 16th row, and the
+// groups' sums are added in order (1024 rows of 9,248: 155 us with a thread
+// per column, now 6).
+constexpr int kRedGroups = 16;
+__global__ __launch_bounds__(64 * kRedGroups) void k_reduce(const float *__restrict__ part, int nb, int len,
+                                                            int stride, float *__restrict__ out)
 {
-    for (int j = blockIdx.x * NB + threadIdx.x; j < len; j += gridDim.x * NB) {
-        double s = 0.0;
-        for (int b = 0; b < nb; ++b) s += part[(long)b * len + j];
-        out[j] = (float)s;
+    __shared__ double sm[kRedGroups][64];
+    const int c = threadIdx.x & 63, gr = threadIdx.x >> 6;
+    const int j = blockIdx.x * 64 + c;
+    double s = 0.0;
+    if (j < len) {
+#pragma unroll 8
+        for (int b = gr; b < nb; b += kRedGroups) s += part[(long)b * stride + j];
+    }
+    sm[gr][c] = s;
+    __syncthreads();
+    if (gr == 0 && j < len) {
+        double t = 0.0;
+#pragma unroll
+        for (int i = 0; i < kRedGroups; ++i) t += sm[i][c];
+        out[j] = (float)t;
     }
 }
 
@@ -530,8 +831,6 @@ __global__ __launch_bounds__(NB) void k_bf16_params(const float *__restrict__ pr
     }
 }
 
-int grid_px(long np) { return (int)((np + PIX_BLK - 1) / PIX_BLK); }
-
 }  // namespace
 
 struct trlnet {
@@ -554,8 +853,6 @@ struct trlnet {
 };
 
 namespace {
-
-constexpr int kDwBlocks = 256;  // blocks of the weight-gradient reductions
 
 #define NTRY(e)                                  \
     do {                                         \
@@ -610,7 +907,7 @@ int refresh_bf16(trlnet *t)
 // (activations are channel-last, pixel p at p * C).
 int forward(trlnet *t, const Geo &g, long off = 0)
 {
-    const int gb = grid_px(g.np);
+    const int gb = (int)conv_blocks(g);
     const long oc = off * C;
     hipLaunchKernelGGL(k_fwd1, dim3(gb), dim3(NB), 0, t->s, g, t->x + off, t->wb + OW1, t->prm + OB1,
                        t->a1 + oc);
@@ -647,7 +944,7 @@ int forward_groups(trlnet *t, int ngroups, const int *nimg, const int *h, const 
     for (int i = 0; i < ngroups; ++i) {
         const Geo g{nimg[i], h[i], w[i], (long)nimg[i] * h[i] * w[i]};
         gg[i] = GroupGeo{g, off};
-        const long nb = (long)pre[i] + grid_px(g.np);
+        const long nb = (long)pre[i] + conv_blocks(g);
         if (nb > 0x7fffffffL) return TRLNET_EINVAL;
         pre[i + 1] = (int)nb;
         off += g.np;
@@ -670,28 +967,28 @@ int forward_groups(trlnet *t, int ngroups, const int *nimg, const int *h, const 
 // loss and gradient into t->grad (device); *loss on the host
 int backward(trlnet *t, const Geo &g, double *loss)
 {
-    const int gb = grid_px(g.np);
-    hipLaunchKernelGGL(k_loss, dim3(g.nimg), dim3(NB), 0, t->s, g, t->o, t->tg, t->dO, t->lpart);
-    // layer 4
-    hipLaunchKernelGGL(k_dw_small, dim3(kDwBlocks), dim3(NB), 0, t->s, g, 4, (const bf16_t *)nullptr,
-                       (const float *)nullptr, t->dO, t->a3, t->part);
-    hipLaunchKernelGGL(k_reduce, dim3(2), dim3(NB), 0, t->s, t->part, kDwBlocks, C * T + C, t->part + (long)kDwBlocks * (C * T + C));
-    NTRY(hipMemcpyAsync(t->grad + OW4, t->part + (long)kDwBlocks * (C * T + C), sizeof(float) * (C * T + 1),
-                        hipMemcpyDeviceToDevice, t->s));
-    hipLaunchKernelGGL(k_bwd4, dim3(gb), dim3(NB), 0, t->s, g, t->dO, t->wb + OW4, t->a3, t->d2);
+    const int gb = (int)conv_blocks(g);
+    const int NW = C * T * C + C, NV = C * T + C, np = kDwBlocks * (NB / 64);
+    const dim3 dwb(kDwBlocks), blk(NB);
+    auto reduce = [&](int len, int stride, float *out) {
+        hipLaunchKernelGGL(k_reduce, dim3((len + 63) / 64), dim3(64 * kRedGroups), 0, t->s, t->part, np, len, stride, out);
+    };
+    hipLaunchKernelGGL(k_loss, dim3(g.nimg), blk, 0, t->s, g, t->o, t->tg, t->dO, t->lpart);
+    // layer 4 (its gradient ends with the one bias)
+    hipLaunchKernelGGL((k_dw_edge<true>), dwb, blk, 0, t->s, g, t->a3, t->dO, t->part);
+    reduce(C * T + 1, NV, t->grad + OW4);
+    hipLaunchKernelGGL(k_bwd4, dim3(gb), blk, 0, t->s, g, t->dO, t->wb + OW4, t->a3, t->d2);
     // layer 3: dY = d2 (for a3), X = a2
-    const int NW = C * T * C + C;
-    hipLaunchKernelGGL(k_dw32, dim3(kDwBlocks), dim3(NB), 0, t->s, g, t->d2, t->a2, t->part);
-    hipLaunchKernelGGL(k_reduce, dim3((NW + NB - 1) / NB), dim3(NB), 0, t->s, t->part, kDwBlocks * 4, NW, t->grad + OW3);
-    hipLaunchKernelGGL(k_bwd32, dim3(gb), dim3(NB), 0, t->s, g, t->d2, t->wt3, t->a2, t->d1);
+    hipLaunchKernelGGL(k_dw32, dwb, blk, 0, t->s, g, t->d2, t->a2, t->part);
+    reduce(NW, NW, t->grad + OW3);
+    hipLaunchKernelGGL(k_bwd32, dim3(gb), blk, 0, t->s, g, t->d2, t->wt3, t->a2, t->d1);
     // layer 2: dY = d1 (for a2), X = a1
-    hipLaunchKernelGGL(k_dw32, dim3(kDwBlocks), dim3(NB), 0, t->s, g, t->d1, t->a1, t->part);
-    hipLaunchKernelGGL(k_reduce, dim3((NW + NB - 1) / NB), dim3(NB), 0, t->s, t->part, kDwBlocks * 4, NW, t->grad + OW2);
-    hipLaunchKernelGGL(k_bwd32, dim3(gb), dim3(NB), 0, t->s, g, t->d1, t->wt2, t->a1, t->d2);
+    hipLaunchKernelGGL(k_dw32, dwb, blk, 0, t->s, g, t->d1, t->a1, t->part);
+    reduce(NW, NW, t->grad + OW2);
+    hipLaunchKernelGGL(k_bwd32, dim3(gb), blk, 0, t->s, g, t->d1, t->wt2, t->a1, t->d2);
     // layer 1: dY = d2 (for a1), X = potential
-    hipLaunchKernelGGL(k_dw_small, dim3(kDwBlocks), dim3(NB), 0, t->s, g, 1, t->d2, t->x,
-                       (const float *)nullptr, (const bf16_t *)nullptr, t->part);
-    hipLaunchKernelGGL(k_reduce, dim3(2), dim3(NB), 0, t->s, t->part, kDwBlocks, C * T + C, t->grad + OW1);
+    hipLaunchKernelGGL((k_dw_edge<false>), dwb, blk, 0, t->s, g, t->d2, t->x, t->part);
+    reduce(NV, NV, t->grad + OW1);
     if (hipGetLastError() != hipSuccess) return TRLNET_EHIP;
     std::vector<double> lp((size_t)g.nimg);
     NTRY(hipMemcpyAsync(lp.data(), t->lpart, sizeof(double) * g.nimg, hipMemcpyDeviceToHost, t->s));
