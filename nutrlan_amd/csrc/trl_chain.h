@@ -29,17 +29,18 @@
 // columns are read and written by their owner only.  The CSR kinds gather the
 // new vector with ordinary loads after an agent-scope acquire.
 //
-// Termination: the workgroups first meet at a gate (chain_gate).  Either all
-// of them are running and the chain starts, or -- the device is filled by
-// other work -- the gate closes after kGateTicks, nothing has been written
-// and the host runs the step's ordinary kernels.  Past the gate every
-// workgroup is resident, so each barrier ends; its wait is bounded all the
-// same.
+// Termination: a chain's workgroups first meet at a gate (chain_gate).
+// Either all of them are running and the chain starts, or -- the device is
+// filled by other work -- the gate closes after a while, nothing has been
+// written and the host runs the step's ordinary kernels.  Past the gate
+// every workgroup is resident, so each barrier ends; its wait is bounded all
+// the same.
 #ifndef TRL_CHAIN_H
 #define TRL_CHAIN_H
 
-constexpr unsigned long long kGateTicks = 200000;      // 2 ms at 100 MHz
-constexpr unsigned long long kBarrierTicks = 200000000;  // 2 s
+// ticks of 10 ns: a single solve gives up soon, a batch's chains also wait for each other
+constexpr unsigned long long kGateTicks = 200000, kBatchGateTicks = 20000000;  // 2 ms, 200 ms
+constexpr unsigned long long kBarrierTicks = 6000000000ull;  // 60 s
 
 struct ChainArgs {
     int n, g, steps, first, qa, qb, rcol, jnd, kept, ntot;
@@ -57,9 +58,11 @@ struct ChainArgs {
     const double *coef;     // first step: its jnd - 1 coefficients
     double *hm;             // host-coherent: step 0's results, status at 6
     double *hchain;         // followers' results, 7 each
-    unsigned *sync;         // flags, then the two gate words
+    unsigned *sync;         // a flag per workgroup
     unsigned base;          // flag value before this launch
-    int parity;             // the gate word of this launch
+    unsigned *gate;         // this launch's gate word (zero)
+    unsigned *gate_next;    // the next launch's, cleared at the end, or null
+    unsigned long long gate_ticks;
 };
 
 __device__ __forceinline__ double ld_agent(const double *p)
@@ -103,14 +106,14 @@ __device__ __forceinline__ bool chain_poll(const unsigned *flags, int g, unsigne
 // visible to agent-scope loads.  *ok_s: the workgroup's flag in LDS.
 // ACQ: visible to ordinary loads too.
 template <bool ACQ = false>
-__device__ __forceinline__ bool chain_barrier(const ChainArgs &q, unsigned want, int *ok_s)
+__device__ __forceinline__ bool chain_barrier(const ChainArgs &q, int b, unsigned want, int *ok_s)
 {
     stores_done();
     __syncthreads();
     if (q.g > 1) {
         if (threadIdx.x < 64) {
             if (threadIdx.x == 0)
-                __hip_atomic_store(q.sync + blockIdx.x, want, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(q.sync + b, want, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const bool ok = chain_poll(q.sync, q.g, want);
             if (threadIdx.x == 0 && !ok) *ok_s = 0;
             if constexpr (ACQ) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -123,15 +126,15 @@ __device__ __forceinline__ bool chain_barrier(const ChainArgs &q, unsigned want,
 // The gate: true in every workgroup when all g are running, false in every
 // workgroup when one of them gave up waiting first (the gate word is set
 // once: 1 open, 2 closed).
-__device__ __forceinline__ bool chain_gate(const ChainArgs &q, int *ok_s)
+__device__ __forceinline__ bool chain_gate(const ChainArgs &q, int b, int *ok_s)
 {
     if (q.g == 1) return true;
-    unsigned *gate = q.sync + kChainGate + 32 * q.parity;
+    unsigned *gate = q.gate;
     const unsigned want = q.base + 1;
     if (threadIdx.x < 64) {
         const int lane = threadIdx.x;
         if (lane == 0)
-            __hip_atomic_store(q.sync + blockIdx.x, want, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(q.sync + b, want, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const unsigned long long t0 = wall_clock64();
         unsigned st = 0;
         while (!st) {
@@ -141,7 +144,7 @@ __device__ __forceinline__ bool chain_gate(const ChainArgs &q, int *ok_s)
                 in = in && (int)(f - want) >= 0;
             }
             const bool all = __all(in);
-            const bool late = wall_clock64() - t0 > kGateTicks;
+            const bool late = wall_clock64() - t0 > q.gate_ticks;
             if (lane == 0) {
                 if (all || late) {
                     unsigned seen = 0;
@@ -317,7 +320,7 @@ __device__ __forceinline__ double norm4(const double r[4], int row, int n)
 // KIND as spmv_kind: -3 / -2 periodic stencils, -1 packed CSR, 0 CSR.  VS =
 // what the Gram-Schmidt pass reads (float: the FP32 shadow).
 template <int RW, int KIND, typename VS>
-__global__ __launch_bounds__(256 * RW) void k_chain(ChainArgs q)
+__device__ __forceinline__ void chain_body(const ChainArgs &q, const int b)
 {
     constexpr int R = 256 * RW, NT = 256 * RW, NWAVE = 4 * RW;
     constexpr bool kStencil = KIND <= -2;
@@ -336,7 +339,6 @@ __global__ __launch_bounds__(256 * RW) void k_chain(ChainArgs q)
     __shared__ int ok_s;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int rw = w % RW, k = w / RW;  // row wave, column group
-    const int b = blockIdx.x;
     const int n = q.n, g = q.g;
     const int R0 = b * R;
     const int row = R0 + rw * 256 + 4 * lane;  // first of this lane's four rows
@@ -351,10 +353,10 @@ __global__ __launch_bounds__(256 * RW) void k_chain(ChainArgs q)
         VG = q.V + vrow;
     if (t == 0) ok_s = 1;
     __syncthreads();
-    if (!chain_gate(q, &ok_s)) {
+    if (!chain_gate(q, b, &ok_s)) {
         if (b == 0 && t == 0) {
             q.hm[6] = 2.0;
-            q.sync[kChainGate + 32 * (1 - q.parity)] = 0;
+            if (q.gate_next) *q.gate_next = 0;
         }
         return;
     }
@@ -456,7 +458,7 @@ __global__ __launch_bounds__(256 * RW) void k_chain(ChainArgs q)
                 if (q.V32) q.V32[(size_t)qa * q.ld + srow] = (float)xr;
             }
         }
-        if (!chain_barrier(q, ++want, &ok_s)) break;
+        if (!chain_barrier(q, b, ++want, &ok_s)) break;
         // ---- alpha; r = y - beta q_b - alpha q_a (or the restart's columns)
         if (t < 256) {
             const double v = wave_sum(strided_sum_agent(q.part_alpha, q.nb, t, 256));
@@ -556,7 +558,7 @@ __global__ __launch_bounds__(256 * RW) void k_chain(ChainArgs q)
         if (k == 0)
 #pragma unroll
             for (int j = 0; j < 4; ++j) ys[lrow + j] = r4[j];
-        if (!chain_barrier(q, ++want, &ok_s)) break;
+        if (!chain_barrier(q, b, ++want, &ok_s)) break;
         // ---- h, then s = r - V h and its norm
         {
             const int np = RW == 4 ? nrb : nw;
@@ -620,7 +622,7 @@ __global__ __launch_bounds__(256 * RW) void k_chain(ChainArgs q)
                 st_agent(q.part_update + b, s);
             }
         }
-        if (!chain_barrier<!kStencil>(q, ++want, &ok_s)) break;
+        if (!chain_barrier<!kStencil>(q, b, ++want, &ok_s)) break;
         // ---- the norms, the step's results, the decision for the next step
         if (w < 2) {
             const double v = wave_ordered_sum<RW>(w == 0 ? q.part_recur : q.part_update, nrb, nw);
@@ -662,7 +664,45 @@ __global__ __launch_bounds__(256 * RW) void k_chain(ChainArgs q)
     }
     if (b == 0 && t == 0) {
         q.hm[6] = status == 0 ? 1.0 : 3.0;
-        q.sync[kChainGate + 32 * (1 - q.parity)] = 0;
+        if (q.gate_next) *q.gate_next = 0;
+    }
+}
+
+template <int RW, int KIND, typename VS>
+__global__ __launch_bounds__(256 * RW) void k_chain(ChainArgs q)
+{
+    chain_body<RW, KIND, VS>(q, blockIdx.x);
+}
+
+// The chains of many solves in one launch.  At most one workgroup per CU is
+// launched; each takes pieces (one workgroup's share of one chain, pieces of
+// a chain consecutive) by ticket until none are left, so the pieces taken
+// are always the first ones.  A chain waits at its gate for pieces that
+// workgroups free of earlier chains take next; with at most a quarter of the
+// CUs' workgroups per chain that holds also when other lanes' launches or
+// other work take part of the device, and should the device be taken
+// altogether the gate closes and the host runs that chain's step otherwise.
+// (A workgroup per piece does not do: workgroups go to the XCDs round-robin,
+// so the last ones may all belong to one XCD and wait for each other's
+// place there.)  Flags, gate words and ticket start at zero: they are copied
+// with the launch's records.
+template <int RW, int KIND, typename VS>
+__global__ __launch_bounds__(256 * RW) void kb_chain(const ChainArgs *__restrict__ d,
+                                                     const int *__restrict__ pre, int nreq,
+                                                     unsigned *__restrict__ ticket)
+{
+    __shared__ int mine;
+    const int total = pre[nreq];
+    for (;;) {
+        if (threadIdx.x == 0)
+            mine = (int)__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        const int i = __builtin_amdgcn_readfirstlane(mine);
+        if (i >= total) return;
+        const int p = __builtin_amdgcn_readfirstlane(batch_find(pre, nreq, i));
+        const ChainArgs q = d[p];
+        chain_body<RW, KIND, VS>(q, i - pre[p]);
+        __syncthreads();  // the LDS of this piece has been read
     }
 }
 

@@ -2046,7 +2046,6 @@ bool recproj_ok(const trlhip_ctx *c)
 // prefetched nonzeros no longer fit the 128 registers a thread of 16 waves
 // has (n = 50,001, 17 nonzeros a row: the product takes 30 us against 16).
 int chain_rw(const trlhip_csr *A) { return spmv_kind(A) <= -2 && A->n > 32768 ? 4 : 2; }
-int chain_wgs(const trlhip_csr *A) { return (A->n + 256 * chain_rw(A) - 1) / (256 * chain_rw(A)); }
 
 // Whether a step of a single solve runs as a chain kernel: real solves with
 // a stencil or CSR-stream operator whose workgroups fit kChainMaxWG (n <=
@@ -2056,14 +2055,43 @@ int chain_wgs(const trlhip_csr *A) { return (A->n + 256 * chain_rw(A) - 1) / (25
 // 10,000 (2D) 11.7 -> 6.4, n = 62,500 16.7 -> 9.9, n = 262,144 24.9 -> 23.3;
 // random rows n = 50,001 69 -> 48 ms.
 constexpr int kChainCsrIter = 4;
+bool chain_fits_wg(const trlhip_ctx *c, const trlhip_csr *A, int jnd, int rw, int maxg)
+{
+    if (!A || c->E != 1 || c->chain_off || A->lpr || A->pn_on || jnd > kChainMaxCols) return false;
+    const int g = (A->n + 256 * rw - 1) / (256 * rw);
+    if (g > maxg || A->nb > kSpmvGrid) return false;
+    if (spmv_kind(A) <= -2) return true;
+    return A->max_blk_nnz <= kNnzBlk && (A->nb + g * rw - 1) / (g * rw) <= kChainCsrIter;
+}
 bool chain_fits(const trlhip_ctx *c, const trlhip_csr *A, int jnd)
 {
-    if (!A || c->batch || c->E != 1 || c->chain_off || A->lpr || A->pn_on || jnd > kChainMaxCols) return false;
-    const int g = chain_wgs(A);
-    if (g > kChainMaxWG || A->nb > kSpmvGrid) return false;
-    if (spmv_kind(A) <= -2) return true;
-    const int groups = g * chain_rw(A);
-    return A->max_blk_nnz <= kNnzBlk && (A->nb + groups - 1) / groups <= kChainCsrIter;
+    return !c->batch && A && chain_fits_wg(c, A, jnd, chain_rw(A), kChainMaxWG);
+}
+
+// A batch's launch runs its steps as chains (kb_chain) while the solves that
+// fit hold at most kBatchChainRows rows together.  The device holds 262,144
+// rows of a chain kernel at once (1024 a workgroup, one workgroup per CU) and
+// steps them in about 14 us; the phase kernels take 25 us and 40 more per
+// million rows.  Batches with the limit at 0, 300,000, 600,000 and 1,500,000:
+// 40 lattices of 48-160 61.2, 44.1, 44.8, 44.5 ms; 16 of 100-220, mixed,
+// 56.5, 39.9, 39.8, 37.8; 90 of 60-180 84.8, 77.5, 77.6, 79.6; 192 of 64-256,
+// mixed, 183, 170, 170, 174 (whose later rounds fit).
+constexpr long kBatchChainRows = 600000;
+constexpr int kBatchChainWG = 64;  // workgroups of one solve at most, and a quarter of the CUs
+
+// CUs of the current device (queried once: the answer does not change).
+int device_cus()
+{
+    static std::atomic<int> cus{0};
+    int n = cus.load(std::memory_order_relaxed);
+    if (!n) {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1)
+            n = 1;
+        cus.store(n, std::memory_order_relaxed);
+    }
+    return n;
 }
 
 // Workgroups of the stencil SpMV: kStRB row blocks each (one alpha partial
@@ -2900,6 +2928,54 @@ int batch_run(hipStream_t s, const GroupInfo &gi, const BDesc *dd, const int *dp
     return hipGetLastError() == hipSuccess ? 0 : TRLHIP_EHIP;
 }
 
+// A chain's arguments apart from its input vector, coefficients and flags.
+static void chain_args(ChainArgs &q, trlhip_ctx *c, const trlhip_csr *A, int rw, int first, int qa, int qb,
+                       double beta_prev, int jnd, int rcol, int K, int kept, int ntot)
+{
+    q.n = c->n;
+    q.g = (c->n + 256 * rw - 1) / (256 * rw);
+    q.steps = K;
+    q.first = first;
+    q.qa = qa;
+    q.qb = first ? -1 : qb;
+    q.rcol = rcol;
+    q.jnd = jnd;
+    q.kept = kept;
+    q.ntot = ntot;
+    q.kind = spmv_kind(A);
+    q.nb = A->nb;
+    q.L = A->st_L;
+    q.off = A->st_off;
+    q.ld = c->ld;
+    q.beta_prev = beta_prev;
+    q.eps = c->V32 ? (double)FLT_EPSILON : DBL_EPSILON;
+    q.V = colp<double>(c, 0);
+    q.V32 = c->V32;
+    q.scratch = colp<double>(c, c->ncols);
+    q.dg = A->dg;
+    q.val = A->val;
+    q.tab = A->tab;
+    q.rb = A->rb;
+    q.rp = A->rp;
+    q.ci = A->ci;
+    q.pk = A->pk;
+    q.part_alpha = part_alpha(c);
+    q.part_recur = part_recur(c);
+    q.part_update = part_update(c);
+    q.part_proj = part_proj(c);
+    q.hm = c->dres;
+    q.hchain = c->dres + hres_chain(c->ncols);
+}
+
+// The chain's algorithmic bytes if every step runs.
+static double chain_bytes(const trlhip_ctx *c, const trlhip_csr *A, int jnd, int K)
+{
+    double bytes = 0.0;
+    for (int k = 0; k < K; ++k)
+        bytes += spmv_bytes(A, 1, 8, 8) + ((c->V32 ? 8.0 : 16.0) * (jnd + k) + 40.0) * c->n;
+    return bytes;
+}
+
 // (Grouping the launches group-major instead, so one group's vectors stay
 // in the last-level cache from phase to phase, measured 7-33 % slower on
 // the batched 2D Anderson workload: the smaller launches lose more than
@@ -2912,7 +2988,67 @@ struct StepsPlan {
     std::vector<BatchStep> order;
     std::vector<GroupInfo> groups;
     size_t npre = 0, off_pre = 0, off_cb = 0, total = 0;
+    // the steps that run as chains (kb_chain): groups by SpMV kernel and
+    // basis precision; records, prefix tables, then the flags and a ticket
+    // per group, which start at zero
+    struct Chain {
+        BatchStep st;
+        int K;
+    };
+    struct ChainGroup {
+        int kind, R, wgs;
+        bool mixed;
+        size_t doff, poff, foff;  // first record, prefix entry, flag word (the ticket)
+        double bytes;
+    };
+    std::vector<Chain> chains;
+    std::vector<ChainGroup> cgroups;
+    int rw = 4;  // row waves a workgroup (stencils)
+    size_t off_ch = 0, off_chpre = 0, off_flags = 0;
 };
+
+// Moves the steps that run as chains into the plan: all that fit, when
+// their rows are few enough.
+void chains_plan(const trlhip_batch *b, StepsPlan &P, std::vector<char> &taken)
+{
+    long rows = 0;
+    int maxn = 0;
+    for (const BatchStep &st : b->steps)
+        if (st.ci == 0 && chain_fits_wg(st.c, st.A, st.jnd, 4, kBatchChainWG)) {
+            rows += st.c->n;
+            maxn = std::max(maxn, st.c->n);
+        }
+    if (!rows || rows > kBatchChainRows) return;
+    // short phases while every workgroup runs at once, else the most rows
+    // the device holds
+    const int maxg = std::min(kBatchChainWG, device_cus() / 4);
+    P.rw = rows <= 512 * 256 && maxn <= 512 * maxg ? 2 : 4;
+    const auto &S = b->steps;
+    for (size_t i = 0; i < S.size(); ++i) {
+        if (taken[i] || S[i].ci != 0) continue;
+        const int rw0 = spmv_kind(S[i].A) <= -2 ? P.rw : 2;
+        if (!chain_fits_wg(S[i].c, S[i].A, S[i].jnd, rw0, maxg)) continue;
+        StepsPlan::ChainGroup cg{};
+        cg.kind = spmv_kind(S[i].A);
+        cg.mixed = S[i].c->V32 != nullptr;
+        cg.doff = P.chains.size();
+        for (size_t k = i; k < S.size(); ++k) {
+            if (taken[k] || S[k].ci != 0 || spmv_kind(S[k].A) != cg.kind || (S[k].c->V32 != nullptr) != cg.mixed ||
+                !chain_fits_wg(S[k].c, S[k].A, S[k].jnd, rw0, maxg))
+                continue;
+            // its followers are recorded right after it
+            StepsPlan::Chain ch{S[k], 1};
+            taken[k] = 1;
+            for (size_t f = k + 1; f < S.size() && S[f].c == S[k].c && S[f].ci == ch.K; ++f) {
+                taken[f] = 1;
+                if (S[f].jnd <= kChainMaxCols) ++ch.K;
+            }
+            P.chains.push_back(ch);
+        }
+        cg.R = (int)(P.chains.size() - cg.doff);
+        P.cgroups.push_back(cg);
+    }
+}
 
 void steps_plan(const trlhip_batch *b, StepsPlan &P)
 {
@@ -2920,6 +3056,7 @@ void steps_plan(const trlhip_batch *b, StepsPlan &P)
     auto &groups = P.groups;
     order.reserve(b->steps.size());
     std::vector<char> taken(b->steps.size(), 0);
+    chains_plan(b, P, taken);
     size_t npre = 0;
     // chain position first: a context's follower runs after its step
     // before it, so all steps at position 0 launch first, then position 1 ...
@@ -2952,6 +3089,27 @@ void steps_plan(const trlhip_batch *b, StepsPlan &P)
     P.off_pre = up(sizeof(BDesc) * order.size());
     P.off_cb = up(P.off_pre + sizeof(int) * npre);
     P.total = P.off_cb + sizeof(double) * b->cbuf.size();
+    if (!P.cgroups.empty()) {
+        size_t cpre = 0, flags = 0;
+        for (StepsPlan::ChainGroup &cg : P.cgroups) {
+            const int rw = cg.kind <= -2 ? P.rw : 2;
+            cg.poff = cpre;
+            cg.foff = flags;
+            cpre += (size_t)cg.R + 1;
+            flags += 64;  // the ticket
+            for (int i = 0; i < cg.R; ++i) {
+                const BatchStep &st = P.chains[cg.doff + i].st;
+                const int g = (st.c->n + 256 * rw - 1) / (256 * rw);
+                cg.wgs += g;
+                cg.bytes += chain_bytes(st.c, st.A, st.jnd, P.chains[cg.doff + i].K);
+                flags += 64 + (size_t)((g + 63) & ~63);  // its gate word, its flags
+            }
+        }
+        P.off_ch = up(P.total);
+        P.off_chpre = up(P.off_ch + sizeof(ChainArgs) * P.chains.size());
+        P.off_flags = up(P.off_chpre + sizeof(int) * cpre);
+        P.total = P.off_flags + sizeof(unsigned) * flags;
+    }
 }
 
 // Writes the plan's descriptors, prefix tables and coefficients into the
@@ -2964,6 +3122,34 @@ void steps_fill(const trlhip_batch *b, StepsPlan &P, char *h, const char *d)
     for (GroupInfo &gi : P.groups)
         batch_fill(P.order.data() + gi.doff, gi.R, hdesc + gi.doff, hpre + gi.poff, gi, dcbuf);
     if (!b->cbuf.empty()) memcpy(h + P.off_cb, b->cbuf.data(), sizeof(double) * b->cbuf.size());
+    if (P.cgroups.empty()) return;
+    memset(h + P.off_flags, 0, P.total - P.off_flags);
+    ChainArgs *hd = reinterpret_cast<ChainArgs *>(h + P.off_ch);
+    int *hp = reinterpret_cast<int *>(h + P.off_chpre);
+    unsigned *df = reinterpret_cast<unsigned *>(const_cast<char *>(d) + P.off_flags);
+    for (const StepsPlan::ChainGroup &cg : P.cgroups) {
+        const int rw = cg.kind <= -2 ? P.rw : 2;
+        int *pp = hp + cg.poff;
+        size_t fl = cg.foff + 64;
+        pp[0] = 0;
+        for (int i = 0; i < cg.R; ++i) {
+            const StepsPlan::Chain &ch = P.chains[cg.doff + i];
+            const BatchStep &st = ch.st;
+            ChainArgs &q = hd[cg.doff + i];
+            q = ChainArgs{};
+            chain_args(q, st.c, st.A, rw, st.first, st.qa, st.qb, st.beta_prev, st.jnd, st.rcol, ch.K, st.kept,
+                       st.ntot);
+            q.x = colp<double>(st.c, st.fuse ? st.fuse_src : st.qa);
+            q.xscale = st.fuse ? st.fuse_s : 1.0;
+            q.store_q = st.fuse;
+            q.coef = st.coff >= 0 ? dcbuf + st.coff : nullptr;
+            q.gate = df + fl;
+            q.gate_ticks = kBatchGateTicks;
+            q.sync = df + fl + 64;
+            fl += 64 + (size_t)((q.g + 63) & ~63);
+            pp[i + 1] = pp[i] + q.g;
+        }
+    }
 }
 
 // Launches every recorded step, in the order form_residual + run_proj +
@@ -2977,6 +3163,37 @@ int steps_launch(hipStream_t s, const StepsPlan &P, const char *h, const char *d
     const int *hpre = reinterpret_cast<const int *>(h + P.off_pre);
     for (const GroupInfo &gi : P.groups)
         if (int rc = batch_run(s, gi, ddesc + gi.doff, dpre + gi.poff, hpre + gi.poff)) return rc;
+    const ChainArgs *dch = reinterpret_cast<const ChainArgs *>(d + P.off_ch);
+    const int *dcp = reinterpret_cast<const int *>(d + P.off_chpre);
+    unsigned *df = reinterpret_cast<unsigned *>(const_cast<char *>(d) + P.off_flags);
+    for (const StepsPlan::ChainGroup &cg : P.cgroups) {
+        Timed t(TRLHIP_K_MISC, s, cg.bytes);
+        const ChainArgs *q = dch + cg.doff;
+        const int *pp = dcp + cg.poff;
+        unsigned *ticket = df + cg.foff;
+        const dim3 grid(std::min(cg.wgs, device_cus()));
+#define KB_CHAIN(RW, KIND)                                                                      \
+    do {                                                                                        \
+        if (cg.mixed)                                                                           \
+            KLAUNCH((kb_chain<RW, KIND, float>), grid, dim3(256 * RW), 0, s, q, pp, cg.R, ticket); \
+        else                                                                                    \
+            KLAUNCH((kb_chain<RW, KIND, double>), grid, dim3(256 * RW), 0, s, q, pp, cg.R, ticket); \
+    } while (0)
+        switch (cg.kind) {
+        case -3:
+            if (P.rw == 4) KB_CHAIN(4, -3);
+            else KB_CHAIN(2, -3);
+            break;
+        case -2:
+            if (P.rw == 4) KB_CHAIN(4, -2);
+            else KB_CHAIN(2, -2);
+            break;
+        case -1: KB_CHAIN(2, -1); break;
+        default: KB_CHAIN(2, 0); break;
+        }
+#undef KB_CHAIN
+        if (hipGetLastError() != hipSuccess) return TRLHIP_EHIP;
+    }
     return 0;
 }
 
@@ -4302,23 +4519,7 @@ static int run_chain(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int 
 {
     ChainArgs q{};
     const int rw = chain_rw(A);
-    q.n = c->n;
-    q.g = chain_wgs(A);
-    q.steps = K;
-    q.first = first;
-    q.qa = qa;
-    q.qb = first ? -1 : qb;
-    q.rcol = rcol;
-    q.jnd = jnd;
-    q.kept = c->ch_kept;
-    q.ntot = c->ch_ntot;
-    q.kind = spmv_kind(A);
-    q.nb = A->nb;
-    q.L = A->st_L;
-    q.off = A->st_off;
-    q.ld = c->ld;
-    q.beta_prev = beta_prev;
-    q.eps = c->V32 ? (double)FLT_EPSILON : DBL_EPSILON;
+    chain_args(q, c, A, rw, first, qa, qb, beta_prev, jnd, rcol, K, c->ch_kept, c->ch_ntot);
     if (c->pend_dst == qa && rcol != c->pend_src) {
         q.x = colp<double>(c, c->pend_src);
         q.xscale = c->pend_s;
@@ -4328,35 +4529,17 @@ static int run_chain(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int 
         q.x = colp<double>(c, qa);
         q.xscale = 1.0;
     }
-    q.V = colp<double>(c, 0);
-    q.V32 = c->V32;
-    q.scratch = colp<double>(c, c->ncols);
-    q.dg = A->dg;
-    q.val = A->val;
-    q.tab = A->tab;
-    q.rb = A->rb;
-    q.rp = A->rp;
-    q.ci = A->ci;
-    q.pk = A->pk;
-    q.part_alpha = part_alpha(c);
-    q.part_recur = part_recur(c);
-    q.part_update = part_update(c);
-    q.part_proj = part_proj(c);
     if (first) memcpy(c->hres + hres_coef(c->ncols), beta, sizeof(double) * (size_t)(jnd - 1));
     q.coef = c->dres + hres_coef(c->ncols);
-    q.hm = c->dres;
-    q.hchain = c->dres + hres_chain(c->ncols);
     q.sync = c->sync;
     q.base = c->sync_base;
-    q.parity = c->gate_parity;
+    q.gate = c->sync + kChainGate + 32 * c->gate_parity;
+    q.gate_next = c->sync + kChainGate + 32 * (1 - c->gate_parity);
+    q.gate_ticks = kGateTicks;
     c->hres[6] = 0.0;
     for (int k = 1; k < K; ++k) c->hres[hres_chain(c->ncols) + 7 * (size_t)(k - 1) + 4] = 0.0;
     {
-        // the chain's bytes if every step runs
-        double bytes = 0.0;
-        for (int k = 0; k < K; ++k)
-            bytes += spmv_bytes(A, 1, 8, 8) + ((c->V32 ? 8.0 : 16.0) * (jnd + k) + 40.0) * c->n;
-        Timed t(TRLHIP_K_MISC, c->s, bytes);
+        Timed t(TRLHIP_K_MISC, c->s, chain_bytes(c, A, jnd, K));
 #define CHAIN_LAUNCH(RW, KIND)                                                                 \
     do {                                                                                       \
         if (c->V32)                                                                            \
@@ -4474,8 +4657,28 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
         c->ch_n = K;
         c->ch_next = K > 1 ? 1 : 0;
         c->ch_copy_ok = 0;
+        c->hres[6] = 0.0;
         if (int rc = ctx_wait(c)) return rc;
         const volatile double *hr = c->hres;
+        if (hr[6] == 2.0) {
+            // its chain's gate closed before anything was written: the step
+            // alone, as ordinary kernels (this context's from now on)
+            c->chain_off = 1;
+            c->ch_next = 0;
+            st.decide = 0;
+            {
+                std::lock_guard<SpinLock> lk(c->batch->mu);
+                if (st.coff >= 0) {
+                    st.coff = (long)c->batch->cbuf.size();
+                    c->batch->cbuf.insert(c->batch->cbuf.end(), beta, beta + (jnd - 1));
+                    c->batch->cbuf.push_back(0.0);
+                }
+                c->batch->steps.push_back(st);
+            }
+            c->hres[6] = 0.0;
+            if (int rc = ctx_wait(c)) return rc;
+        }
+        if (hr[6] == 3.0) return TRLHIP_EHIP;  // a chain kernel's wait ran out
         out[0] = hr[S_ALPHA];
         out[1] = hr[S_RR2];
         out[2] = hr[S_HH];

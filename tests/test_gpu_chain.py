@@ -1,9 +1,12 @@
-"""Chains of steps in one kernel (a single real solve on a stencil or
-CSR-stream operator) against the batched kernels, which run every step as
-kernels of their own: the same eigenvalues, vectors, residual estimates and
+"""Chains of steps in one kernel (real solves on stencil or CSR-stream
+operators, alone and in small batches) against the kernels that run a step
+phase by phase: the same eigenvalues, vectors, residual estimates and
 counters bit for bit, at sizes around the kernels' edges (256 rows a wave,
 512 and 1024 a workgroup, 64 row blocks a reduction wave, ragged ends), and
-with several solves on the device at once."""
+with several solves on the device at once.
+
+A batch too large for chains runs phase by phase, so each solve is compared
+with itself in a batch beside operators that fill it up."""
 import threading
 
 import numpy as np
@@ -22,6 +25,15 @@ def same(a, b):
         assert np.array_equal(a[k], b[k]), k
 
 
+_fill = []
+
+
+def filler(T):
+    if not _fill:
+        _fill.append((T.Csr(*W.anderson2d_csr(255, 6.0, seed=255)[0]), W.start_vector(255 * 255, seed=1)))
+    return _fill[0]
+
+
 def both(T, csr, mixed, lohi, ned, maxlan, tol=1e-8, maxmv=4000, seed=3):
     n = len(csr[0]) - 1
     A = T.Csr(*csr, mixed=mixed)
@@ -29,10 +41,17 @@ def both(T, csr, mixed, lohi, ned, maxlan, tol=1e-8, maxmv=4000, seed=3):
     x0 = W.start_vector(n, seed=seed)
     print(f"n={n} mixed={mixed} stencil={A.stencil} packed={A.packed}", flush=True)
     one = T.solve_csr(A, *args, x0)
-    rc, many, _ = T.solve_batch([(A,) + args + (x0,)])
+    rc, small, _ = T.solve_batch([(A,) + args + (x0,)])
+    assert rc == 0
+    # 2 x 11 fillers of 65,025 rows that stop after the same number of steps:
+    # each of the batch's two lanes holds over 600,000 rows
+    F, fx = filler(T)
+    fill = [(F, -1, 2, maxlan, 1e-14, 1, one["matvec"] + maxlan, 2, fx)] * 11
+    rc, large, _ = T.solve_batch([(A,) + args + (x0,)] + [fill[0]] + fill + fill[:9])
     A.close()
     assert rc == 0
-    same(one, many[0])
+    same(one, small[0])
+    same(one, large[0])
 
 
 @pytest.mark.parametrize("mixed", [False, True])
@@ -64,6 +83,26 @@ def test_chain_wide_basis(gpu_lib):
     """More basis columns than a chain kernel takes: its last steps of a
     cycle run as ordinary kernels."""
     both(gpu_lib, W.random_sym_csr(3001, seed=9), False, 1, 6, 200, maxmv=450)
+
+
+def test_chain_batch_mixed_kinds(gpu_lib):
+    """A small batch of stencils, packed and random operators in both
+    precisions: several chain groups in a launch, each solve as alone."""
+    T = gpu_lib
+    spec = [(W.anderson2d_csr(L, 4.0, seed=L)[0], m, -1, 6, 24) for L, m in ((40, 0), (41, 1), (90, 0), (200, 1), (250, 0))]
+    spec += [(W.laplace3d_csr(L, seed=L), m, 1, 6, 30) for L, m in ((9, 0), (20, 1))]
+    spec += [(W.diag_csr(900), 0, 1, 5, 30), (W.random_sym_csr(2500, seed=2), 0, 1, 8, 40),
+             (W.random_sym_csr(30001, seed=3), 1, 1, 8, 40)]
+    probs = []
+    for i, (csr, m, lohi, ned, maxlan) in enumerate(spec):
+        probs.append((T.Csr(*csr, mixed=bool(m)), lohi, ned, maxlan, 1e-8, 1, 400, ned,
+                      W.start_vector(len(csr[0]) - 1, seed=i)))
+    alone = [T.solve_csr(*p) for p in probs]
+    rc, got, _ = T.solve_batch(probs)
+    assert rc == 0
+    for p, a, b in zip(probs, alone, got):
+        p[0].close()
+        same(a, b)
 
 
 def test_chain_concurrent_solves(gpu_lib):
