@@ -22,6 +22,9 @@
 // partial, so the partials cross workgroups as wave totals and the reader
 // adds the four in order.
 //
+// Lanes load four rows at once up to the padding of a context's columns (ld
+// is n rounded up to 64; the padding holds zeros).
+//
 // Visibility: what another workgroup reads (partials, the new vector's rows,
 // y of a CSR operator) is stored and loaded with agent-scope atomics, which
 // go to the device's point of coherence; before a workgroup raises its flag
@@ -209,57 +212,6 @@ __device__ __forceinline__ double wave_ordered_sum(const double *p, int nrb, int
     double t = 0.0;
     for (int v = 0; v < kBlock / 64 && v * 64 < nrb; ++v) t += wave_sum(row_partial<RW>(p, nrb, nw, v * 64 + lane));
     return t;
-}
-
-// Four consecutive rows of a column (the padding rows of a context's
-// columns, up to ld, hold zeros).
-__device__ __forceinline__ void rows4(const float *p, double v[4])
-{
-    const f32x4 t = *reinterpret_cast<const f32x4 *>(p);
-    v[0] = t.x;
-    v[1] = t.y;
-    v[2] = t.z;
-    v[3] = t.w;
-}
-__device__ __forceinline__ void rows4(const double *p, double v[4]) { load4(p, v); }
-
-// Column group k's running sum of the update over columns [0, m) for four
-// rows: in each full group of 8 columns those with c mod 4 = k, and for k =
-// 0 the columns after the last full group (update_rows4's sums, in order).  Vc: the first
-// row in column 0.
-template <typename VS>
-__device__ __forceinline__ void column_sums(const VS *Vc, long ld, int m, const double *hs, int k,
-                                            double s[4])
-{
-    s[0] = s[1] = s[2] = s[3] = 0.0;
-    const int full = m & ~7;
-    int c = 0;
-    for (; c + 16 <= full; c += 16) {
-        double v[4][4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) rows4(Vc + (size_t)(c + 4 * i + k) * ld, v[i]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) s[j] += v[i][j] * hs[c + 4 * i + k];
-    }
-    for (; c < full; c += 8) {
-        double v[2][4];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) rows4(Vc + (size_t)(c + 4 * i + k) * ld, v[i]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) s[j] += v[i][j] * hs[c + 4 * i + k];
-    }
-    if (k == 0) {
-        for (; c < m; ++c) {
-            double v[4];
-            rows4(Vc + (size_t)c * ld, v);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) s[j] += v[j] * hs[c];
-        }
-    }
 }
 
 // One thread's part of a row block of a CSR operator (at most kNnzBlk
@@ -479,7 +431,7 @@ __device__ __forceinline__ void chain_body(const ChainArgs &q, const int b)
             // the columns split over the groups as in the update
             __syncthreads();
             double s[4] = {0.0, 0.0, 0.0, 0.0};
-            column_sums(q.V + vrow, q.ld, rm, hs, k, s);
+            group_sums(q.V + vrow, q.ld, rm, hs, k, s);
             if (k > 0)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) pool[(k - 1) * R + lrow + j] = s[j];
@@ -525,7 +477,7 @@ __device__ __forceinline__ void chain_body(const ChainArgs &q, const int b)
 #pragma unroll
             for (int c = 0; c < CH; ++c) {
                 p[c] = 0.0;
-                rows4(VG + (size_t)min(cb + c, jnd - 1) * q.ld, v[c]);
+                ld4(VG + (size_t)min(cb + c, jnd - 1) * q.ld, v[c]);
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j)
@@ -586,7 +538,7 @@ __device__ __forceinline__ void chain_body(const ChainArgs &q, const int b)
         __syncthreads();
         {
             double s[4] = {0.0, 0.0, 0.0, 0.0};
-            column_sums(VG, q.ld, jnd, hs, k, s);
+            group_sums(VG, q.ld, jnd, hs, k, s);
             if (k > 0)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) pool[(k - 1) * R + lrow + j] = s[j];

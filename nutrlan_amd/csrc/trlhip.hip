@@ -1307,6 +1307,174 @@ __global__ __launch_bounds__(kBlock) void k_update(
     update_body<VS, RS, E, RU, NTV>(n, V, ld, c0, m, h, h0, cpart, cnp, cslot, rin, rout, part, out_hh, out_coef, blockIdx.x, gridDim.x);
 }
 
+// k_update over the same 1024-row blocks with 1024 threads: real bases split
+// the columns over four groups of 256 threads, by the running sum of
+// update_rows4 a column goes to (c mod 4; after the last full group of 8 all
+// to the first); complex bases give each group one of a thread's four rows.
+// The sums and their order are k_update's, so are the bits.  For row counts
+// whose blocks leave most of the device idle it puts four times the loads in
+// flight.  Whole passes (trlhip_cgs_pass_noalloc) before and after: complex n
+// = 60,000, m = 60 93 -> 55 us, FP64 n = 100,000, m = 80 81 -> 53, n =
+// 260,000, m = 30 66 -> 52, FP32 n = 200,000, m = 60 74 -> 50 (some 13 us of
+// each are the one copy back instead of two); the 48^3 complex lattice 132 ->
+// 104 ms a solve.  Above kWideRows the 256-thread blocks fill the device.
+constexpr int kWide = 4 * kBlock;
+
+// Column group k's running sums of update_rows4 over columns [0, m) for four
+// rows (Vc: the first row in column 0).
+// Its loads are ordinary ones: at these sizes the projection has left the
+// columns in the caches.
+__device__ __forceinline__ void ld4(const float *p, double v[4])
+{
+    const f32x4 t = *reinterpret_cast<const f32x4 *>(p);
+    v[0] = t.x;
+    v[1] = t.y;
+    v[2] = t.z;
+    v[3] = t.w;
+}
+__device__ __forceinline__ void ld4(const double *p, double v[4]) { load4(p, v); }
+template <typename VS>
+__device__ __forceinline__ void group_sums(const VS *Vc, long ld, int m, const double *hs, int k, double s[4])
+{
+    s[0] = s[1] = s[2] = s[3] = 0.0;
+    const int full = m & ~7;
+    int c = 0;
+    for (; c + 16 <= full; c += 16) {
+        double v[4][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ld4(Vc + (size_t)(c + 4 * i + k) * ld, v[i]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] += v[i][j] * hs[c + 4 * i + k];
+    }
+    for (; c < full; c += 8) {
+        double v[2][4];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) ld4(Vc + (size_t)(c + 4 * i + k) * ld, v[i]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] += v[i][j] * hs[c + 4 * i + k];
+    }
+    if (k == 0) {
+        for (; c < m; ++c) {
+            double v[4];
+            ld4(Vc + (size_t)c * ld, v);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] += v[j] * hs[c];
+        }
+    }
+}
+
+template <typename VS, int E>
+__global__ __launch_bounds__(kWide) void k_update_wide(int n, const VS *__restrict__ V, long ld, int m,
+                                                       const double *__restrict__ h, const double *rin,
+                                                       double *rout, double *__restrict__ part,
+                                                       double *__restrict__ out_hh)
+{
+    extern __shared__ double hs[];
+    __shared__ double sm[3][4 * kBlock];
+    __shared__ double wt[kBlock / 64];
+    const int t = threadIdx.x, tg = t & (kBlock - 1), k = t >> 8, lane = t & 63, w = t >> 6;
+    for (int i = t; i < E * m; i += kWide) hs[i] = h[i];
+    __syncthreads();
+    const int R0 = blockIdx.x * 4 * kBlock;
+    double acc = 0.0;
+    if constexpr (E == 1) {
+        const int row = R0 + 4 * tg;
+        double s[4];
+        if (row < n) {
+            group_sums(V + row, ld, m, hs, k, s);
+            if (k > 0)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) sm[k - 1][4 * tg + j] = s[j];
+        }
+        __syncthreads();
+        if (k == 0 && row < n) {
+            double ro[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) ro[j] = (s[j] + sm[0][4 * tg + j]) + (sm[1][4 * tg + j] + sm[2][4 * tg + j]);
+            if (row + 3 < n) {
+                double ri[4];
+                load4(rin + row, ri);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) ro[j] = ri[j] - ro[j];
+                store4(rout + row, ro);
+                acc = sumsq4(ro);
+            } else {
+                for (int j = 0; row + j < n; ++j) {
+                    const double v = rin[row + j] - ro[j];
+                    rout[row + j] = v;
+                    acc = fma(v, v, acc);
+                }
+            }
+        }
+    } else {
+        const int row = R0 + t;
+        double p = 0.0;
+        if (row < n) {
+            const double2 *V2 = reinterpret_cast<const double2 *>(V) + row;
+            double ar = 0.0, ai = 0.0, br = 0.0, bi = 0.0;
+            int c = 0;
+            auto four = [&](const double2 v[4], int c0) {
+#pragma unroll
+                for (int q = 0; q < 4; q += 2) {
+                    const double h0r = hs[2 * (c0 + q)], h0i = hs[2 * (c0 + q) + 1];
+                    const double h1r = hs[2 * (c0 + q + 1)], h1i = hs[2 * (c0 + q + 1) + 1];
+                    ar += v[q].x * h0r - v[q].y * h0i;
+                    ai += v[q].x * h0i + v[q].y * h0r;
+                    br += v[q + 1].x * h1r - v[q + 1].y * h1i;
+                    bi += v[q + 1].x * h1i + v[q + 1].y * h1r;
+                }
+            };
+            for (; c + 8 <= m; c += 8) {
+                double2 v[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) v[q] = V2[(size_t)(c + q) * ld];
+                four(v, c);
+                four(v + 4, c + 4);
+            }
+            for (; c + 4 <= m; c += 4) {
+                double2 v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = V2[(size_t)(c + q) * ld];
+                four(v, c);
+            }
+            for (; c < m; ++c) {
+                const double2 v = V2[(size_t)c * ld];
+                ar += v.x * hs[2 * c] - v.y * hs[2 * c + 1];
+                ai += v.x * hs[2 * c + 1] + v.y * hs[2 * c];
+            }
+            const double2 ri = reinterpret_cast<const double2 *>(rin)[row];
+            double2 ro;
+            ro.x = ri.x - (ar + br);
+            ro.y = ri.y - (ai + bi);
+            reinterpret_cast<double2 *>(rout)[row] = ro;
+            p = ro.x * ro.x + ro.y * ro.y;
+        }
+        if (k > 0) sm[k - 1][tg] = p;
+        __syncthreads();
+        if (k == 0) acc = ((p + sm[0][tg]) + sm[1][tg]) + sm[2][tg];
+    }
+    if (k == 0) {
+        acc = wave_sum(acc);
+        if (lane == 0) wt[w] = acc;
+    }
+    __syncthreads();
+    if (t == 0) {
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < kBlock / 64; ++i) s += wt[i];
+        part[blockIdx.x] = s;
+    }
+    if (out_hh && blockIdx.x == 0 && t == kWide - 1) {
+        double s = 0.0;
+        for (int i = 0; i < E * m; ++i) s += hs[i] * hs[i];
+        out_hh[0] = s;
+    }
+}
+
 // The recurrence and the first Gram-Schmidt projection of a real step in
 // one pass, over the FP32 shadow (VS = float) or the FP64 basis (VS =
 // double) (n <= kMaxGrid * kMinRowsUpd rows):
@@ -2277,6 +2445,19 @@ void launch_update(trlhip_ctx *c, int g, const VS *V, int c0, int m, const doubl
             pdst, o_hh, c->dscal + S_ALPHA);
 }
 
+// Whether a Gram-Schmidt update runs as k_update_wide: up to a block per CU.
+constexpr int kWideRows = 262144;
+bool update_wide_ok(int n) { return n <= kWideRows; }
+
+template <typename VS, int E>
+void launch_update_wide(int n, const VS *V, long ld, int m, const double *dh, const double *rin, double *rout,
+                        double *part, double *o_hh, hipStream_t s)
+{
+    const int g = grid_for(n, kMinRowsUpd, kMaxGrid);
+    KLAUNCH((k_update_wide<VS, E>), dim3(g), dim3(kWide), sizeof(double) * (size_t)E * m, s, n, V, ld, m, dh,
+            rin, rout, part, o_hh);
+}
+
 // rout = rin - V(:, c0:c0+m) dh; coefficient aslot (if >= 0) is the alpha
 // left in part_alpha (also stored to dscal[S_ALPHA]); ||rout||^2 -> o_rr2
 // and ||dh||^2 -> o_hh when requested.  dh == nullptr: coefficients
@@ -2294,7 +2475,18 @@ int run_update(trlhip_ctx *c, int c0, int m, const double *dh, int aslot, int ri
     const bool s32 = shadow && c->V32;
     {
         Timed t(kind, c->s, s32 ? (4.0 * m + 16.0) * c->n : (double)c->esz * c->n * (m + 2));
-        if (s32)
+        if (shadow && aslot < 0 && update_wide_ok(c->n)) {
+            const double *r0 = colp<double>(c, rin);
+            if (s32)
+                launch_update_wide<float, 1>(c->n, c->V32 + (size_t)c0 * c->ld, c->ld, m, dh, r0, colp<double>(c, rout),
+                                             pdst, o_hh, c->s);
+            else if (c->E == 1)
+                launch_update_wide<double, 1>(c->n, colp<double>(c, c0), c->ld, m, dh, r0, colp<double>(c, rout), pdst,
+                                              o_hh, c->s);
+            else
+                launch_update_wide<double, 2>(c->n, colp<double>(c, c0), c->ld, m, dh, r0, colp<double>(c, rout), pdst,
+                                              o_hh, c->s);
+        } else if (s32)
             launch_update<float, 1, 4>(c, g, c->V32, c0, m, dh, h0, aslot, rin, rout, o_hh, pdst);
         else if (c->E == 1 && shadow)  // the plain path's Gram-Schmidt update
             launch_update<double, 1, 4>(c, g, colp<double>(c, 0), c0, m, dh, h0, aslot, rin, rout,
@@ -5295,12 +5487,12 @@ namespace {
 constexpr int kNoAllocMaxCols = 256;  // TRLHIP_NOALLOC_MAX_COLS
 constexpr int kMaxDevices = 64;
 // partial rows: kProjGrid per coefficient, 2 coefficients per complex
-// column; then h (2 per column), the update partials, 8 scalars
+// column; then 8 scalars, h (2 per column), the update partials
 constexpr size_t kScrProj = 0;
-constexpr size_t kScrH = kScrProj + (size_t)kProjGrid * 2 * kNoAllocMaxCols;
+constexpr size_t kScrScal = kScrProj + (size_t)kProjGrid * 2 * kNoAllocMaxCols;
+constexpr size_t kScrH = kScrScal + 8;  // scalars and h go back in one copy
 constexpr size_t kScrUpd = kScrH + 2 * (size_t)kNoAllocMaxCols;
-constexpr size_t kScrScal = kScrUpd + kMaxGrid;
-constexpr size_t kScrCount = kScrScal + 8;
+constexpr size_t kScrCount = kScrUpd + kMaxGrid;
 }  // namespace
 
 static __device__ __align__(256) double scratch[kScrCount];
@@ -5353,10 +5545,14 @@ int noalloc_launch(int n, int m, const VS *V, long ld, double *r, double *scr, h
     if (hipGetLastError() != hipSuccess) return TRLHIP_EHIP;
     KLAUNCH(k_colsum, dim3(m * E), dim3(kBlock), 0, s, pproj, gx, dh);
     const int g = grid_for(n, kMinRowsUpd, kMaxGrid);
-    const size_t shm = sizeof(double) * (size_t)E * m;
-    KLAUNCH((k_update<VS, double, E, 4>), dim3(g), dim3(kBlock), shm, s, n, V, ld, 0, m,
-            (const double *)dh, 0.0, (const double *)nullptr, 0, -1, (const double *)r, r, pupd,
-            dscal + S_HH, dscal + S_ALPHA);
+    if (update_wide_ok(n)) {
+        launch_update_wide<VS, E>(n, V, ld, m, dh, r, r, pupd, dscal + S_HH, s);
+    } else {
+        const size_t shm = sizeof(double) * (size_t)E * m;
+        KLAUNCH((k_update<VS, double, E, 4>), dim3(g), dim3(kBlock), shm, s, n, V, ld, 0, m,
+                (const double *)dh, 0.0, (const double *)nullptr, 0, -1, (const double *)r, r, pupd,
+                dscal + S_HH, dscal + S_ALPHA);
+    }
     if (hipGetLastError() != hipSuccess) return TRLHIP_EHIP;
     return launch_sum(pupd, g, dscal + S_RR2, s);
 }
@@ -5385,12 +5581,11 @@ int trlhip_cgs_pass_noalloc(int n, int m, int vtype, const void *V, long ld, voi
     else
         rc = noalloc_launch<double, 2>(n, m, (const double *)V, ld, (double *)r, scr, s);
     if (rc) return rc;
-    const int E = vtype == TRLHIP_C128 ? 2 : 1;
-    double sc[3];
-    TRY(hipMemcpyAsync(sc, scr + kScrScal, sizeof sc, hipMemcpyDeviceToHost, s));
-    if (h_out)
-        TRY(hipMemcpyAsync(h_out, scr + kScrH, sizeof(double) * E * (size_t)m, hipMemcpyDeviceToHost, s));
+    const size_t nh = h_out ? (size_t)(vtype == TRLHIP_C128 ? 2 : 1) * m : 0;
+    double sc[8 + 2 * kNoAllocMaxCols];
+    TRY(hipMemcpyAsync(sc, scr + kScrScal, sizeof(double) * (nh ? 8 + nh : 3), hipMemcpyDeviceToHost, s));
     TRY(hipStreamSynchronize(s));
+    if (nh) memcpy(h_out, sc + 8, sizeof(double) * nh);
     if (hh) *hh = sc[S_HH];
     if (rr2) *rr2 = sc[S_RR2];
     return 0;
