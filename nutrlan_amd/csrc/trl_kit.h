@@ -50,6 +50,9 @@ void trlkit_householder(int n, double *a, double *d, double *e);
  * a <- eigenvectors, w <- eigenvalues ascending.  Returns 0 on success. */
 int trlkit_syev(int n, double *a, double *w);
 
+/* out = R x for an n x n matrix R of leading dimension ld. */
+void trlkit_apply(int n, const double *R, int ld, const double *x, double *out);
+
 /* Restatements of the reference's host decisions, same arguments. */
 void trlkit_convergence_test(int nd, double *lambda, double *res, int *tag,
                              trl_info *info);

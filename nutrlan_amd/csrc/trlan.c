@@ -452,11 +452,7 @@ static int lz_get_tvec(lz_t *z, int nd, int irot, int nrot, const double *alf,
         double *tmp = z->dsc;
         for (int j = 0; j < nlam; ++j) {
             double *y = yy + (size_t)j * nd + irot;
-            for (int r = 0; r < nrot; ++r) {
-                double s = 0.0;
-                for (int q = 0; q < nrot; ++q) s += z->rot[(size_t)q * nrot + r] * y[q];
-                tmp[r] = s;
-            }
+            trlkit_apply(nrot, z->rot, nrot, y, tmp);
             memcpy(y, tmp, sizeof(double) * (size_t)nrot);
         }
     }
@@ -1460,8 +1456,8 @@ static int lz_setup(lz_t *z, trl_matvec op, ztrl_matvec zop, trl_uo user_ortho, 
         __atomic_add_fetch(&g_ns_alloc, ta1 - ta0, __ATOMIC_RELAXED);
         __atomic_add_fetch(&g_ns_ctx, lz_ns() - ta1, __ATOMIC_RELAXED);
     }
-    /* a single real solve's inner steps run as chains in one kernel each
-     * where the operator allows (trlhip_step_cgs), up to the next
+    /* a single solve's inner steps run as chains (trlhip_step_cgs), in one
+     * kernel each where the operator and size allow, up to the next
      * convergence test or the end of the cycle;
      * batched real solves chain up to 8 inner steps per round (measured
      * on the batched 2D Anderson workload: 4 steps 8,344, 6: 8,560,
@@ -1469,7 +1465,7 @@ static int lz_setup(lz_t *z, trl_matvec op, ztrl_matvec zop, trl_uo user_ortho, 
      * host/device overlap coarser); TRLHIP_BATCH_CHAIN=k: at most k, 0 or
      * 1: one step per round */
     const char *ec = getenv("TRLHIP_BATCH_CHAIN");
-    z->chain = (z->A != NULL && !cplx) ? (b == NULL ? 32 : ec ? atoi(ec) : 8) : 0;
+    z->chain = z->A != NULL ? (b == NULL ? 32 : ec ? atoi(ec) : 8) : 0;
     if (z->chain < 2) z->chain = 0;
     return 1;
 }
