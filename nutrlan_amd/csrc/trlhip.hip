@@ -51,6 +51,7 @@ constexpr int kRowsBlk = kBlock;       // rows per SpMV row block (at most)
 constexpr int kMinRowsUpd = 4 * kBlock;
 constexpr int kMinSpmvRowBlocks = 1;
 constexpr int kChainMax = 32;  // Lanczos steps one batched context may record per round
+constexpr int kPhaseChain = 16;  // steps of a single solve queued at once (run_phases)
 // chain kernels (trl_chain.h): workgroups at most (their flags), basis
 // columns at most, the gate words after the flags, 32-bit words in all
 constexpr int kChainMaxWG = 256, kChainMaxCols = 192, kChainGate = 512, kChainSync = 640;
@@ -1368,10 +1369,9 @@ __device__ __forceinline__ void group_sums(const VS *Vc, long ld, int m, const d
 }
 
 template <typename VS, int E>
-__global__ __launch_bounds__(kWide) void k_update_wide(int n, const VS *__restrict__ V, long ld, int m,
-                                                       const double *__restrict__ h, const double *rin,
-                                                       double *rout, double *__restrict__ part,
-                                                       double *__restrict__ out_hh)
+__device__ __forceinline__ void update_wide_body(int n, const VS *__restrict__ V, long ld, int m,
+                                                 const double *__restrict__ h, const double *rin, double *rout,
+                                                 double *__restrict__ part, double *__restrict__ out_hh, int bid)
 {
     extern __shared__ double hs[];
     __shared__ double sm[3][4 * kBlock];
@@ -1379,7 +1379,7 @@ __global__ __launch_bounds__(kWide) void k_update_wide(int n, const VS *__restri
     const int t = threadIdx.x, tg = t & (kBlock - 1), k = t >> 8, lane = t & 63, w = t >> 6;
     for (int i = t; i < E * m; i += kWide) hs[i] = h[i];
     __syncthreads();
-    const int R0 = blockIdx.x * 4 * kBlock;
+    const int R0 = bid * 4 * kBlock;
     double acc = 0.0;
     if constexpr (E == 1) {
         const int row = R0 + 4 * tg;
@@ -1466,13 +1466,22 @@ __global__ __launch_bounds__(kWide) void k_update_wide(int n, const VS *__restri
         double s = 0.0;
 #pragma unroll
         for (int i = 0; i < kBlock / 64; ++i) s += wt[i];
-        part[blockIdx.x] = s;
+        part[bid] = s;
     }
-    if (out_hh && blockIdx.x == 0 && t == kWide - 1) {
+    if (out_hh && bid == 0 && t == kWide - 1) {
         double s = 0.0;
         for (int i = 0; i < E * m; ++i) s += hs[i] * hs[i];
         out_hh[0] = s;
     }
+}
+
+template <typename VS, int E>
+__global__ __launch_bounds__(kWide) void k_update_wide(int n, const VS *__restrict__ V, long ld, int m,
+                                                       const double *__restrict__ h, const double *rin,
+                                                       double *rout, double *__restrict__ part,
+                                                       double *__restrict__ out_hh)
+{
+    update_wide_body<VS, E>(n, V, ld, m, h, rin, rout, part, out_hh, blockIdx.x);
 }
 
 // The recurrence and the first Gram-Schmidt projection of a real step in
@@ -2692,6 +2701,7 @@ std::vector<int> row_blocks(int n, const int *rp)
 // Parameters of one recorded step (device copy, one per request).
 struct BDesc {
     int n, ld, jnd, np_alpha, g_upd, gx, gy, rm, rc0, nb;
+    int ncoef;            // projection coefficients: jnd, complex 2 jnd
     const int *rb, *rp, *ci;
     const double *val;
     const uint32_t *pk;   // packed nonzeros (kb_spmv_pk), with dg and tab
@@ -2850,7 +2860,7 @@ __global__ __launch_bounds__(kBlock) void kb_colsum(const BDesc *__restrict__ d,
     BATCH_LOCATE(BP_COLSUM)
     (void)nblk_;
     const int lane = threadIdx.x & 63, c = 4 * bid_ + (threadIdx.x >> 6);
-    if (c >= q.jnd) return;
+    if (c >= q.ncoef) return;
     const double *pc = q.part_proj + (size_t)c * q.gx;
     double t = 0.0;
 #pragma unroll
@@ -2869,6 +2879,47 @@ __global__ __launch_bounds__(kBlock) void kb_update(const BDesc *__restrict__ d,
     update_body<VS, double, 1, 4>(q.n, (const VS *)q.VG, q.ld, 0, q.jnd, q.dh, 0.0, nullptr, 0, -1,
                                   q.r, q.scratch, q.part_update, q.dscal + S_HH, nullptr, bid_,
                                   nblk_);
+}
+
+// The same update with 1024 threads a block, for a single solve's chains
+// (batch_run).
+template <typename VS, int E>
+__global__ __launch_bounds__(kWide) void kb_update_wide(const BDesc *__restrict__ d, const int *pre, int nreq)
+{
+    BATCH_LOCATE(BP_UPDATE)
+    (void)nblk_;
+    update_wide_body<VS, E>(q.n, (const VS *)q.VG, q.ld, q.jnd, q.dh, q.r, q.scratch, q.part_update,
+                            q.dscal + S_HH, bid_);
+}
+
+// Complex steps of a single solve's chains: the single-step kernels' bodies.
+__global__ __launch_bounds__(kBlock) void kbz_spmv(const BDesc *__restrict__ d, const int *pre, int nreq)
+{
+    BATCH_LOCATE_SPMV
+    spmv_stream_body<double, double, 2, true>(q.nb, q.rb, q.rp, q.ci, q.val, q.x, q.r, q.part_alpha, xs_, q.xq,
+                                              nullptr, bid_, nblk_);
+}
+
+__global__ __launch_bounds__(kBlock) void kbz_recur(const BDesc *__restrict__ d, const int *pre, int nreq)
+{
+    BATCH_LOCATE(BP_RECUR)
+    update_body<double, double, 2, 4, true>(q.n, q.V, q.ld, q.rc0, q.rm, q.rh, q.drh0 ? *q.drh0 : q.rh0,
+                                            q.part_alpha, q.np_alpha, q.rm - 1, q.r, q.r, q.part_recur,
+                                            nullptr, q.dscal + S_ALPHA, bid_, nblk_);
+}
+
+__global__ __launch_bounds__(kBlock) void kbz_proj(const BDesc *__restrict__ d, const int *pre, int nreq)
+{
+    BATCH_LOCATE(BP_PROJ)
+    proj_body<double, double, 2, 4, 4>(q.n, (const double *)q.VG, q.ld, 0, q.jnd, q.r, q.part_proj, q.gx,
+                                       q.gy, bid_, nblk_);
+}
+
+__global__ __launch_bounds__(kBlock) void kbz_update(const BDesc *__restrict__ d, const int *pre, int nreq)
+{
+    BATCH_LOCATE(BP_UPDATE)
+    update_body<double, double, 2, 4>(q.n, (const double *)q.VG, q.ld, 0, q.jnd, q.dh, 0.0, nullptr, 0, -1,
+                                      q.r, q.scratch, q.part_update, q.dscal + S_HH, nullptr, bid_, nblk_);
 }
 
 // Whether a chain follower runs: the solver's own decisions after a step
@@ -2957,6 +3008,9 @@ struct GroupInfo {
                  // CSR-stream, -2 / -3: 2D / 3D stencil)
     bool mixed;
     bool fused;         // recurrence and first projection in one kernel (recproj_ok)
+    int E;              // doubles per element (complex 2: a single solve's chain)
+    bool single;        // a single solve's chain: timed as its kernels
+    bool wide;          // its update's blocks have 1024 threads (update_wide_ok)
     int cb;             // projection columns per block, read once for the group
     size_t doff, poff;  // offsets into the staging arrays
     double bytes[BP_COUNT];
@@ -2982,7 +3036,8 @@ void batch_fill(const BatchStep *steps, int R, BDesc *desc, int *pre, GroupInfo 
         c->np_alpha = d.np_alpha;
         d.g_upd = grid_for(n, kMinRowsUpd, kMaxGrid);
         const int cb = gi.cb;
-        d.gx = gi.fused ? d.g_upd : proj_gx(c, jnd, cb, gi.mixed ? 4 : 8);  // fused: one block per row block
+        d.ncoef = gi.E * jnd;
+        d.gx = gi.fused ? d.g_upd : proj_gx(c, jnd, cb, gi.mixed ? 4 : 8 * gi.E);  // fused: one block per row block
         d.gy = gi.fused ? 1 : (jnd + cb - 1) / cb;
         if (st.first) {
             d.rm = jnd;
@@ -3038,23 +3093,23 @@ void batch_fill(const BatchStep *steps, int R, BDesc *desc, int *pre, GroupInfo 
         d.dres = c->dres;
         const int kind = spmv_kind_batch(A);
         const int spmv_wg = (kind == -2 || kind == -3) ? stencil_wgs(A) : d.np_alpha;
-        const int nb[BP_COUNT] = {spmv_wg, d.g_upd, d.gx * d.gy, (jnd + 3) / 4, d.g_upd, 1};
+        const int nb[BP_COUNT] = {spmv_wg, d.g_upd, d.gx * d.gy, (d.ncoef + 3) / 4, d.g_upd, 1};
         for (int ph = 0; ph < BP_COUNT; ++ph) {
             int *pp = pre + (size_t)ph * (R + 1);
             pp[i + 1] = pp[i] + nb[ph];
         }
-        const double vs = gi.mixed ? 4.0 : 8.0;
+        const double vs = gi.mixed ? 4.0 : 8.0 * gi.E, rs = 8.0 * gi.E;
         const double sb = spmv_kind_batch(A) == spmv_kind(A)
-                              ? spmv_bytes(A, 1, 8, 8)
+                              ? spmv_bytes(A, gi.E, 8, 8)
                               : 12.0 * (double)A->nnz + 4.0 * (n + 1) + 16.0 * n;
-        gi.bytes[BP_SPMV] += sb + (st.fuse ? (gi.mixed ? 12.0 : 8.0) * n : 0.0);
+        gi.bytes[BP_SPMV] += sb + (st.fuse ? (gi.mixed ? 12.0 : rs) * n : 0.0);
         if (gi.fused) {  // y, the recurrence columns, r written once; the shadow basis
-            gi.bytes[BP_PROJ] += 8.0 * n * (d.rm + 2) + vs * jnd * n;
+            gi.bytes[BP_PROJ] += rs * n * (d.rm + 2) + vs * jnd * n;
         } else {
-            gi.bytes[BP_RECUR] += 8.0 * n * (d.rm + 2);
-            gi.bytes[BP_PROJ] += (vs * jnd + 8.0) * n;
+            gi.bytes[BP_RECUR] += rs * n * (d.rm + 2);
+            gi.bytes[BP_PROJ] += (vs * jnd + rs) * n;
         }
-        gi.bytes[BP_UPDATE] += (vs * jnd + 16.0) * n;
+        gi.bytes[BP_UPDATE] += (vs * jnd + 2.0 * rs) * n;
         gi.maxrm = std::max(gi.maxrm, d.rm);
         gi.maxj = std::max(gi.maxj, jnd);
     }
@@ -3066,9 +3121,12 @@ int batch_run(hipStream_t s, const GroupInfo &gi, const BDesc *dd, const int *dp
 {
     const int R = gi.R;
     auto blocks = [&](int ph) { return dim3(hpre[(size_t)ph * (R + 1) + R]); };
+    const bool z = gi.E == 2;
     {
-        Timed t(TRLHIP_K_BSPMV, s, gi.bytes[BP_SPMV]);
-        switch (gi.lpr) {
+        Timed t(gi.single ? TRLHIP_K_SPMV : TRLHIP_K_BSPMV, s, gi.bytes[BP_SPMV]);
+        if (z)
+            KLAUNCH(kbz_spmv, blocks(BP_SPMV), dim3(kBlock), 0, s, dd, dp, R);
+        else switch (gi.lpr) {
         case -1: KLAUNCH(kb_spmv_pk, blocks(BP_SPMV), dim3(kBlock), 0, s, dd, dp, R); break;
         case -2: KLAUNCH((kb_spmv_st<2>), blocks(BP_SPMV), dim3(kBlock), 0, s, dd, dp, R); break;
         case -3: KLAUNCH((kb_spmv_st<3>), blocks(BP_SPMV), dim3(kBlock), 0, s, dd, dp, R); break;
@@ -3081,11 +3139,14 @@ int batch_run(hipStream_t s, const GroupInfo &gi, const BDesc *dd, const int *dp
         }
     }
     if (!gi.fused) {
-        Timed t(TRLHIP_K_BRECUR, s, gi.bytes[BP_RECUR]);
-        KLAUNCH(kb_recur, blocks(BP_RECUR), dim3(kBlock), sizeof(double) * gi.maxrm, s, dd, dp, R);
+        Timed t(gi.single ? TRLHIP_K_RECUR : TRLHIP_K_BRECUR, s, gi.bytes[BP_RECUR]);
+        if (z)
+            KLAUNCH(kbz_recur, blocks(BP_RECUR), dim3(kBlock), 2 * sizeof(double) * gi.maxrm, s, dd, dp, R);
+        else
+            KLAUNCH(kb_recur, blocks(BP_RECUR), dim3(kBlock), sizeof(double) * gi.maxrm, s, dd, dp, R);
     }
     {
-        Timed t(TRLHIP_K_BPROJ, s, gi.bytes[BP_PROJ]);
+        Timed t(gi.single ? TRLHIP_K_PROJ : TRLHIP_K_BPROJ, s, gi.bytes[BP_PROJ]);
 #define KB_PROJ_CB(CB)                                                                        \
     case CB:                                                                                  \
         if (gi.fused && gi.mixed)                                                             \
@@ -3099,7 +3160,9 @@ int batch_run(hipStream_t s, const GroupInfo &gi, const BDesc *dd, const int *dp
         else                                                                                  \
             KLAUNCH((kb_proj<double, CB>), blocks(BP_PROJ), dim3(kBlock), 0, s, dd, dp, R);   \
         break;
-        switch (gi.cb) {
+        if (z)
+            KLAUNCH(kbz_proj, blocks(BP_PROJ), dim3(kBlock), 0, s, dd, dp, R);
+        else switch (gi.cb) {
             KB_PROJ_CB(4)
             KB_PROJ_CB(16)
             default: KB_PROJ_CB(8)
@@ -3108,8 +3171,18 @@ int batch_run(hipStream_t s, const GroupInfo &gi, const BDesc *dd, const int *dp
     }
     KLAUNCH(kb_colsum, blocks(BP_COLSUM), dim3(kBlock), 0, s, dd, dp, R);
     {
-        Timed t(TRLHIP_K_BUPDATE, s, gi.bytes[BP_UPDATE]);
-        if (gi.mixed)
+        Timed t(gi.single ? TRLHIP_K_UPDATE : TRLHIP_K_BUPDATE, s, gi.bytes[BP_UPDATE]);
+        const size_t hsz = sizeof(double) * gi.E * gi.maxj;
+        const bool wide = gi.single && gi.wide;
+        if (z && wide)
+            KLAUNCH((kb_update_wide<double, 2>), blocks(BP_UPDATE), dim3(kWide), hsz, s, dd, dp, R);
+        else if (z)
+            KLAUNCH(kbz_update, blocks(BP_UPDATE), dim3(kBlock), hsz, s, dd, dp, R);
+        else if (wide && gi.mixed)
+            KLAUNCH((kb_update_wide<float, 1>), blocks(BP_UPDATE), dim3(kWide), hsz, s, dd, dp, R);
+        else if (wide)
+            KLAUNCH((kb_update_wide<double, 1>), blocks(BP_UPDATE), dim3(kWide), hsz, s, dd, dp, R);
+        else if (gi.mixed)
             KLAUNCH((kb_update<float>), blocks(BP_UPDATE), dim3(kBlock), sizeof(double) * gi.maxj, s,
                     dd, dp, R);
         else
@@ -3201,11 +3274,11 @@ struct StepsPlan {
 
 // Moves the steps that run as chains into the plan: all that fit, when
 // their rows are few enough.
-void chains_plan(const trlhip_batch *b, StepsPlan &P, std::vector<char> &taken)
+void chains_plan(const std::vector<BatchStep> &S, StepsPlan &P, std::vector<char> &taken)
 {
     long rows = 0;
     int maxn = 0;
-    for (const BatchStep &st : b->steps)
+    for (const BatchStep &st : S)
         if (st.ci == 0 && chain_fits_wg(st.c, st.A, st.jnd, 4, kBatchChainWG)) {
             rows += st.c->n;
             maxn = std::max(maxn, st.c->n);
@@ -3215,7 +3288,6 @@ void chains_plan(const trlhip_batch *b, StepsPlan &P, std::vector<char> &taken)
     // the device holds
     const int maxg = std::min(kBatchChainWG, device_cus() / 4);
     P.rw = rows <= 512 * 256 && maxn <= 512 * maxg ? 2 : 4;
-    const auto &S = b->steps;
     for (size_t i = 0; i < S.size(); ++i) {
         if (taken[i] || S[i].ci != 0) continue;
         const int rw0 = spmv_kind(S[i].A) <= -2 ? P.rw : 2;
@@ -3242,30 +3314,34 @@ void chains_plan(const trlhip_batch *b, StepsPlan &P, std::vector<char> &taken)
     }
 }
 
-void steps_plan(const trlhip_batch *b, StepsPlan &P)
+// single: one real or complex solve's chain, step by step (run_phases).
+void steps_plan(const std::vector<BatchStep> &steps, size_t ncbuf, StepsPlan &P, bool single = false)
 {
     auto &order = P.order;
     auto &groups = P.groups;
-    order.reserve(b->steps.size());
-    std::vector<char> taken(b->steps.size(), 0);
-    chains_plan(b, P, taken);
+    order.reserve(steps.size());
+    std::vector<char> taken(steps.size(), 0);
+    if (!single) chains_plan(steps, P, taken);
     size_t npre = 0;
     // chain position first: a context's follower runs after its step
     // before it, so all steps at position 0 launch first, then position 1 ...
     int maxci = 0;
-    for (const BatchStep &st : b->steps) maxci = std::max(maxci, st.ci);
+    for (const BatchStep &st : steps) maxci = std::max(maxci, st.ci);
     for (int ci = 0; ci <= maxci; ++ci)
-        for (size_t i = 0; i < b->steps.size(); ++i) {
-            if (taken[i] || b->steps[i].ci != ci) continue;
+        for (size_t i = 0; i < steps.size(); ++i) {
+            if (taken[i] || steps[i].ci != ci) continue;
             GroupInfo gi{};
-            gi.lpr = spmv_kind_batch(b->steps[i].A);
-            gi.mixed = b->steps[i].c->V32 != nullptr;
-            gi.fused = recproj_ok(b->steps[i].c);
-            gi.cb = g_proj_cb[gi.mixed ? 1 : 0].load(std::memory_order_relaxed);
+            gi.lpr = spmv_kind_batch(steps[i].A);
+            gi.mixed = steps[i].c->V32 != nullptr;
+            gi.fused = recproj_ok(steps[i].c);
+            gi.E = steps[i].c->E;
+            gi.single = single;
+            gi.wide = update_wide_ok(steps[i].c->n);
+            gi.cb = gi.E == 2 ? 4 : g_proj_cb[gi.mixed ? 1 : 0].load(std::memory_order_relaxed);
             gi.doff = order.size();
             gi.poff = npre;
-            for (size_t k = i; k < b->steps.size(); ++k) {
-                const BatchStep &st = b->steps[k];
+            for (size_t k = i; k < steps.size(); ++k) {
+                const BatchStep &st = steps[k];
                 if (!taken[k] && st.ci == ci && spmv_kind_batch(st.A) == gi.lpr &&
                     (st.c->V32 != nullptr) == gi.mixed && recproj_ok(st.c) == gi.fused) {
                     order.push_back(st);
@@ -3280,7 +3356,7 @@ void steps_plan(const trlhip_batch *b, StepsPlan &P)
     P.npre = npre;
     P.off_pre = up(sizeof(BDesc) * order.size());
     P.off_cb = up(P.off_pre + sizeof(int) * npre);
-    P.total = P.off_cb + sizeof(double) * b->cbuf.size();
+    P.total = P.off_cb + sizeof(double) * ncbuf;
     if (!P.cgroups.empty()) {
         size_t cpre = 0, flags = 0;
         for (StepsPlan::ChainGroup &cg : P.cgroups) {
@@ -3306,14 +3382,14 @@ void steps_plan(const trlhip_batch *b, StepsPlan &P)
 
 // Writes the plan's descriptors, prefix tables and coefficients into the
 // staging block (h: host, d: the device address it is copied to).
-void steps_fill(const trlhip_batch *b, StepsPlan &P, char *h, const char *d)
+void steps_fill(const std::vector<double> &cbuf, StepsPlan &P, char *h, const char *d)
 {
     BDesc *hdesc = reinterpret_cast<BDesc *>(h);
     int *hpre = reinterpret_cast<int *>(h + P.off_pre);
     const double *dcbuf = reinterpret_cast<const double *>(d + P.off_cb);
     for (GroupInfo &gi : P.groups)
         batch_fill(P.order.data() + gi.doff, gi.R, hdesc + gi.doff, hpre + gi.poff, gi, dcbuf);
-    if (!b->cbuf.empty()) memcpy(h + P.off_cb, b->cbuf.data(), sizeof(double) * b->cbuf.size());
+    if (!cbuf.empty()) memcpy(h + P.off_cb, cbuf.data(), sizeof(double) * cbuf.size());
     if (P.cgroups.empty()) return;
     memset(h + P.off_flags, 0, P.total - P.off_flags);
     ChainArgs *hd = reinterpret_cast<ChainArgs *>(h + P.off_ch);
@@ -3776,6 +3852,21 @@ int ops_launch(const OpsPlan &P, const char *h, const char *d, hipStream_t s)
 }
 
 
+// Grows a context's staging (h, d: pinned / device, cap bytes) to `bytes`.
+int staging_fit(size_t bytes, char *&h, char *&d, size_t &cap)
+{
+    if (bytes <= cap) return 0;
+    if (h) (void)hipHostFree(h);
+    if (d) (void)hipFree(d);
+    h = d = nullptr;
+    cap = 0;
+    const size_t ncap = bytes + bytes / 2 + 4096;
+    if (hipHostMalloc((void **)&h, ncap, 0) != hipSuccess || hipMalloc((void **)&d, ncap) != hipSuccess)
+        return TRLHIP_ENOMEM;
+    cap = ncap;
+    return 0;
+}
+
 // Runs recorded operations outside a batch: stage (h, d: pinned / device,
 // cap bytes, grown as needed), copy, launch.
 int ops_run(const std::vector<BatchOp> &ops, const std::vector<double> &ybuf, char *&h, char *&d,
@@ -3784,16 +3875,7 @@ int ops_run(const std::vector<BatchOp> &ops, const std::vector<double> &ybuf, ch
     OpsPlan P;
     ops_plan(ops, ybuf, P);
     const size_t bytes = P.bytes;
-    if (bytes > cap) {
-        if (h) (void)hipHostFree(h);
-        if (d) (void)hipFree(d);
-        h = d = nullptr;
-        cap = 0;
-        const size_t ncap = bytes + bytes / 2 + 4096;
-        if (hipHostMalloc((void **)&h, ncap, 0) != hipSuccess || hipMalloc((void **)&d, ncap) != hipSuccess)
-            return TRLHIP_ENOMEM;
-        cap = ncap;
-    }
+    if (int rc = staging_fit(bytes, h, d, cap)) return rc;
     ops_fill(P, ybuf, h, d);
     TRY(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, s));
     return ops_launch(P, h, d, s);
@@ -4701,6 +4783,62 @@ int trlhip_restart_step(trlhip_ctx *c, const trlhip_csr *A, int qa, const double
     return 0;
 }
 
+// The K - 1 followers of step st, appended to `steps` and set up in its
+// context for the solver to take.
+static void chain_followers(const BatchStep &st, int K, std::vector<BatchStep> &steps)
+{
+    trlhip_ctx *c = st.c;
+    for (int k = 1; k < K; ++k) {
+        BatchStep f{c, st.A, 0, st.rcol + k - 1, k >= 2 ? st.rcol + k - 2 : st.qa, st.rcol + k, st.jnd + k, 0.0,
+                    1, 1.0, -1, c->ncols, k, k + 1 < K, c->ch_kept, c->ch_ntot};
+        c->ch_qa[k] = f.qa;
+        c->ch_qb[k] = f.qb;
+        c->ch_rcol[k] = f.rcol;
+        c->ch_jnd[k] = f.jnd;
+        c->hres[hres_chain(c->ncols) + 7 * (size_t)(k - 1) + 4] = 0.0;  // set if it runs
+        steps.push_back(f);
+    }
+    c->ch_n = K;
+    c->ch_next = K > 1 ? 1 : 0;
+    c->ch_copy_ok = 0;
+}
+
+// Whether a single solve's chain runs step by step on the device
+// (run_phases): the batched kernels and their complex forms cover the
+// operator.
+static bool phases_fit(const trlhip_ctx *c, const trlhip_csr *A)
+{
+    return A && !c->batch && !A->pn_on && (c->E == 1 || !A->lpr);
+}
+
+// Runs a step and K - 1 followers of a single solve with a launch per phase
+// and step, queued at once: each follower's kernels read the go flag and the
+// normalisation the step before it left (chain_go in kb_sum2), so the host
+// waits once per chain instead of once per step.
+static int run_phases(trlhip_ctx *c, const trlhip_csr *A, int qa, int qb, double beta_prev, int jnd, int rcol,
+                      int K)
+{
+    BatchStep st{c, A, 0, qa, qb, rcol, jnd, beta_prev, 0, 1.0, -1, 0, 0, 1, c->ch_kept, c->ch_ntot};
+    if (c->pend_dst == qa && rcol != c->pend_src) {
+        st.fuse = 1;
+        st.fuse_s = c->pend_s;
+        st.fuse_src = c->pend_src;
+        c->pend_dst = -1;
+    } else if (int rc = settle(c)) {
+        return rc;
+    }
+    std::vector<BatchStep> steps{st};
+    chain_followers(st, K, steps);
+    const std::vector<double> none;
+    StepsPlan P;
+    steps_plan(steps, 0, P, true);
+    if (int rc = staging_fit(P.total, c->hops, c->dops, c->ocap)) return rc;
+    steps_fill(none, P, c->hops, c->dops);
+    TRY(hipMemcpyAsync(c->dops, c->hops, P.total, hipMemcpyHostToDevice, c->s));
+    if (int rc = steps_launch(c->s, P, c->hops, c->dops)) return rc;
+    return ctx_wait(c);
+}
+
 // Runs a step and up to K - 1 followers of a single real solve as one
 // kernel (k_chain); sets the followers up as a batch's recorded chain does.
 // Returns 1 when the step ran, 0 when it must run as ordinary kernels (the
@@ -4835,20 +4973,8 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
                 c->batch->cbuf.push_back(0.0);
             }
             c->batch->steps.push_back(st);
-            for (int k = 1; k < K; ++k) {
-                BatchStep f{c, A, 0, rcol + k - 1, k >= 2 ? rcol + k - 2 : qa, rcol + k, jnd + k, 0.0,
-                            1, 1.0, -1, c->ncols, k, k + 1 < K, c->ch_kept, c->ch_ntot};
-                c->ch_qa[k] = f.qa;
-                c->ch_qb[k] = f.qb;
-                c->ch_rcol[k] = f.rcol;
-                c->ch_jnd[k] = f.jnd;
-                c->hres[hres_chain(c->ncols) + 7 * (size_t)(k - 1) + 4] = 0.0;  // set if it runs
-                c->batch->steps.push_back(f);
-            }
+            chain_followers(st, K, c->batch->steps);
         }
-        c->ch_n = K;
-        c->ch_next = K > 1 ? 1 : 0;
-        c->ch_copy_ok = 0;
         c->hres[6] = 0.0;
         if (int rc = ctx_wait(c)) return rc;
         const volatile double *hr = c->hres;
@@ -4880,9 +5006,9 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
     if (int rc = batch_drain(c)) return rc;
     int K = first ? 1 : std::max(1, std::min(c->ch_budget, kChainMax));
     c->ch_budget = 0;
+    while (K > 1 && (!valid_col(c, rcol + K - 1) || jnd + K - 1 > c->ncols)) --K;
     if (chain_fits(c, A, jnd)) {
-        while (K > 1 && (!valid_col(c, rcol + K - 1) || jnd + K - 1 > c->ncols || jnd + K - 1 > kChainMaxCols))
-            --K;
+        while (K > 1 && jnd + K - 1 > kChainMaxCols) --K;
         const int ran = run_chain(c, A, first, qa, qb, beta_prev, beta, jnd, rcol, K);
         if (ran < 0) return ran;
         if (ran) {
@@ -4893,6 +5019,15 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
             out[3] = hr[S_RR2B];
             return 0;
         }
+    }
+    if (K > 1 && phases_fit(c, A)) {
+        if (int rc = run_phases(c, A, qa, qb, beta_prev, jnd, rcol, std::min(K, kPhaseChain))) return rc;
+        const volatile double *hr = c->hres;
+        out[0] = hr[S_ALPHA];
+        out[1] = hr[S_RR2];
+        out[2] = hr[S_HH];
+        out[3] = hr[S_RR2B];
+        return 0;
     }
     int rc;
     if (recproj_ok(c)) {
@@ -4957,7 +5092,7 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
 int trlhip_step_chain(trlhip_ctx *c, int steps, int kept, int ntot)
 {
     if (!c) return TRLHIP_EINVAL;
-    if (c->E != 1) return 0;
+    if (c->batch && c->E != 1) return 0;  // a batch's steps are real
     c->ch_budget = steps;
     c->ch_kept = kept;
     c->ch_ntot = ntot;
@@ -5377,7 +5512,7 @@ int trlhip_batch_launch(trlhip_batch *b)
             ops_plan(b->ops, b->ybuf, op);
             o_bytes = (op.bytes + 255) & ~(size_t)255;
         }
-        if (!b->steps.empty()) steps_plan(b, sp);
+        if (!b->steps.empty()) steps_plan(b->steps, b->cbuf.size(), sp);
         total = o_bytes + sp.total;
         if (total > b->scap) {
             // a kept staging pair that fits (the largest), else a new one
@@ -5414,7 +5549,7 @@ int trlhip_batch_launch(trlhip_batch *b)
         }
         if (!rc) {
             if (!b->ops.empty()) ops_fill(op, b->ybuf, b->hstg, b->dstg);
-            if (!b->steps.empty()) steps_fill(b, sp, b->hstg + o_bytes, b->dstg + o_bytes);
+            if (!b->steps.empty()) steps_fill(b->cbuf, sp, b->hstg + o_bytes, b->dstg + o_bytes);
             if (hipMemcpyAsync(b->dstg, b->hstg, total, hipMemcpyHostToDevice, b->s) != hipSuccess)
                 rc = TRLHIP_EHIP;
         }
