@@ -269,9 +269,21 @@ __device__ __forceinline__ double norm4(const double r[4], int row, int n)
     return acc;
 }
 
+// Four rows of a column as stored.
+__device__ __forceinline__ void res4(const float *p, float v[4])
+{
+    const f32x4 t = *reinterpret_cast<const f32x4 *>(p);
+    v[0] = t.x;
+    v[1] = t.y;
+    v[2] = t.z;
+    v[3] = t.w;
+}
+__device__ __forceinline__ void res4(const double *p, double v[4]) { load4(p, v); }
+
 // KIND as spmv_kind: -3 / -2 periodic stencils, -1 packed CSR, 0 CSR.  VS =
-// what the Gram-Schmidt pass reads (float: the FP32 shadow).
-template <int RW, int KIND, typename VS>
+// what the Gram-Schmidt pass reads (float: the FP32 shadow).  NRES = columns
+// per group (c mod 4 = k, c < 4 NRES) that stay in registers for the chain.
+template <int RW, int KIND, typename VS, int NRES = 0>
 __device__ __forceinline__ void chain_body(const ChainArgs &q, const int b)
 {
     constexpr int R = 256 * RW, NT = 256 * RW, NWAVE = 4 * RW;
@@ -329,6 +341,14 @@ __device__ __forceinline__ void chain_body(const ChainArgs &q, const int b)
     const int niter = kStencil ? 0 : (q.nb + g * RW - 1) / (g * RW);
     CsrPart<KIND> cur;
     if constexpr (!kStencil) cur.load(q, b * RW + (t >> 8), t & 255);
+    VS vres[NRES > 0 ? NRES : 1][4];
+#pragma unroll
+    for (int i = 0; i < NRES; ++i) {
+        const int c = 4 * i + k;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) vres[i][j] = 0;
+        if (c < jnd - 1) res4(VG + (size_t)c * q.ld, vres[i]);
+    }
     // q_b of the first step
     if (!q.first && q.qb >= 0)
         qbs[t] = srow < n ? q.V[(size_t)q.qb * q.ld + srow] : 0.0;
@@ -470,8 +490,26 @@ __device__ __forceinline__ void chain_body(const ChainArgs &q, const int b)
                     st_agent(q.part_recur + gw, a);
             }
         }
-        // ---- projection partials, chunks of CH columns over the groups
-        for (int cb = CH * k; cb < jnd; cb += 4 * CH) {
+        // ---- projection partials: the resident columns, then chunks of CH
+        // columns over the groups
+        if constexpr (NRES > 0) {
+            double p[NRES];
+#pragma unroll
+            for (int i = 0; i < NRES; ++i) {
+                if (qa == 4 * i + k)  // q_a joins the resident columns
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) vres[i][j] = (VS)qas[lrow + j];
+                p[i] = 0.0;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < NRES; ++i) p[i] += (double)vres[i][j] * r4[j];
+            const double tot = wave_transpose_sum<NRES>(p, lane);
+            const int c = 4 * (lane / (64 / NRES)) + k;
+            if (lane % (64 / NRES) == 0 && c < jnd && gw < nw) st_agent(q.part_proj + (size_t)c * nw + gw, tot);
+        }
+        for (int cb = 4 * NRES + CH * k; cb < jnd; cb += 4 * CH) {
             double p[CH];
             double v[CH][4];
 #pragma unroll
@@ -538,7 +576,12 @@ __device__ __forceinline__ void chain_body(const ChainArgs &q, const int b)
         __syncthreads();
         {
             double s[4] = {0.0, 0.0, 0.0, 0.0};
-            group_sums(VG, q.ld, jnd, hs, k, s);
+#pragma unroll
+            for (int i = 0; i < NRES; ++i)
+                if (4 * i < (jnd & ~7))
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) s[j] += (double)vres[i][j] * hs[4 * i + k];
+            group_sums<VS, NRES == 0>(VG, q.ld, jnd, hs, k, s, 4 * NRES);
             if (k > 0)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) pool[(k - 1) * R + lrow + j] = s[j];
@@ -620,10 +663,16 @@ __device__ __forceinline__ void chain_body(const ChainArgs &q, const int b)
     }
 }
 
+// 8 waves of a stencil in FP64 leave 64 registers free: the first 32 columns
+// are read once a chain and not twice a step (2-D lattice, n = 10^4: a solve
+// of 268 steps 6.15 -> 5.71 ms).  Elsewhere it costs more than it gives:
+// 16 waves and the batch's kernel spill, the CSR products need the
+// registers, and the conversion of FP32 columns is kept as doubles
+// (n = 181^2, mixed: 9.84 -> 10.48 ms with 32 columns).
 template <int RW, int KIND, typename VS>
 __global__ __launch_bounds__(256 * RW) void k_chain(ChainArgs q)
 {
-    chain_body<RW, KIND, VS>(q, blockIdx.x);
+    chain_body<RW, KIND, VS, RW == 2 && KIND <= -2 && std::is_same<VS, double>::value ? 8 : 0>(q, blockIdx.x);
 }
 
 // The chains of many solves in one launch.  At most one workgroup per CU is

@@ -1334,12 +1334,14 @@ __device__ __forceinline__ void ld4(const float *p, double v[4])
     v[3] = t.w;
 }
 __device__ __forceinline__ void ld4(const double *p, double v[4]) { load4(p, v); }
-template <typename VS>
-__device__ __forceinline__ void group_sums(const VS *Vc, long ld, int m, const double *hs, int k, double s[4])
+// With ZERO the sums start at 0; else they go on from column c, the first one
+// not in s yet (a multiple of 16; past the full groups only the tail is left).
+template <typename VS, bool ZERO = true>
+__device__ __forceinline__ void group_sums(const VS *Vc, long ld, int m, const double *hs, int k, double s[4],
+                                           int c = 0)
 {
-    s[0] = s[1] = s[2] = s[3] = 0.0;
+    if (ZERO) s[0] = s[1] = s[2] = s[3] = 0.0;
     const int full = m & ~7;
-    int c = 0;
     for (; c + 16 <= full; c += 16) {
         double v[4][4];
 #pragma unroll
@@ -1359,7 +1361,7 @@ __device__ __forceinline__ void group_sums(const VS *Vc, long ld, int m, const d
             for (int j = 0; j < 4; ++j) s[j] += v[i][j] * hs[c + 4 * i + k];
     }
     if (k == 0) {
-        for (; c < m; ++c) {
+        for (c = ZERO ? c : full; c < m; ++c) {
             double v[4];
             ld4(Vc + (size_t)c * ld, v);
 #pragma unroll
