@@ -500,7 +500,14 @@ __global__ __launch_bounds__(NB) void k_bwd32(Geo g, const bf16_t *__restrict__ 
 // 650 us each (now 17).
 constexpr int kDwW = 32, kDwRows = 8;
 constexpr int kTr = 18;               // dwords per channel: 36 pixels
-constexpr int kDwBlocks = 256;        // blocks (4 waves each, a partial per wave)
+constexpr int kDwBlocks = 256;        // blocks (4 waves each)
+// Partials of the four layers: a row per block (layers 3 and 2), per wave
+// (4 and 1), and where each starts.
+constexpr int kRowMid = C * T * C + C, kRowEdge = C * T + C;
+constexpr long kPart3 = 0, kPart2 = kPart3 + (long)kDwBlocks * kRowMid,
+               kPart4 = kPart2 + (long)kDwBlocks * kRowMid,
+               kPart1 = kPart4 + (long)kDwBlocks * (NB / 64) * kRowEdge,
+               kPartCount = kPart1 + (long)kDwBlocks * (NB / 64) * kRowEdge;
 
 __host__ __device__ inline long dw_tasks(const Geo &g)
 {
@@ -557,14 +564,17 @@ __device__ __forceinline__ bf16x8 frag(const uint32_t d[4])
 // Weight gradient dW[co][t][ci] = sum_p dY[p][co] X[nbr(p,t)][ci] of a
 // 32 -> 32 layer: M = co, N = ci.  Three rows of X stay in LDS (a row
 // serves the dY rows above, at and below it); a lane reads 12 pixels of a
-// channel and shifts them by one for the left and right taps.  The wave's
-// partial (co, t, ci) and bias sums (a product with ones) go to
-// part[4 blockIdx + wave].
+// channel and shifts them by one for the left and right taps.  The block's
+// partial (co, t, ci) and bias sums (a product with ones), its four waves
+// added in FP64, go to part[blockIdx]: a partial per wave was 38 MB to write
+// and read again, more than the activations of 64 images of 64 x 64 (34).
 __global__ __launch_bounds__(NB) void k_dw32(Geo g, const bf16_t *__restrict__ dy,
                                              const bf16_t *__restrict__ x, float *__restrict__ part)
 {
     constexpr int NW = C * T * C;
+    constexpr int kSr = C + 4;
     __shared__ __align__(16) uint32_t lds[NB / 64][4][C * kTr];
+    __shared__ float bs[NB / 64][C];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int m = lane & 15, kq = lane >> 4;
     const int pp = lane >> 2, cg = lane & 3;
@@ -665,23 +675,47 @@ __global__ __launch_bounds__(NB) void k_dw32(Geo g, const bf16_t *__restrict__ d
             __builtin_amdgcn_wave_barrier();
         }
     }
-    float *out = part + ((long)blockIdx.x * (NB / 64) + wv) * (NW + C);
+    // the four waves' sums, tap by tap through the two halves of the LDS
+    // (rows of 36 put a wave's writes on different banks)
+    static_assert(2 * (NB / 64) * C * kSr * sizeof(float) == sizeof(lds), "two taps' sums of four waves");
+    float *sums = reinterpret_cast<float *>(&lds[0][0][0]);
+    if (m == 0)
 #pragma unroll
-    for (int t = 0; t < T; ++t)
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bs[wv][16 * mt + 4 * kq + i] = bacc[mt][i];
+    __syncthreads();
+    float *out = part + (long)blockIdx.x * (NW + C);
+    const int co = threadIdx.x / (C / 4), ci = 4 * (threadIdx.x % (C / 4));
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        float *b = sums + (t & 1) * (NB / 64) * C * kSr;
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
             for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int co = 16 * mt + 4 * kq + i, ci = 16 * nt + m;
-                    out[((long)co * T + t) * C + ci] = acc[t][mt][nt][i];
-                }
-    if (m == 0)
+                for (int i = 0; i < 4; ++i)
+                    b[(wv * C + 16 * mt + 4 * kq + i) * kSr + 16 * nt + m] = acc[t][mt][nt][i];
+        __syncthreads();
+        double s[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
+        for (int w = 0; w < NB / 64; ++w) {
+            const f4 v = *reinterpret_cast<const f4 *>(b + (w * C + co) * kSr + ci);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) out[NW + 16 * mt + 4 * kq + i] = bacc[mt][i];
+            for (int i = 0; i < 4; ++i) s[i] += v[i];
+        }
+        f4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = (float)s[i];
+        *reinterpret_cast<f4 *>(out + (co * T + t) * C + ci) = o;
+    }
+    if (threadIdx.x < C) {
+        double s = 0.0;
+#pragma unroll
+        for (int w = 0; w < NB / 64; ++w) s += bs[w][threadIdx.x];
+        out[NW + threadIdx.x] = (float)s;
+    }
 }
 
 // Weight gradients of the layers with a one-channel side: M = the 32
@@ -775,29 +809,55 @@ __global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict_
     }
 }
 
-// out[j] = sum_b part[b][j] over nb rows of stride len, in FP64: a block
-// takes 64 columns, its 16 groups of 64 threads every 16th row, and the
-// groups' sums are added in order (1024 rows of 9,248: 155 us with a thread
-// per column, now 6).
+// grad = the sums over the partials' rows, in FP64, of all four layers in one
+// launch: a block takes 64 columns of a layer, its 16 groups of 64 threads
+// every 16th row, and the groups' sums are added in order.  (A launch per
+// layer: 24 us and the gaps between them, of 340 for 64 images of 64 x 64.)
 constexpr int kRedGroups = 16;
-__global__ __launch_bounds__(64 * kRedGroups) void k_reduce(const float *__restrict__ part, int nb, int len,
-                                                            int stride, float *__restrict__ out)
+struct RedSeg {
+    long part;
+    int nb, len, stride, out, blk0;
+};
+struct RedArgs {
+    RedSeg s[4];
+    int blocks;
+};
+constexpr RedArgs red_args()
 {
+    RedArgs a{};
+    a.s[0] = {kPart3, kDwBlocks, kRowMid, kRowMid, OW3, 0};
+    a.s[1] = {kPart2, kDwBlocks, kRowMid, kRowMid, OW2, 0};
+    a.s[2] = {kPart4, kDwBlocks * (NB / 64), C * T + 1, kRowEdge, OW4, 0};  // layer 4 has one bias
+    a.s[3] = {kPart1, kDwBlocks * (NB / 64), kRowEdge, kRowEdge, OW1, 0};
+    for (int i = 0; i < 4; ++i) {
+        a.s[i].blk0 = a.blocks;
+        a.blocks += (a.s[i].len + 63) / 64;
+    }
+    return a;
+}
+__global__ __launch_bounds__(64 * kRedGroups) void k_reduce(const float *__restrict__ part, float *__restrict__ grad)
+{
+    constexpr RedArgs a = red_args();
     __shared__ double sm[kRedGroups][64];
     const int c = threadIdx.x & 63, gr = threadIdx.x >> 6;
-    const int j = blockIdx.x * 64 + c;
+    RedSeg q = a.s[0];
+#pragma unroll
+    for (int i = 1; i < 4; ++i)
+        if ((int)blockIdx.x >= a.s[i].blk0) q = a.s[i];
+    const int j = ((int)blockIdx.x - q.blk0) * 64 + c;
     double s = 0.0;
-    if (j < len) {
+    if (j < q.len) {
+        const float *p = part + q.part + j;
 #pragma unroll 8
-        for (int b = gr; b < nb; b += kRedGroups) s += part[(long)b * stride + j];
+        for (int b = gr; b < q.nb; b += kRedGroups) s += p[(long)b * q.stride];
     }
     sm[gr][c] = s;
     __syncthreads();
-    if (gr == 0 && j < len) {
+    if (gr == 0 && j < q.len) {
         double t = 0.0;
 #pragma unroll
         for (int i = 0; i < kRedGroups; ++i) t += sm[i][c];
-        out[j] = (float)t;
+        grad[q.out + j] = (float)t;
     }
 }
 
@@ -878,7 +938,7 @@ int ensure(trlnet *t, long np, int nimg)
         NTRY(hipMalloc((void **)&t->d2, sizeof(bf16_t) * C * np));
         t->cap = np;
     }
-    const long need = (long)kDwBlocks * 4 * (C * T * C + C);
+    const long need = kPartCount;
     if (need > t->partcap) {
         if (t->part) (void)hipFree(t->part);
         t->partcap = 0;
@@ -968,27 +1028,20 @@ int forward_groups(trlnet *t, int ngroups, const int *nimg, const int *h, const 
 int backward(trlnet *t, const Geo &g, double *loss)
 {
     const int gb = (int)conv_blocks(g);
-    const int NW = C * T * C + C, NV = C * T + C, np = kDwBlocks * (NB / 64);
     const dim3 dwb(kDwBlocks), blk(NB);
-    auto reduce = [&](int len, int stride, float *out) {
-        hipLaunchKernelGGL(k_reduce, dim3((len + 63) / 64), dim3(64 * kRedGroups), 0, t->s, t->part, np, len, stride, out);
-    };
     hipLaunchKernelGGL(k_loss, dim3(g.nimg), blk, 0, t->s, g, t->o, t->tg, t->dO, t->lpart);
-    // layer 4 (its gradient ends with the one bias)
-    hipLaunchKernelGGL((k_dw_edge<true>), dwb, blk, 0, t->s, g, t->a3, t->dO, t->part);
-    reduce(C * T + 1, NV, t->grad + OW4);
+    // layer 4
+    hipLaunchKernelGGL((k_dw_edge<true>), dwb, blk, 0, t->s, g, t->a3, t->dO, t->part + kPart4);
     hipLaunchKernelGGL(k_bwd4, dim3(gb), blk, 0, t->s, g, t->dO, t->wb + OW4, t->a3, t->d2);
     // layer 3: dY = d2 (for a3), X = a2
-    hipLaunchKernelGGL(k_dw32, dwb, blk, 0, t->s, g, t->d2, t->a2, t->part);
-    reduce(NW, NW, t->grad + OW3);
+    hipLaunchKernelGGL(k_dw32, dwb, blk, 0, t->s, g, t->d2, t->a2, t->part + kPart3);
     hipLaunchKernelGGL(k_bwd32, dim3(gb), blk, 0, t->s, g, t->d2, t->wt3, t->a2, t->d1);
     // layer 2: dY = d1 (for a2), X = a1
-    hipLaunchKernelGGL(k_dw32, dwb, blk, 0, t->s, g, t->d1, t->a1, t->part);
-    reduce(NW, NW, t->grad + OW2);
+    hipLaunchKernelGGL(k_dw32, dwb, blk, 0, t->s, g, t->d1, t->a1, t->part + kPart2);
     hipLaunchKernelGGL(k_bwd32, dim3(gb), blk, 0, t->s, g, t->d1, t->wt2, t->a1, t->d2);
     // layer 1: dY = d2 (for a1), X = potential
-    hipLaunchKernelGGL((k_dw_edge<false>), dwb, blk, 0, t->s, g, t->d2, t->x, t->part);
-    reduce(NV, NV, t->grad + OW1);
+    hipLaunchKernelGGL((k_dw_edge<false>), dwb, blk, 0, t->s, g, t->d2, t->x, t->part + kPart1);
+    hipLaunchKernelGGL(k_reduce, dim3(red_args().blocks), dim3(64 * kRedGroups), 0, t->s, t->part, t->grad);
     if (hipGetLastError() != hipSuccess) return TRLNET_EHIP;
     std::vector<double> lp((size_t)g.nimg);
     NTRY(hipMemcpyAsync(lp.data(), t->lpart, sizeof(double) * g.nimg, hipMemcpyDeviceToHost, t->s));
