@@ -16,8 +16,8 @@
 // elements 8*(l/16) .. +7, B column l%16 with the same K elements, result
 // D[4*(l/16) + i][l%16] in accumulator element i.
 //
-// A wave takes a strip of 16 pixels of one image row and walks down kRows
-// rows: each input row is loaded once (three column shifts) and feeds the
+// A wave takes a strip of 16 pixels of one image row and walks down up to
+// kRows rows: each input row is loaded once (three column shifts) and feeds the
 // three output rows that use it, the layer's weights stay in registers, and
 // the weights are the A operand, so a lane holds four consecutive channels
 // of one pixel and stores them together.  What bounds the forward is the
@@ -27,6 +27,7 @@
 // first and last layers 0.54 and 0.44, now 0.18 each.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdint>
@@ -44,7 +45,7 @@ constexpr int C = 32;          // hidden channels
 constexpr int T = 9;           // 3x3 taps
 constexpr int NB = 256;        // threads per block
 constexpr int kStrip = 16;     // pixels of a row per wave
-constexpr int kRows = 8;       // rows a wave walks
+constexpr int kRows = 8;       // rows a wave walks at most
 
 // parameter offsets in the flat FP32 vector
 constexpr int OW1 = 0, OB1 = OW1 + C * T;             // W1[co][t]
@@ -78,6 +79,7 @@ __device__ inline __bf16 as_bf(bf16_t h) { return __builtin_bit_cast(__bf16, h);
 struct Geo {
     int nimg, h, w;
     long np;  // pixels
+    int rows;  // rows a wave of a convolution walks (conv_rows)
 };
 
 __device__ inline bf16x8 load8(const bf16_t *p)
@@ -90,9 +92,32 @@ __device__ inline bf16x8 zero8() { return __builtin_bit_cast(bf16x8, uint4{0, 0,
 
 // Wave tasks of a convolution: strips x row segments of every image.
 __host__ __device__ inline int strips_of(int w) { return (w + kStrip - 1) / kStrip; }
-__host__ __device__ inline int segs_of(int h) { return (h + kRows - 1) / kRows; }
-__host__ __device__ inline long conv_tasks(const Geo &g) { return (long)g.nimg * strips_of(g.w) * segs_of(g.h); }
+__host__ __device__ inline int segs_of(int h, int rows) { return (h + rows - 1) / rows; }
+__host__ __device__ inline long conv_tasks(const Geo &g)
+{
+    return (long)g.nimg * strips_of(g.w) * segs_of(g.h, g.rows);
+}
 inline long conv_blocks(const Geo &g) { return (conv_tasks(g) + NB / 64 - 1) / (NB / 64); }
+
+// Rows a wave walks for the images of all groups of a launch: shorter walks
+// while there is at most a wave per SIMD.  Forward and backward of 8 images
+// of 64 x 64 (1,024 waves of 2 rows, 256 of 8) 229 -> 196 us; with limits of
+// 3,072 to 8,192 waves 32 and 64 such images are 0 to 9 % slower: every wave
+// loads the layer's weights and two more rows.
+constexpr long kConvWaves = 1024;
+constexpr int kMinRows = 2;
+inline int conv_rows(int ngroups, const int *nimg, const int *h, const int *w)
+{
+    int rows = kRows;
+    while (rows > kMinRows) {
+        long n = 0;
+        for (int i = 0; i < ngroups; ++i) n += (long)nimg[i] * strips_of(w[i]) * segs_of(h[i], rows / 2);
+        if (n > kConvWaves) break;
+        rows /= 2;
+    }
+    return rows;
+}
+inline Geo geo_of(int nimg, int h, int w, int rows) { return Geo{nimg, h, w, (long)nimg * h * w, rows}; }
 
 // A wave's strip: its image's first pixel, columns, rows [y0, y1).
 struct Strip {
@@ -104,7 +129,7 @@ struct Strip {
 __device__ __forceinline__ bool strip_of(const Geo &g, long task, Strip &s)
 {
     if (task >= conv_tasks(g)) return false;
-    const int ns = strips_of(g.w), per = ns * segs_of(g.h);
+    const int ns = strips_of(g.w), per = ns * segs_of(g.h, g.rows);
     const int img = (int)(task / per), r = (int)(task - (long)img * per);
     const int seg = r / ns, strip = r - seg * ns;
     const int x = strip * kStrip + (int)(threadIdx.x & 15);
@@ -114,8 +139,8 @@ __device__ __forceinline__ bool strip_of(const Geo &g, long task, Strip &s)
     s.xc[1] = s.x;
     s.xc[2] = s.x == g.w - 1 ? 0 : s.x + 1;
     s.base = (long)img * g.h * g.w;
-    s.y0 = seg * kRows;
-    s.y1 = s.y0 + kRows < g.h ? s.y0 + kRows : g.h;
+    s.y0 = seg * g.rows;
+    s.y1 = s.y0 + g.rows < g.h ? s.y0 + g.rows : g.h;
     return true;
 }
 
@@ -502,7 +527,7 @@ constexpr int kDwW = 32, kDwRows = 8;
 constexpr int kTr = 18;               // dwords per channel: 36 pixels
 constexpr int kDwBlocks = 256;        // blocks (4 waves each)
 // Partials of the four layers: a row per block (layers 3 and 2), per wave
-// (4 and 1), and where each starts.
+// (4 and 1), and where each starts.  Blocks without a strip are not launched.
 constexpr int kRowMid = C * T * C + C, kRowEdge = C * T + C;
 constexpr long kPart3 = 0, kPart2 = kPart3 + (long)kDwBlocks * kRowMid,
                kPart4 = kPart2 + (long)kDwBlocks * kRowMid,
@@ -816,7 +841,7 @@ __global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict_
 constexpr int kRedGroups = 16;
 struct RedSeg {
     long part;
-    int nb, len, stride, out, blk0;
+    int rows, len, stride, out, blk0;  // rows a block of the gradient kernel leaves
 };
 struct RedArgs {
     RedSeg s[4];
@@ -825,17 +850,18 @@ struct RedArgs {
 constexpr RedArgs red_args()
 {
     RedArgs a{};
-    a.s[0] = {kPart3, kDwBlocks, kRowMid, kRowMid, OW3, 0};
-    a.s[1] = {kPart2, kDwBlocks, kRowMid, kRowMid, OW2, 0};
-    a.s[2] = {kPart4, kDwBlocks * (NB / 64), C * T + 1, kRowEdge, OW4, 0};  // layer 4 has one bias
-    a.s[3] = {kPart1, kDwBlocks * (NB / 64), kRowEdge, kRowEdge, OW1, 0};
+    a.s[0] = {kPart3, 1, kRowMid, kRowMid, OW3, 0};
+    a.s[1] = {kPart2, 1, kRowMid, kRowMid, OW2, 0};
+    a.s[2] = {kPart4, NB / 64, C * T + 1, kRowEdge, OW4, 0};  // layer 4 has one bias
+    a.s[3] = {kPart1, NB / 64, kRowEdge, kRowEdge, OW1, 0};
     for (int i = 0; i < 4; ++i) {
         a.s[i].blk0 = a.blocks;
         a.blocks += (a.s[i].len + 63) / 64;
     }
     return a;
 }
-__global__ __launch_bounds__(64 * kRedGroups) void k_reduce(const float *__restrict__ part, float *__restrict__ grad)
+__global__ __launch_bounds__(64 * kRedGroups) void k_reduce(const float *__restrict__ part, int dwb,
+                                                            float *__restrict__ grad)
 {
     constexpr RedArgs a = red_args();
     __shared__ double sm[kRedGroups][64];
@@ -849,7 +875,7 @@ __global__ __launch_bounds__(64 * kRedGroups) void k_reduce(const float *__restr
     if (j < q.len) {
         const float *p = part + q.part + j;
 #pragma unroll 8
-        for (int b = gr; b < q.nb; b += kRedGroups) s += p[(long)b * q.stride];
+        for (int b = gr; b < q.rows * dwb; b += kRedGroups) s += p[(long)b * q.stride];
     }
     sm[gr][c] = s;
     __syncthreads();
@@ -999,10 +1025,11 @@ int forward_groups(trlnet *t, int ngroups, const int *nimg, const int *h, const 
     }
     GroupGeo *gg = reinterpret_cast<GroupGeo *>(t->hgeo);
     int *pre = reinterpret_cast<int *>(t->hgeo + off_pre);
+    const int rows = conv_rows(ngroups, nimg, h, w);
     long off = 0;
     pre[0] = 0;
     for (int i = 0; i < ngroups; ++i) {
-        const Geo g{nimg[i], h[i], w[i], (long)nimg[i] * h[i] * w[i]};
+        const Geo g = geo_of(nimg[i], h[i], w[i], rows);
         gg[i] = GroupGeo{g, off};
         const long nb = (long)pre[i] + conv_blocks(g);
         if (nb > 0x7fffffffL) return TRLNET_EINVAL;
@@ -1028,7 +1055,8 @@ int forward_groups(trlnet *t, int ngroups, const int *nimg, const int *h, const 
 int backward(trlnet *t, const Geo &g, double *loss)
 {
     const int gb = (int)conv_blocks(g);
-    const dim3 dwb(kDwBlocks), blk(NB);
+    const int ndw = (int)std::min<long>(kDwBlocks, (dw_tasks(g) + NB / 64 - 1) / (NB / 64));
+    const dim3 dwb(ndw), blk(NB);
     hipLaunchKernelGGL(k_loss, dim3(g.nimg), blk, 0, t->s, g, t->o, t->tg, t->dO, t->lpart);
     // layer 4
     hipLaunchKernelGGL((k_dw_edge<true>), dwb, blk, 0, t->s, g, t->a3, t->dO, t->part + kPart4);
@@ -1041,7 +1069,8 @@ int backward(trlnet *t, const Geo &g, double *loss)
     hipLaunchKernelGGL(k_bwd32, dim3(gb), blk, 0, t->s, g, t->d1, t->wt2, t->a1, t->d2);
     // layer 1: dY = d2 (for a1), X = potential
     hipLaunchKernelGGL((k_dw_edge<false>), dwb, blk, 0, t->s, g, t->d2, t->x, t->part + kPart1);
-    hipLaunchKernelGGL(k_reduce, dim3(red_args().blocks), dim3(64 * kRedGroups), 0, t->s, t->part, t->grad);
+    hipLaunchKernelGGL(k_reduce, dim3(red_args().blocks), dim3(64 * kRedGroups), 0, t->s, t->part, ndw,
+                       t->grad);
     if (hipGetLastError() != hipSuccess) return TRLNET_EHIP;
     std::vector<double> lp((size_t)g.nimg);
     NTRY(hipMemcpyAsync(lp.data(), t->lpart, sizeof(double) * g.nimg, hipMemcpyDeviceToHost, t->s));
@@ -1154,7 +1183,7 @@ int trlnet_set_params(trlnet *t, const float *in, int n)
 int trlnet_forward(trlnet *t, int nimg, int h, int w, const float *in, float *out)
 {
     if (!t || !in || !out || !geo_ok(nimg, h, w)) return TRLNET_EINVAL;
-    const Geo g{nimg, h, w, (long)nimg * h * w};
+    const Geo g = geo_of(nimg, h, w, conv_rows(1, &nimg, &h, &w));
     if (int rc = upload(t, g, in, nullptr)) return rc;
     if (int rc = forward(t, g)) return rc;
     NTRY(hipMemcpyAsync(out, t->o, sizeof(float) * g.np, hipMemcpyDeviceToHost, t->s));
@@ -1282,7 +1311,7 @@ int trlnet_loss_grad(trlnet *t, int nimg, int h, int w, const float *in, const f
                      float *loss, float *grad)
 {
     if (!t || !in || !target || !geo_ok(nimg, h, w)) return TRLNET_EINVAL;
-    const Geo g{nimg, h, w, (long)nimg * h * w};
+    const Geo g = geo_of(nimg, h, w, conv_rows(1, &nimg, &h, &w));
     if (int rc = upload(t, g, in, target)) return rc;
     if (int rc = forward(t, g)) return rc;
     double l = 0.0;

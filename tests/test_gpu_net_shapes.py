@@ -70,3 +70,10 @@ def test_forward_and_gradients(gpu_lib, shape):
         ref = max(np.linalg.norm(b), 1e-2 * np.abs(blocks[6]).max())
         assert np.linalg.norm(d - b) <= TOL * ref, (at, np.linalg.norm(d - b) / ref)
     net.close()
+
+
+@pytest.mark.parametrize("shape", [(130, 17, 33), (90, 33, 18), (33, 30, 47)])
+def test_more_waves(gpu_lib, shape):
+    """Batches of more waves than SIMDs, which walk 8 or 4 rows each (those
+    above walk 2 or 4); ragged in both directions."""
+    test_forward_and_gradients(gpu_lib, shape)
