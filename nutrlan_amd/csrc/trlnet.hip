@@ -101,7 +101,7 @@ inline long conv_blocks(const Geo &g) { return (conv_tasks(g) + NB / 64 - 1) / (
 
 // Rows a wave walks for the images of all groups of a launch: shorter walks
 // while there is at most a wave per SIMD.  Forward and backward of 8 images
-// of 64 x 64 (1,024 waves of 2 rows, 256 of 8) 229 -> 196 us; with limits of
+// of 64 x 64 (1,024 waves of 2 rows, 256 of 8) 229 -> 207 us; with limits of
 // 3,072 to 8,192 waves 32 and 64 such images are 0 to 9 % slower: every wave
 // loads the layer's weights and two more rows.
 constexpr long kConvWaves = 1024;
