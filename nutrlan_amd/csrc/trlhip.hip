@@ -2232,7 +2232,8 @@ int chain_rw(const trlhip_csr *A) { return spmv_kind(A) <= -2 && A->n > 32768 ? 
 // row blocks a thread group (denser operators keep the wider SpMV kernel).
 // Against the single-step kernels, per solve: n = 1,000 9.3 -> 5.1 ms, n =
 // 10,000 (2D) 11.7 -> 6.4, n = 62,500 16.7 -> 9.9, n = 262,144 24.9 -> 23.3;
-// random rows n = 50,001 69 -> 48 ms.
+// random rows n = 50,001 69 -> 48 ms (with the faster restarts and columns
+// kept in registers since: 4.6, 5.4 and, for the random rows, 44 ms).
 constexpr int kChainCsrIter = 4;
 bool chain_fits_wg(const trlhip_ctx *c, const trlhip_csr *A, int jnd, int rw, int maxg)
 {
