@@ -2247,6 +2247,11 @@ bool chain_fits(const trlhip_ctx *c, const trlhip_csr *A, int jnd)
 {
     return !c->batch && A && chain_fits_wg(c, A, jnd, chain_rw(A), kChainMaxWG);
 }
+// The form of a step that chain kernels take, the solver's: q_a is the last
+// basis column and r goes to the column after it.  They keep q_a in LDS and,
+// some of them, the columns before it in registers; the step kernels, which
+// read every column from memory, run the others trlhip_step_cgs accepts.
+bool chain_form(int qa, int jnd, int rcol) { return qa == jnd - 1 && rcol == jnd; }
 
 // A batch's launch runs its steps as chains (kb_chain) while the solves that
 // fit hold at most kBatchChainRows rows together.  The device holds 262,144
@@ -3282,7 +3287,8 @@ void chains_plan(const std::vector<BatchStep> &S, StepsPlan &P, std::vector<char
     long rows = 0;
     int maxn = 0;
     for (const BatchStep &st : S)
-        if (st.ci == 0 && chain_fits_wg(st.c, st.A, st.jnd, 4, kBatchChainWG)) {
+        if (st.ci == 0 && chain_form(st.qa, st.jnd, st.rcol) &&
+            chain_fits_wg(st.c, st.A, st.jnd, 4, kBatchChainWG)) {
             rows += st.c->n;
             maxn = std::max(maxn, st.c->n);
         }
@@ -3294,14 +3300,14 @@ void chains_plan(const std::vector<BatchStep> &S, StepsPlan &P, std::vector<char
     for (size_t i = 0; i < S.size(); ++i) {
         if (taken[i] || S[i].ci != 0) continue;
         const int rw0 = spmv_kind(S[i].A) <= -2 ? P.rw : 2;
-        if (!chain_fits_wg(S[i].c, S[i].A, S[i].jnd, rw0, maxg)) continue;
+        if (!chain_form(S[i].qa, S[i].jnd, S[i].rcol) || !chain_fits_wg(S[i].c, S[i].A, S[i].jnd, rw0, maxg)) continue;
         StepsPlan::ChainGroup cg{};
         cg.kind = spmv_kind(S[i].A);
         cg.mixed = S[i].c->V32 != nullptr;
         cg.doff = P.chains.size();
         for (size_t k = i; k < S.size(); ++k) {
             if (taken[k] || S[k].ci != 0 || spmv_kind(S[k].A) != cg.kind || (S[k].c->V32 != nullptr) != cg.mixed ||
-                !chain_fits_wg(S[k].c, S[k].A, S[k].jnd, rw0, maxg))
+                !chain_form(S[k].qa, S[k].jnd, S[k].rcol) || !chain_fits_wg(S[k].c, S[k].A, S[k].jnd, rw0, maxg))
                 continue;
             // its followers are recorded right after it
             StepsPlan::Chain ch{S[k], 1};
@@ -5010,7 +5016,7 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
     int K = first ? 1 : std::max(1, std::min(c->ch_budget, kChainMax));
     c->ch_budget = 0;
     while (K > 1 && (!valid_col(c, rcol + K - 1) || jnd + K - 1 > c->ncols)) --K;
-    if (chain_fits(c, A, jnd)) {
+    if (chain_form(qa, jnd, rcol) && chain_fits(c, A, jnd)) {
         while (K > 1 && jnd + K - 1 > kChainMaxCols) --K;
         const int ran = run_chain(c, A, first, qa, qb, beta_prev, beta, jnd, rcol, K);
         if (ran < 0) return ran;

@@ -130,3 +130,47 @@ def test_chain_concurrent_solves(gpu_lib):
         A.close()
     for a, b in zip(alone, got):
         same(a, b)
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("kind,size", [("2d", 32), ("2d", 45), ("3d", 11), ("diag", 700), ("random", 3001)])
+def test_step_any_column(gpu_lib, kind, size, mixed):
+    """trlhip_step_cgs with q_a any column and r any column past the basis,
+    against NumPy in FP64.  Columns are FP32 values, so a mixed context's
+    shadow holds them exactly.  Bound: every result is a sum of at most n +
+    jnd products of O(1) magnitude after its factors' own sums, 8 (n + jnd)
+    eps of the magnitudes' sum."""
+    T = gpu_lib
+    csr = {"2d": lambda: W.anderson2d_csr(size, 6.0, seed=size)[0], "3d": lambda: W.laplace3d_csr(size, seed=size),
+           "diag": lambda: W.diag_csr(size), "random": lambda: W.random_sym_csr(size, seed=size)}[kind]()
+    n = len(csr[0]) - 1
+    mv = W.csr_matvec(*csr)
+    A = T.Csr(*csr, mixed=mixed)
+    ncols = 40
+    c = T.Ctx(n, ncols, mixed=mixed)
+    rng = np.random.default_rng(size)
+    V = (rng.standard_normal((ncols, n)) / np.sqrt(n)).astype(np.float32).astype(np.float64)
+    for j in range(ncols):
+        c.set(j, V[j])
+    for jnd in (1, 2, 5, 8, 9, 16, 31, 32, 33):
+        for qa, qb, rcol in ((0, -1, jnd), (jnd // 2, jnd // 2 - 1, jnd), (jnd - 1, jnd - 2, jnd + 2),
+                             (jnd + 1, -1, jnd), (jnd - 1, jnd - 2, jnd)):
+            print(f"{kind} n={n} mixed={mixed} jnd={jnd} qa={qa} qb={qb} rcol={rcol}", flush=True)
+            out = c.step_cgs(A, 0, qa, qb, 0.25, None, jnd, rcol)
+            y = np.asarray(mv(V[qa])).ravel()
+            alpha = V[qa] @ y
+            r = y - alpha * V[qa] - (0.25 * V[qb] if qb >= 0 else 0.0)
+            h = V[:jnd] @ r
+            s = r - h @ V[:jnd]
+            tol = 8 * (n + jnd) * np.finfo(float).eps
+            scale = np.abs(y).max() * 2 + np.linalg.norm(y) * (1 + np.abs(h).max())
+            got_r = c.get(rcol)
+            c.scale_copy(rcol, ncols, 1.0)
+            got_s = c.get(rcol)
+            c.set(rcol, V[rcol])
+            assert np.abs(got_r - r).max() <= tol * scale
+            assert np.abs(got_s - s).max() <= tol * scale * jnd
+            want = np.array([alpha, r @ r, h @ h, s @ s])
+            assert (np.abs(out - want) <= tol * jnd * (1 + scale) ** 2).all(), (out, want)
+    c.close()
+    A.close()
