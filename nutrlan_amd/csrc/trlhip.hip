@@ -1321,10 +1321,9 @@ __global__ __launch_bounds__(kBlock) void k_update(
 // 104 ms a solve.  Above kWideRows the 256-thread blocks fill the device.
 constexpr int kWide = 4 * kBlock;
 
-// Column group k's running sums of update_rows4 over columns [0, m) for four
-// rows (Vc: the first row in column 0).
-// Its loads are ordinary ones: at these sizes the projection has left the
-// columns in the caches.
+// Four rows of a column (ld4; ld4u from any row) and one (ld1) for
+// trl_sums.h.  The loads are ordinary ones: at these sizes the projection has
+// left the columns in the caches.
 __device__ __forceinline__ void ld4(const float *p, double v[4])
 {
     const f32x4 t = *reinterpret_cast<const f32x4 *>(p);
@@ -1334,41 +1333,31 @@ __device__ __forceinline__ void ld4(const float *p, double v[4])
     v[3] = t.w;
 }
 __device__ __forceinline__ void ld4(const double *p, double v[4]) { load4(p, v); }
-// With ZERO the sums start at 0; else they go on from column c, the first one
-// not in s yet (a multiple of 16; past the full groups only the tail is left).
-template <typename VS, bool ZERO = true>
-__device__ __forceinline__ void group_sums(const VS *Vc, long ld, int m, const double *hs, int k, double s[4],
-                                           int c = 0)
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ void ld4u(const float *p, double v[4])
 {
-    if (ZERO) s[0] = s[1] = s[2] = s[3] = 0.0;
-    const int full = m & ~7;
-    for (; c + 16 <= full; c += 16) {
-        double v[4][4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ld4(Vc + (size_t)(c + 4 * i + k) * ld, v[i]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) s[j] += v[i][j] * hs[c + 4 * i + k];
-    }
-    for (; c < full; c += 8) {
-        double v[2][4];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) ld4(Vc + (size_t)(c + 4 * i + k) * ld, v[i]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) s[j] += v[i][j] * hs[c + 4 * i + k];
-    }
-    if (k == 0) {
-        for (c = ZERO ? c : full; c < m; ++c) {
-            double v[4];
-            ld4(Vc + (size_t)c * ld, v);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) s[j] += v[j] * hs[c];
-        }
-    }
+    const f32x4u t = *reinterpret_cast<const f32x4u *>(p);
+    v[0] = t.x;
+    v[1] = t.y;
+    v[2] = t.z;
+    v[3] = t.w;
 }
+__device__ __forceinline__ void ld4u(const double *p, double v[4])
+{
+    const f64x2u a = reinterpret_cast<const f64x2u *>(p)[0], b = reinterpret_cast<const f64x2u *>(p)[1];
+    v[0] = a.x;
+    v[1] = a.y;
+    v[2] = b.x;
+    v[3] = b.y;
+}
+template <typename VS>
+__device__ __forceinline__ double ld1(const VS *p)
+{
+    return (double)*p;
+}
+
+#include "trl_sums.h"
 
 template <typename VS, int E>
 __device__ __forceinline__ void update_wide_body(int n, const VS *__restrict__ V, long ld, int m,
@@ -1387,7 +1376,7 @@ __device__ __forceinline__ void update_wide_body(int n, const VS *__restrict__ V
         const int row = R0 + 4 * tg;
         double s[4];
         if (row < n) {
-            group_sums(V + row, ld, m, hs, k, s);
+            quad_sums(n, row, V, ld, m, hs, k, s);
             if (k > 0)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) sm[k - 1][4 * tg + j] = s[j];

@@ -127,3 +127,43 @@ def test_noalloc_rejects_sizes(gpu_lib):
     assert f(8, 2, T.TRLHIP_R64, d.p, 4, d.p, None, None, None, None) == -1
     assert f(8, 2, T.TRLHIP_R64, d.p, 10, d.p, None, None, None, None) == -1
     d.free()
+
+
+@pytest.mark.parametrize("kind", ["r64", "c128", "r32"])
+@pytest.mark.parametrize("n,m", [(1, 1), (2, 9), (3, 8), (1021, 24), (1022, 7), (1023, 17), (1024, 3), (9002, 33)])
+def test_noalloc_tight_basis(gpu_lib, kind, n, m):
+    """The basis is the front of a larger buffer: its last column ends at row
+    n, and what lies behind a column's rows is NaN."""
+    T = gpu_lib
+    hip = _hip()
+    f = _noalloc_fn(T.lib())
+    rng = np.random.default_rng(n)
+    complex_ = kind == "c128"
+    dt = {"r64": np.float64, "c128": np.complex128, "r32": np.float32}[kind]
+    ld = n + 3 if complex_ else (n + 3) // 4 * 4
+    V = rng.standard_normal((m, n)) + (1j * rng.standard_normal((m, n)) if complex_ else 0)
+    r = rng.standard_normal(n) + (1j * rng.standard_normal(n) if complex_ else 0)
+    print(f"tight n={n} m={m} kind={kind} ld={ld}", flush=True)
+    c = T.Ctx(n, m + 1, complex_, mixed=kind == "r32")
+    for j in range(m):
+        c.set(j, V[j])
+    c.set(m, r)
+    hh_ref, rr2_ref, h_ref = c.cgs_pass(0, m, m)
+    r_ref = c.get(m)
+    c.close()
+    Vh = np.full((m + 1, ld), np.nan, dtype=dt)
+    Vh[:m, :n] = V.astype(dt)
+    dV, dr = DevBuf(hip, Vh.nbytes), DevBuf(hip, r.nbytes)
+    dV.put(Vh)
+    dr.put(r)
+    hh, rr2 = ctypes.c_double(), ctypes.c_double()
+    h = np.zeros(m, dtype=np.complex128 if complex_ else np.float64)
+    vt = {"r64": T.TRLHIP_R64, "c128": T.TRLHIP_C128, "r32": T.TRLHIP_R32}[kind]
+    rc = f(n, m, vt, dV.p, ld, dr.p, ctypes.byref(hh), ctypes.byref(rr2), h.ctypes.data, None)
+    got = dr.get(np.zeros_like(r))
+    dV.free()
+    dr.free()
+    assert rc == 0
+    assert np.array_equal(got, r_ref)
+    assert np.array_equal(h, h_ref)
+    assert hh.value == hh_ref and rr2.value == rr2_ref
