@@ -2451,9 +2451,12 @@ void launch_update(trlhip_ctx *c, int g, const VS *V, int c0, int m, const doubl
             pdst, o_hh, c->dscal + S_ALPHA);
 }
 
-// Whether a Gram-Schmidt update runs as k_update_wide: up to a block per CU.
-constexpr int kWideRows = 262144;
-bool update_wide_ok(int n) { return n <= kWideRows; }
+// Whether a Gram-Schmidt update of ncoef coefficients (two per complex
+// column) runs as k_update_wide: up to a block per CU, and coefficients that
+// leave its block within 64 KiB of LDS beside its 24 KiB of sums (k_update,
+// which holds nothing else there, takes longer bases).
+constexpr int kWideRows = 262144, kWideCoefs = 4096;
+bool update_wide_ok(int n, int ncoef) { return n <= kWideRows && ncoef <= kWideCoefs; }
 
 template <typename VS, int E>
 void launch_update_wide(int n, const VS *V, long ld, int m, const double *dh, const double *rin, double *rout,
@@ -2481,7 +2484,7 @@ int run_update(trlhip_ctx *c, int c0, int m, const double *dh, int aslot, int ri
     const bool s32 = shadow && c->V32;
     {
         Timed t(kind, c->s, s32 ? (4.0 * m + 16.0) * c->n : (double)c->esz * c->n * (m + 2));
-        if (shadow && aslot < 0 && update_wide_ok(c->n)) {
+        if (shadow && aslot < 0 && update_wide_ok(c->n, c->E * m)) {
             const double *r0 = colp<double>(c, rin);
             if (s32)
                 launch_update_wide<float, 1>(c->n, c->V32 + (size_t)c0 * c->ld, c->ld, m, dh, r0, colp<double>(c, rout),
@@ -3334,7 +3337,7 @@ void steps_plan(const std::vector<BatchStep> &steps, size_t ncbuf, StepsPlan &P,
             gi.fused = recproj_ok(steps[i].c);
             gi.E = steps[i].c->E;
             gi.single = single;
-            gi.wide = update_wide_ok(steps[i].c->n);
+            gi.wide = update_wide_ok(steps[i].c->n, gi.E * steps[i].jnd);
             gi.cb = gi.E == 2 ? 4 : g_proj_cb[gi.mixed ? 1 : 0].load(std::memory_order_relaxed);
             gi.doff = order.size();
             gi.poff = npre;
@@ -5678,7 +5681,7 @@ int noalloc_launch(int n, int m, const VS *V, long ld, double *r, double *scr, h
     if (hipGetLastError() != hipSuccess) return TRLHIP_EHIP;
     KLAUNCH(k_colsum, dim3(m * E), dim3(kBlock), 0, s, pproj, gx, dh);
     const int g = grid_for(n, kMinRowsUpd, kMaxGrid);
-    if (update_wide_ok(n)) {
+    if (update_wide_ok(n, E * m)) {
         launch_update_wide<VS, E>(n, V, ld, m, dh, r, r, pupd, dscal + S_HH, s);
     } else {
         const size_t shm = sizeof(double) * (size_t)E * m;

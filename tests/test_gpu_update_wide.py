@@ -39,3 +39,32 @@ def test_wide_update_matches(gpu_lib, n, complex_):
             assert rr2 == ref2
             assert np.array_equal(a, b)
         c.close()
+
+
+@pytest.mark.parametrize("complex_,m", [(False, 4096), (False, 4097), (False, 6000), (False, 17500), (True, 2048),
+                                        (True, 2049), (True, 8700)])
+def test_update_long_basis(gpu_lib, complex_, m):
+    """Coefficients up to and past what the wide update's LDS takes, up to
+    those that fit the 256-thread update alone.  Bounds as above."""
+    T = gpu_lib
+    n = 130
+    rng = np.random.default_rng(m)
+    print(f"n={n} m={m} complex={complex_}", flush=True)
+    V = rng.standard_normal((3, n)) + (1j * rng.standard_normal((3, n)) if complex_ else 0)
+    r = rng.standard_normal(n) + (1j * rng.standard_normal(n) if complex_ else 0)
+    c = T.Ctx(n, m + 1, complex_=complex_)
+    cols = (0, m // 2, m - 1)  # the others stay zero
+    for j, v in zip(cols, V):
+        c.set(j, v / np.sqrt(n))
+    c.set(m, r)
+    hh, rr2, h = c.cgs_pass(0, m, m)
+    got = c.get(m)
+    c.close()
+    Vn = V / np.sqrt(n)
+    href = Vn.conj() @ r
+    want = r - href @ Vn
+    tol = 8 * (n + 8) * np.finfo(float).eps * np.abs(r).max() * 4
+    assert np.count_nonzero(h) == 3
+    assert np.abs(h[list(cols)] - href).max() <= tol * np.sqrt(n)
+    assert np.abs(got - want).max() <= tol * np.sqrt(n)
+    assert abs(hh - np.vdot(href, href).real) <= tol * np.sqrt(n) * 8 and abs(rr2 - np.vdot(want, want).real) <= tol * n * 4
