@@ -41,6 +41,8 @@
 
 namespace {
 
+#include "trl_strips.h"
+
 constexpr int C = 32;          // hidden channels
 constexpr int T = 9;           // 3x3 taps
 constexpr int NB = 256;        // threads per block
@@ -75,12 +77,6 @@ __host__ __device__ inline float bf2f(bf16_t h)
 }
 
 __device__ inline __bf16 as_bf(bf16_t h) { return __builtin_bit_cast(__bf16, h); }
-
-struct Geo {
-    int nimg, h, w;
-    long np;  // pixels
-    int rows;  // rows a wave of a convolution walks (conv_rows)
-};
 
 __device__ inline bf16x8 load8(const bf16_t *p)
 {
@@ -117,7 +113,10 @@ inline int conv_rows(int ngroups, const int *nimg, const int *h, const int *w)
     }
     return rows;
 }
-inline Geo geo_of(int nimg, int h, int w, int rows) { return Geo{nimg, h, w, (long)nimg * h * w, rows}; }
+inline Geo geo_of(int nimg, int h, int w, int rows)
+{
+    return Geo{nimg, h, w, (long)nimg * h * w, rows, dw_rows(nimg, h, w)};
+}
 
 // A wave's strip: its image's first pixel, columns, rows [y0, y1).
 struct Strip {
@@ -518,44 +517,22 @@ __global__ __launch_bounds__(NB) void k_bwd32(Geo g, const bf16_t *__restrict__ 
 // loads, two pixels' channels interleaved by v_perm into dwords [channel]
 // [pixel pair], and read back 8 pixels a lane.  Rows of kTr = 18 dwords put
 // the writes of a wave on 64 different banks.  A wave walks down a strip of
-// 32 x kDwRows pixels and keeps its accumulators over all its strips.
+// up to 32 columns and keeps its accumulators over all its strips (dw_rows).
 // Gathering the operands two bytes at a time with a division per pixel and
 // tap, the two layers took 330 us each at 64 images of 64 x 64 (now 19), and
 // the first and last layers, one thread per weight over a serial pixel loop,
 // 650 us each (now 17).
-constexpr int kDwW = 32, kDwRows = 8;
 constexpr int kTr = 18;               // dwords per channel: 36 pixels
-constexpr int kDwBlocks = 256;        // blocks (4 waves each)
+static_assert(kDwWaves == kDwBlocks * (NB / 64), "waves of the gradient kernels");
 // Partials of the four layers: a row per block (layers 3 and 2), per wave
-// (4 and 1), and where each starts.  Blocks without a strip are not launched.
+// (4 and 1), and where each starts.  They are FP64: the sum over the waves'
+// FP32 accumulators is rounded once, at its end.  Blocks without a strip are
+// not launched.
 constexpr int kRowMid = C * T * C + C, kRowEdge = C * T + C;
 constexpr long kPart3 = 0, kPart2 = kPart3 + (long)kDwBlocks * kRowMid,
                kPart4 = kPart2 + (long)kDwBlocks * kRowMid,
                kPart1 = kPart4 + (long)kDwBlocks * (NB / 64) * kRowEdge,
                kPartCount = kPart1 + (long)kDwBlocks * (NB / 64) * kRowEdge;
-
-__host__ __device__ inline long dw_tasks(const Geo &g)
-{
-    return (long)g.nimg * ((g.w + kDwW - 1) / kDwW) * ((g.h + kDwRows - 1) / kDwRows);
-}
-
-struct DwStrip {
-    long base;
-    int x0, y0, y1;
-};
-
-__device__ __forceinline__ DwStrip dw_strip(const Geo &g, long task)
-{
-    const int ns = (g.w + kDwW - 1) / kDwW, per = ns * ((g.h + kDwRows - 1) / kDwRows);
-    const int img = (int)(task / per), r = (int)(task - (long)img * per);
-    const int seg = r / ns;
-    DwStrip s;
-    s.base = (long)img * g.h * g.w;
-    s.x0 = (r - seg * ns) * kDwW;
-    s.y0 = seg * kDwRows;
-    s.y1 = s.y0 + kDwRows < g.h ? s.y0 + kDwRows : g.h;
-    return s;
-}
 
 // Column x0 + p of a row of w, periodic one pixel beyond either end; further
 // out (a ragged strip's unused pixels) any column.
@@ -591,10 +568,10 @@ __device__ __forceinline__ bf16x8 frag(const uint32_t d[4])
 // serves the dY rows above, at and below it); a lane reads 12 pixels of a
 // channel and shifts them by one for the left and right taps.  The block's
 // partial (co, t, ci) and bias sums (a product with ones), its four waves
-// added in FP64, go to part[blockIdx]: a partial per wave was 38 MB to write
-// and read again, more than the activations of 64 images of 64 x 64 (34).
+// added in FP64, go to part[blockIdx] in FP64 (38 MB for 256 blocks, against
+// 19 in FP32: 128 images of 64 x 64 475 -> 483 us a forward and backward).
 __global__ __launch_bounds__(NB) void k_dw32(Geo g, const bf16_t *__restrict__ dy,
-                                             const bf16_t *__restrict__ x, float *__restrict__ part)
+                                             const bf16_t *__restrict__ x, double *__restrict__ part)
 {
     constexpr int NW = C * T * C;
     constexpr int kSr = C + 4;
@@ -623,7 +600,7 @@ __global__ __launch_bounds__(NB) void k_dw32(Geo g, const bf16_t *__restrict__ d
         const int c0 = dw_col(s.x0 + 2 * pp, g.w), c1 = dw_col(s.x0 + 2 * pp + 1, g.w);
         // the pixels just left and right of the strip, lanes 0..7
         const int ch = dw_col(pp == 0 ? s.x0 - 1 : s.x0 + kDwW, g.w);
-        const bool y0ok = s.x0 + 2 * pp < g.w, y1ok = s.x0 + 2 * pp + 1 < g.w;
+        const bool y0ok = s.x0 + 2 * pp < s.x1, y1ok = s.x0 + 2 * pp + 1 < s.x1;
         auto ldx = [&](int y, Pair &v, uint4 &h) {
             const bf16_t *p = x + (s.base + (long)wrap(y, g.h) * g.w) * C + 8 * cg;
             v.a = *reinterpret_cast<const uint4 *>(p + (long)c0 * C);
@@ -710,7 +687,7 @@ __global__ __launch_bounds__(NB) void k_dw32(Geo g, const bf16_t *__restrict__ d
 #pragma unroll
             for (int i = 0; i < 4; ++i) bs[wv][16 * mt + 4 * kq + i] = bacc[mt][i];
     __syncthreads();
-    float *out = part + (long)blockIdx.x * (NW + C);
+    double *out = part + (long)blockIdx.x * (NW + C);
     const int co = threadIdx.x / (C / 4), ci = 4 * (threadIdx.x % (C / 4));
 #pragma unroll
     for (int t = 0; t < T; ++t) {
@@ -730,16 +707,15 @@ __global__ __launch_bounds__(NB) void k_dw32(Geo g, const bf16_t *__restrict__ d
 #pragma unroll
             for (int i = 0; i < 4; ++i) s[i] += v[i];
         }
-        f4 o;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = (float)s[i];
-        *reinterpret_cast<f4 *>(out + (co * T + t) * C + ci) = o;
+        for (int i = 0; i < 4; i += 2)
+            *reinterpret_cast<double2 *>(out + (co * T + t) * C + ci + i) = make_double2(s[i], s[i + 1]);
     }
     if (threadIdx.x < C) {
         double s = 0.0;
 #pragma unroll
         for (int w = 0; w < NB / 64; ++w) s += bs[w][threadIdx.x];
-        out[NW + threadIdx.x] = (float)s;
+        out[NW + threadIdx.x] = s;
     }
 }
 
@@ -755,7 +731,7 @@ __global__ __launch_bounds__(NB) void k_dw32(Geo g, const bf16_t *__restrict__ d
 // parameters' order.
 template <bool LAST>
 __global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict__ v,
-                                                const float *__restrict__ u, float *__restrict__ part)
+                                                const float *__restrict__ u, double *__restrict__ part)
 {
     constexpr int NV = C * T + C;
     __shared__ __align__(16) uint32_t lds[NB / 64][C * kTr];
@@ -773,12 +749,12 @@ __global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict_
     for (long task = (long)blockIdx.x * (NB / 64) + wv; task < nt_; task += (long)gridDim.x * (NB / 64)) {
         const DwStrip s = dw_strip(g, task);
         const int c0 = dw_col(s.x0 + 2 * pp, g.w), c1 = dw_col(s.x0 + 2 * pp + 1, g.w);
-        const bool ok0 = s.x0 + 2 * pp < g.w, ok1 = s.x0 + 2 * pp + 1 < g.w;
+        const bool ok0 = s.x0 + 2 * pp < s.x1, ok1 = s.x0 + 2 * pp + 1 < s.x1;
         int uc[8];
         bool uok[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            uok[j] = s.x0 + 8 * kq + j < g.w;
+            uok[j] = s.x0 + 8 * kq + j < s.x1;
             uc[j] = dw_col(s.x0 + 8 * kq + j + odx, g.w);
         }
         auto ldv = [&](int y, Pair &p) {
@@ -818,7 +794,7 @@ __global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict_
             __builtin_amdgcn_wave_barrier();
         }
     }
-    float *out = part + ((long)blockIdx.x * (NB / 64) + wv) * NV;
+    double *out = part + ((long)blockIdx.x * (NB / 64) + wv) * NV;
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
@@ -860,7 +836,7 @@ constexpr RedArgs red_args()
     }
     return a;
 }
-__global__ __launch_bounds__(64 * kRedGroups) void k_reduce(const float *__restrict__ part, int dwb,
+__global__ __launch_bounds__(64 * kRedGroups) void k_reduce(const double *__restrict__ part, int dwb,
                                                             float *__restrict__ grad)
 {
     constexpr RedArgs a = red_args();
@@ -873,7 +849,7 @@ __global__ __launch_bounds__(64 * kRedGroups) void k_reduce(const float *__restr
     const int j = ((int)blockIdx.x - q.blk0) * 64 + c;
     double s = 0.0;
     if (j < q.len) {
-        const float *p = part + q.part + j;
+        const double *p = part + q.part + j;
 #pragma unroll 8
         for (int b = gr; b < q.rows * dwb; b += kRedGroups) s += p[(long)b * q.stride];
     }
@@ -927,7 +903,7 @@ struct trlnet {
     long cap = 0;  // pixels
     float *x = nullptr, *tg = nullptr, *o = nullptr, *dO = nullptr;
     bf16_t *a1 = nullptr, *a2 = nullptr, *a3 = nullptr, *d1 = nullptr, *d2 = nullptr;
-    float *part = nullptr;
+    double *part = nullptr;
     long partcap = 0;
     double *lpart = nullptr;
     int lcap = 0;
@@ -968,7 +944,7 @@ int ensure(trlnet *t, long np, int nimg)
     if (need > t->partcap) {
         if (t->part) (void)hipFree(t->part);
         t->partcap = 0;
-        NTRY(hipMalloc((void **)&t->part, sizeof(float) * need));
+        NTRY(hipMalloc((void **)&t->part, sizeof(double) * need));
         t->partcap = need;
     }
     if (nimg > t->lcap) {
