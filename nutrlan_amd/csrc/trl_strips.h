@@ -23,21 +23,25 @@ __host__ __device__ inline long dw_tasks(const Geo &g)
     return (long)g.nimg * dw_strips(g.w) * dw_segs(g.h, g.dwr);
 }
 
-// The strip height with which the busiest wave has the fewest rows, the
-// largest of these (a strip loads two rows of inputs more than it has): a
-// wave's FP32 sums then run over no more pixels than an even split gives it,
-// some 32 up to 1,024 strips of one row.  Forward and backward of 1, 8 and 32
-// images of 64 x 64 with 8-row strips throughout: 211, 200 and 256 us, so 174,
-// 171 and 240 (more waves).
+// Strip height.  A strip of r rows loads r + 2 rows of inputs, but a wave's
+// FP32 sums are to run over no more pixels than an even split gives them (32
+// up to 1,024 strips of one row), but for an eighth: of the heights that keep
+// to that, the one with the fewest rows to load for the busiest wave.  Forward
+// and backward of 1, 8 and 32 images of 64 x 64 with 8-row strips throughout:
+// 211, 200 and 256 us, so 174, 171 and 240 (more waves).
+__host__ __device__ inline long dw_wave_strips(int nimg, int h, int w, int r)
+{
+    return ((long)nimg * dw_strips(w) * dw_segs(h, r) + kDwWaves - 1) / kDwWaves;
+}
 inline int dw_rows(int nimg, int h, int w)
 {
-    int best = kDwRows;
-    long least = 0;
-    for (int r = kDwRows; r >= 1; --r) {
-        const long tasks = (long)nimg * dw_strips(w) * dw_segs(h, r);
-        const long rows = (tasks + kDwWaves - 1) / kDwWaves * (r < h ? r : h);
-        if (r == kDwRows || rows < least) {
-            least = rows;
+    const long even = dw_wave_strips(nimg, h, w, 1);
+    int best = 1;
+    long least = 3 * even;
+    for (int r = 2; r <= kDwRows && r <= h; ++r) {
+        const long n = dw_wave_strips(nimg, h, w, r);
+        if (n * r <= even + even / 8 && n * (r + 2) < least) {
+            least = n * (r + 2);
             best = r;
         }
     }

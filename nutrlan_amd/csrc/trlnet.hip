@@ -811,10 +811,11 @@ __global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict_
 }
 
 // grad = the sums over the partials' rows, in FP64, of all four layers in one
-// launch: a block takes 64 columns of a layer, its 16 groups of 64 threads
-// every 16th row, and the groups' sums are added in order.  (A launch per
-// layer: 24 us and the gaps between them, of 340 for 64 images of 64 x 64.)
-constexpr int kRedGroups = 16;
+// launch: a block takes 32 columns of a layer, its 32 groups of threads every
+// 32nd row, all their loads in flight, and the groups' sums are added in
+// order.  (A launch per layer: 24 us and the gaps between them, of 340 for 64
+// images of 64 x 64; 38 MB with 16 groups of 64 columns: 14.0 us, now 10.3.)
+constexpr int kRedGroups = 32, kRedCols = 32;
 struct RedSeg {
     long part;
     int rows, len, stride, out, blk0;  // rows a block of the gradient kernel leaves
@@ -832,21 +833,21 @@ constexpr RedArgs red_args()
     a.s[3] = {kPart1, NB / 64, kRowEdge, kRowEdge, OW1, 0};
     for (int i = 0; i < 4; ++i) {
         a.s[i].blk0 = a.blocks;
-        a.blocks += (a.s[i].len + 63) / 64;
+        a.blocks += (a.s[i].len + kRedCols - 1) / kRedCols;
     }
     return a;
 }
-__global__ __launch_bounds__(64 * kRedGroups) void k_reduce(const double *__restrict__ part, int dwb,
+__global__ __launch_bounds__(kRedCols * kRedGroups) void k_reduce(const double *__restrict__ part, int dwb,
                                                             float *__restrict__ grad)
 {
     constexpr RedArgs a = red_args();
-    __shared__ double sm[kRedGroups][64];
-    const int c = threadIdx.x & 63, gr = threadIdx.x >> 6;
+    __shared__ double sm[kRedGroups][kRedCols];
+    const int c = threadIdx.x % kRedCols, gr = threadIdx.x / kRedCols;
     RedSeg q = a.s[0];
 #pragma unroll
     for (int i = 1; i < 4; ++i)
         if ((int)blockIdx.x >= a.s[i].blk0) q = a.s[i];
-    const int j = ((int)blockIdx.x - q.blk0) * 64 + c;
+    const int j = ((int)blockIdx.x - q.blk0) * kRedCols + c;
     double s = 0.0;
     if (j < q.len) {
         const double *p = part + q.part + j;
@@ -1045,7 +1046,7 @@ int backward(trlnet *t, const Geo &g, double *loss)
     hipLaunchKernelGGL(k_bwd32, dim3(gb), blk, 0, t->s, g, t->d1, t->wt2, t->a1, t->d2);
     // layer 1: dY = d2 (for a1), X = potential
     hipLaunchKernelGGL((k_dw_edge<false>), dwb, blk, 0, t->s, g, t->d2, t->x, t->part + kPart1);
-    hipLaunchKernelGGL(k_reduce, dim3(red_args().blocks), dim3(64 * kRedGroups), 0, t->s, t->part, ndw,
+    hipLaunchKernelGGL(k_reduce, dim3(red_args().blocks), dim3(kRedCols * kRedGroups), 0, t->s, t->part, ndw,
                        t->grad);
     if (hipGetLastError() != hipSuccess) return TRLNET_EHIP;
     std::vector<double> lp((size_t)g.nimg);

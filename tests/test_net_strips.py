@@ -1,7 +1,7 @@
 """The start net's division of images among waves (csrc/trl_strips.h),
 compiled for the CPU: every pixel belongs to exactly one strip, and no wave
 sums more of a weight gradient in FP32 than an even split of the pixels in
-runs of 32 over 1,024 waves gives it, within a strip's row."""
+runs of 32 over 1,024 waves gives it, within an eighth and a strip's row."""
 import os
 import subprocess
 
@@ -11,7 +11,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "nutrlan_amd", "csrc")
 SHAPES = [(1, 3, 3), (1, 64, 64), (8, 64, 64), (9, 65, 63), (16, 64, 33), (40, 64, 33), (64, 64, 64), (70, 64, 64),
           (64, 3, 3), (3000, 3, 3), (500, 5, 7), (64, 8, 8), (200, 31, 16), (90, 12, 40), (130, 17, 33), (4, 256, 256),
-          (1, 512, 512), (16, 100, 100), (6, 200, 200), (2, 1000, 3), (2, 3, 1000)]
+          (1, 512, 512), (16, 100, 100), (6, 200, 200), (2, 1000, 3), (2, 3, 1000),
+          (900, 15, 15), (1500, 11, 11), (10000, 5, 5), (500, 33, 33)]
 
 
 @pytest.fixture(scope="module")
@@ -30,4 +31,4 @@ def test_gradient_strips(exe):
         width = -(-w // -(-w // 32))
         even = 32 * -(-(-(-nimg * h * w // 32)) // 1024)
         assert bad == 0, (nimg, h, w)
-        assert most <= even + width, (nimg, h, w, most, even)
+        assert most <= even + even // 8 + width, (nimg, h, w, most, even)
