@@ -6,9 +6,66 @@
 struct Geo {
     int nimg, h, w;
     long np;   // pixels
-    int rows;  // rows a wave of a convolution walks (conv_rows)
+    // a convolution's wave: the rows it walks (conv_rows), the images side by
+    // side (strip_images); how many there are
+    int rows, ni;
+    long tasks;
     int dwr;   // rows of a weight-gradient strip (dw_rows)
 };
+
+// Convolutions: a wave takes strips of kStrip columns of an image, or, where
+// an image has at most half as many, of as many images side by side as fit,
+// and walks down up to kRows rows of them.  With one 3 x 3 image to a strip 13
+// of 16 lanes have no pixel: the forward pass of 20,000 such images, host to
+// host, took 218 us (174 with 16 consecutive pixels to a wave), now 140; 64
+// images of 400 x 3 107 (95), now 90.
+constexpr int kStrip = 16, kRows = 8;
+
+__host__ __device__ inline int strips_of(int w) { return (w + kStrip - 1) / kStrip; }
+__host__ __device__ inline int segs_of(int h, int rows) { return (h + rows - 1) / rows; }
+inline int strip_images(int h, int w)
+{
+    return 2 * w <= kStrip && h <= 65536 ? kStrip / w : 1;  // the images' offset is an int
+}
+inline long conv_tasks(int nimg, int h, int w, int rows)
+{
+    const int ni = strip_images(h, w);
+    return (long)((nimg + ni - 1) / ni) * strips_of(w) * segs_of(h, rows);
+}
+
+// A lane's part of a wave's strip: pixel (y, its column) is base + y w + x,
+// its neighbours' columns (periodic) are xc.  Its image's offset from the
+// wave's first is part of x and xc, so that base stays the wave's.
+struct Strip {
+    long base;
+    int x, xc[3], y0, y1;  // rows [y0, y1)
+    bool ok;               // it has a pixel (others repeat one)
+};
+
+__host__ __device__ inline bool strip_of(const Geo &g, long task, int lane, Strip &s)
+{
+    if (task >= g.tasks) return false;
+    const int ns = strips_of(g.w), per = ns * segs_of(g.h, g.rows), ni = g.ni;
+    const int grp = (int)(task / per), r = (int)(task - (long)grp * per);
+    const int seg = r / ns, strip = r - seg * ns;
+    int x = strip * kStrip + lane, off = 0;
+    s.ok = x < g.w;
+    if (ni > 1) {
+        const int i = lane / g.w, last = g.nimg - 1 - grp * ni;
+        x = lane - i * g.w;
+        s.ok = i < ni && i <= last;
+        off = (i < last ? i : last) * g.h * g.w;
+    }
+    x = x < g.w ? x : g.w - 1;
+    s.x = off + x;
+    s.xc[0] = off + (x == 0 ? g.w - 1 : x - 1);
+    s.xc[1] = s.x;
+    s.xc[2] = off + (x == g.w - 1 ? 0 : x + 1);
+    s.base = (long)grp * ni * g.h * g.w;
+    s.y0 = seg * g.rows;
+    s.y1 = s.y0 + g.rows < g.h ? s.y0 + g.rows : g.h;
+    return true;
+}
 
 // Weight gradients: strips of at most kDwW columns, equally wide, and dwr <=
 // kDwRows rows, dealt to the waves of at most kDwBlocks blocks in turn.
@@ -46,6 +103,11 @@ inline int dw_rows(int nimg, int h, int w)
         }
     }
     return best;
+}
+
+inline Geo geo_of(int nimg, int h, int w, int rows)
+{
+    return Geo{nimg, h, w, (long)nimg * h * w, rows, strip_images(h, w), conv_tasks(nimg, h, w, rows), dw_rows(nimg, h, w)};
 }
 
 struct DwStrip {

@@ -46,8 +46,6 @@ namespace {
 constexpr int C = 32;          // hidden channels
 constexpr int T = 9;           // 3x3 taps
 constexpr int NB = 256;        // threads per block
-constexpr int kStrip = 16;     // pixels of a row per wave
-constexpr int kRows = 8;       // rows a wave walks at most
 
 // parameter offsets in the flat FP32 vector
 constexpr int OW1 = 0, OB1 = OW1 + C * T;             // W1[co][t]
@@ -86,14 +84,7 @@ __device__ inline bf16x8 load8(const bf16_t *p)
 
 __device__ inline bf16x8 zero8() { return __builtin_bit_cast(bf16x8, uint4{0, 0, 0, 0}); }
 
-// Wave tasks of a convolution: strips x row segments of every image.
-__host__ __device__ inline int strips_of(int w) { return (w + kStrip - 1) / kStrip; }
-__host__ __device__ inline int segs_of(int h, int rows) { return (h + rows - 1) / rows; }
-__host__ __device__ inline long conv_tasks(const Geo &g)
-{
-    return (long)g.nimg * strips_of(g.w) * segs_of(g.h, g.rows);
-}
-inline long conv_blocks(const Geo &g) { return (conv_tasks(g) + NB / 64 - 1) / (NB / 64); }
+inline long conv_blocks(const Geo &g) { return (g.tasks + NB / 64 - 1) / (NB / 64); }
 
 // Rows a wave walks for the images of all groups of a launch: shorter walks
 // while there is at most a wave per SIMD.  Forward and backward of 8 images
@@ -107,40 +98,11 @@ inline int conv_rows(int ngroups, const int *nimg, const int *h, const int *w)
     int rows = kRows;
     while (rows > kMinRows) {
         long n = 0;
-        for (int i = 0; i < ngroups; ++i) n += (long)nimg[i] * strips_of(w[i]) * segs_of(h[i], rows / 2);
+        for (int i = 0; i < ngroups; ++i) n += conv_tasks(nimg[i], h[i], w[i], rows / 2);
         if (n > kConvWaves) break;
         rows /= 2;
     }
     return rows;
-}
-inline Geo geo_of(int nimg, int h, int w, int rows)
-{
-    return Geo{nimg, h, w, (long)nimg * h * w, rows, dw_rows(nimg, h, w)};
-}
-
-// A wave's strip: its image's first pixel, columns, rows [y0, y1).
-struct Strip {
-    long base;
-    int x, xc[3], y0, y1;  // the lane's column, its neighbours' (periodic), the rows
-    bool ok;               // the lane's column exists (others repeat the last one)
-};
-
-__device__ __forceinline__ bool strip_of(const Geo &g, long task, Strip &s)
-{
-    if (task >= conv_tasks(g)) return false;
-    const int ns = strips_of(g.w), per = ns * segs_of(g.h, g.rows);
-    const int img = (int)(task / per), r = (int)(task - (long)img * per);
-    const int seg = r / ns, strip = r - seg * ns;
-    const int x = strip * kStrip + (int)(threadIdx.x & 15);
-    s.ok = x < g.w;
-    s.x = s.ok ? x : g.w - 1;
-    s.xc[0] = s.x == 0 ? g.w - 1 : s.x - 1;
-    s.xc[1] = s.x;
-    s.xc[2] = s.x == g.w - 1 ? 0 : s.x + 1;
-    s.base = (long)img * g.h * g.w;
-    s.y0 = seg * g.rows;
-    s.y1 = s.y0 + g.rows < g.h ? s.y0 + g.rows : g.h;
-    return true;
 }
 
 __device__ __forceinline__ int wrap(int y, int h) { return y < 0 ? y + h : (y >= h ? y - h : y); }
@@ -162,7 +124,7 @@ __device__ __forceinline__ void fwd1_body(const Geo &g, long bid, const float *_
 {
     const int lane = threadIdx.x & 63;
     Strip s;
-    if (!strip_of(g, bid * (NB / 64) + (threadIdx.x >> 6), s)) return;
+    if (!strip_of(g, bid * (NB / 64) + (threadIdx.x >> 6), threadIdx.x & 15, s)) return;
     const int m = lane & 15, kq = lane >> 4;
     bf16x8 wt[2];
     float bs[2][4];
@@ -232,7 +194,7 @@ __device__ __forceinline__ void conv32_body(const Geo &g, long bid, const bf16_t
 {
     const int lane = threadIdx.x & 63;
     Strip s;
-    if (!strip_of(g, bid * (NB / 64) + (threadIdx.x >> 6), s)) return;
+    if (!strip_of(g, bid * (NB / 64) + (threadIdx.x >> 6), threadIdx.x & 15, s)) return;
     const int m = lane & 15, kq = lane >> 4;
     bf16x8 wt[T][2];
 #pragma unroll
@@ -311,7 +273,7 @@ __device__ __forceinline__ void fwd4_body(const Geo &g, long bid, const bf16_t *
 {
     const int lane = threadIdx.x & 63;
     Strip s;
-    if (!strip_of(g, bid * (NB / 64) + (threadIdx.x >> 6), s)) return;
+    if (!strip_of(g, bid * (NB / 64) + (threadIdx.x >> 6), threadIdx.x & 15, s)) return;
     const int m = lane & 15, kq = lane >> 4;
     bf16x8 wt[T];
 #pragma unroll
@@ -451,7 +413,7 @@ __global__ __launch_bounds__(NB) void k_bwd4(Geo g, const float *__restrict__ do
 {
     const int lane = threadIdx.x & 63;
     Strip s;
-    if (!strip_of(g, (long)blockIdx.x * (NB / 64) + (threadIdx.x >> 6), s)) return;
+    if (!strip_of(g, (long)blockIdx.x * (NB / 64) + (threadIdx.x >> 6), threadIdx.x & 15, s)) return;
     const int m = lane & 15, kq = lane >> 4;
     bf16x8 wt[2];
 #pragma unroll
@@ -814,7 +776,7 @@ __global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict_
 // launch: a block takes 32 columns of a layer, its 32 groups of threads every
 // 32nd row, all their loads in flight, and the groups' sums are added in
 // order.  (A launch per layer: 24 us and the gaps between them, of 340 for 64
-// images of 64 x 64; 38 MB with 16 groups of 64 columns: 14.0 us, now 10.3.)
+// images of 64 x 64; 38 MB with 16 groups of 64 columns: 14 us, now 10.3.)
 constexpr int kRedGroups = 32, kRedCols = 32;
 struct RedSeg {
     long part;

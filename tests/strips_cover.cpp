@@ -1,6 +1,8 @@
 // The start net's strips (csrc/trl_strips.h) on the CPU: for each "nimg h w"
 // on the command line prints the weight-gradient strips' pixels that are not
-// covered exactly once, and the most pixels and the rows any wave has.
+// covered exactly once, the most pixels and rows any wave has, the pixels that
+// the convolutions' strips of 8, 4 and 2 rows do not cover exactly once, their
+// neighbours that are not the image's, and the convolutions' waves of 8 rows.
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -14,9 +16,7 @@
 int main(int argc, char **argv)
 {
     for (int a = 1; a + 2 < argc; a += 3) {
-        Geo g{std::atoi(argv[a]), std::atoi(argv[a + 1]), std::atoi(argv[a + 2]), 0, 0, 0};
-        g.np = (long)g.nimg * g.h * g.w;
-        g.dwr = dw_rows(g.nimg, g.h, g.w);
+        Geo g = geo_of(std::atoi(argv[a]), std::atoi(argv[a + 1]), std::atoi(argv[a + 2]), kRows);
         std::vector<int> seen(g.np, 0);
         const long nt = dw_tasks(g);
         const long nw = std::min<long>(kDwBlocks, (nt + 3) / 4) * 4;
@@ -35,7 +35,25 @@ int main(int argc, char **argv)
         }
         long bad = 0;
         for (int c : seen) bad += c != 1;
-        std::printf("%ld %ld %ld\n", bad, most, rows);
+        long cbad = 0, nbad = 0, waves = 0;
+        for (int r = kRows; r >= 2; r /= 2) {
+            g = geo_of(g.nimg, g.h, g.w, r);
+            if (r == kRows) waves = g.tasks;
+            std::fill(seen.begin(), seen.end(), 0);
+            Strip s;
+            for (long t = 0; t < g.tasks; ++t)
+                for (int lane = 0; lane < kStrip; ++lane) {
+                    if (!strip_of(g, t, lane, s)) std::abort();
+                    const long hw = (long)g.h * g.w, img = (s.base + s.x) / hw, x = (s.base + s.x) % hw;
+                    nbad += s.base % hw != 0 || s.base < 0 || img >= g.nimg || x >= g.w || s.y1 > g.h;
+                    for (int d = 0; d < 3; ++d) nbad += s.base + s.xc[d] != img * hw + (x + d - 1 + g.w) % g.w;
+                    if (s.ok)
+                        for (int y = s.y0; y < s.y1; ++y) ++seen[s.base + (long)y * g.w + s.x];
+                }
+            if (strip_of(g, g.tasks, 0, s)) std::abort();
+            for (int c : seen) cbad += c != 1;
+        }
+        std::printf("%ld %ld %ld %ld %ld %ld\n", bad, most, rows, cbad, nbad, waves);
     }
     return 0;
 }

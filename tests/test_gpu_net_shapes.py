@@ -77,3 +77,17 @@ def test_more_waves(gpu_lib, shape):
     """Batches of more waves than SIMDs, which walk 8 or 4 rows each (those
     above walk 2 or 4); ragged in both directions."""
     test_forward_and_gradients(gpu_lib, shape)
+
+
+@pytest.mark.parametrize("shape", [(1, 4, 3), (5, 9, 3), (6, 17, 3), (16, 5, 4), (7, 6, 5), (9, 3, 6), (4, 11, 7),
+                                   (3, 8, 8), (66, 3, 8), (2, 5, 9)])
+def test_narrow_images(gpu_lib, shape):
+    """Images that share a strip: each one's output is that of the image
+    alone."""
+    test_forward_and_gradients(gpu_lib, shape)
+    net = learned.Net(seed=21)
+    x = np.random.default_rng(23).uniform(-1, 1, shape).astype(np.float32)
+    y = net.forward(x)
+    for i in range(len(x)):
+        assert np.array_equal(net.forward(x[i:i + 1])[0], y[i]), i
+    net.close()

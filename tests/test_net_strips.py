@@ -23,12 +23,25 @@ def exe(tmp_path_factory):
     return out
 
 
-def test_gradient_strips(exe):
+@pytest.fixture(scope="module")
+def counts(exe):
     args = [str(v) for s in SHAPES for v in s]
-    lines = subprocess.run([exe, *args], capture_output=True, text=True, check=True).stdout.split("\n")
-    for (nimg, h, w), line in zip(SHAPES, lines):
-        bad, most, _ = (int(v) for v in line.split())
+    out = subprocess.run([exe, *args], capture_output=True, text=True, check=True).stdout.splitlines()
+    return [(s, [int(v) for v in line.split()]) for s, line in zip(SHAPES, out)]
+
+
+def test_gradient_strips(counts):
+    for (nimg, h, w), (bad, most, *_) in counts:
         width = -(-w // -(-w // 32))
         even = 32 * -(-(-(-nimg * h * w // 32)) // 1024)
         assert bad == 0, (nimg, h, w)
         assert most <= even + even // 8 + width, (nimg, h, w, most, even)
+
+
+def test_convolution_strips(counts):
+    """Every pixel once, at every height a walk may have; narrow images share
+    strips, so that 9 of 16 lanes or more have a pixel (but in the last)."""
+    for (nimg, h, w), (_, _, _, bad, neighbours, waves) in counts:
+        assert bad == 0 and neighbours == 0, (nimg, h, w)
+        if w <= 8:
+            assert 9 * waves <= -(-h // 8) * (nimg * w + 16), (nimg, h, w, waves)
