@@ -1899,6 +1899,7 @@ struct trlhip_ctx {
     unsigned *sync;
     unsigned sync_base;
     int gate_parity, chain_off;
+    int cus;                          // CUs of its device
     int ch_copy_ok;                   // that follower's fused normalisation was claimed
     int ch_qa[kChainMax], ch_qb[kChainMax], ch_rcol[kChainMax], ch_jnd[kChainMax];
 };
@@ -1974,6 +1975,7 @@ struct trlhip_batch {
     void (*yield)(void *) = nullptr;
     void *user = nullptr;
     int err = 0;                  // sticky device error of a flush
+    int cus = 1;                  // CUs of its device
     SpinLock mu;                  // guards the records (coroutines run on several host threads)
     std::mutex arena_mu;          // guards the arenas (contexts are created on several threads)
     std::vector<BatchStep> steps;
@@ -2213,7 +2215,7 @@ bool recproj_ok(const trlhip_ctx *c)
 // sites: 6.5 with 4, 6.4 with 2).  The CSR kinds keep 2: with 4, their
 // prefetched nonzeros no longer fit the 128 registers a thread of 16 waves
 // has (n = 50,001, 17 nonzeros a row: the product takes 30 us against 16).
-int chain_rw(const trlhip_csr *A) { return spmv_kind(A) <= -2 && A->n > 32768 ? 4 : 2; }
+int chain_rw(int kind, int n) { return kind <= -2 && n > 32768 ? 4 : 2; }
 
 // Whether a step of a single solve runs as a chain kernel: real solves with
 // a stencil or CSR-stream operator whose workgroups fit kChainMaxWG (n <=
@@ -2224,17 +2226,23 @@ int chain_rw(const trlhip_csr *A) { return spmv_kind(A) <= -2 && A->n > 32768 ? 
 // random rows n = 50,001 69 -> 48 ms (with the faster restarts and columns
 // kept in registers since: 4.6, 5.4 and, for the random rows, 44 ms).
 constexpr int kChainCsrIter = 4;
+int chain_wgs(int n, int rw) { return (n + 256 * rw - 1) / (256 * rw); }
+bool chain_shape(int n, int kind, int nb, int max_blk_nnz, int jnd, int rw, int maxg)
+{
+    const int g = chain_wgs(n, rw);
+    if (g > maxg || nb > kSpmvGrid || jnd > kChainMaxCols) return false;
+    return kind <= -2 || (max_blk_nnz <= kNnzBlk && (nb + g * rw - 1) / (g * rw) <= kChainCsrIter);
+}
 bool chain_fits_wg(const trlhip_ctx *c, const trlhip_csr *A, int jnd, int rw, int maxg)
 {
-    if (!A || c->E != 1 || c->chain_off || A->lpr || A->pn_on || jnd > kChainMaxCols) return false;
-    const int g = (A->n + 256 * rw - 1) / (256 * rw);
-    if (g > maxg || A->nb > kSpmvGrid) return false;
-    if (spmv_kind(A) <= -2) return true;
-    return A->max_blk_nnz <= kNnzBlk && (A->nb + g * rw - 1) / (g * rw) <= kChainCsrIter;
+    if (!A || c->E != 1 || c->chain_off || A->lpr || A->pn_on) return false;
+    return chain_shape(A->n, spmv_kind(A), A->nb, A->max_blk_nnz, jnd, rw, maxg);
 }
+// At most a workgroup per CU: they all wait for each other.
+int chain_max_wgs(int cus) { return std::min(kChainMaxWG, cus); }
 bool chain_fits(const trlhip_ctx *c, const trlhip_csr *A, int jnd)
 {
-    return !c->batch && A && chain_fits_wg(c, A, jnd, chain_rw(A), kChainMaxWG);
+    return !c->batch && A && chain_fits_wg(c, A, jnd, chain_rw(spmv_kind(A), A->n), chain_max_wgs(c->cus));
 }
 // The form of a step that chain kernels take, the solver's: q_a is the last
 // basis column and r goes to the column after it.  They keep q_a in LDS and,
@@ -2243,7 +2251,7 @@ bool chain_fits(const trlhip_ctx *c, const trlhip_csr *A, int jnd)
 bool chain_form(int qa, int jnd, int rcol) { return qa == jnd - 1 && rcol == jnd; }
 
 // A batch's launch runs its steps as chains (kb_chain) while the solves that
-// fit hold at most kBatchChainRows rows together.  The device holds 262,144
+// fit hold at most kBatchChainRows rows together (on 256 CUs).  The device holds 262,144
 // rows of a chain kernel at once (1024 a workgroup, one workgroup per CU) and
 // steps them in about 14 us; the phase kernels take 25 us and 40 more per
 // million rows.  Batches with the limit at 0, 300,000, 600,000 and 1,500,000:
@@ -2253,17 +2261,25 @@ bool chain_form(int qa, int jnd, int rcol) { return qa == jnd - 1 && rcol == jnd
 constexpr long kBatchChainRows = 600000;
 constexpr int kBatchChainWG = 64;  // workgroups of one solve at most, and a quarter of the CUs
 
-// CUs of the current device (queried once: the answer does not change).
+// A chain of a batch has at most maxg workgroups, of two row waves while all
+// rows of the launch run at once (512 a CU), else four.
+int batch_chain_wgs(int cus) { return std::min(kBatchChainWG, cus / 4); }
+int batch_chain_rw(long rows, int maxn, int cus)
+{
+    return rows <= 512L * cus && maxn <= 512 * batch_chain_wgs(cus) ? 2 : 4;
+}
+
+// CUs of the current device, queried once for each device.
+constexpr int kMaxDevices = 64;
 int device_cus()
 {
-    static std::atomic<int> cus{0};
-    int n = cus.load(std::memory_order_relaxed);
+    static std::atomic<int> cus[kMaxDevices];
+    int dev = -1, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 1;
+    if (dev < kMaxDevices) n = cus[dev].load(std::memory_order_relaxed);
     if (!n) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1)
-            n = 1;
-        cus.store(n, std::memory_order_relaxed);
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 1;
+        if (dev < kMaxDevices) cus[dev].store(n, std::memory_order_relaxed);
     }
     return n;
 }
@@ -3269,6 +3285,7 @@ struct StepsPlan {
     std::vector<Chain> chains;
     std::vector<ChainGroup> cgroups;
     int rw = 4;  // row waves a workgroup (stencils)
+    int cus = 1;
     size_t off_ch = 0, off_chpre = 0, off_flags = 0;
 };
 
@@ -3278,17 +3295,16 @@ void chains_plan(const std::vector<BatchStep> &S, StepsPlan &P, std::vector<char
 {
     long rows = 0;
     int maxn = 0;
+    P.cus = S[0].c->cus;
+    const int maxg = batch_chain_wgs(P.cus);
     for (const BatchStep &st : S)
         if (st.ci == 0 && chain_form(st.qa, st.jnd, st.rcol) &&
-            chain_fits_wg(st.c, st.A, st.jnd, 4, kBatchChainWG)) {
+            chain_fits_wg(st.c, st.A, st.jnd, 4, maxg)) {
             rows += st.c->n;
             maxn = std::max(maxn, st.c->n);
         }
-    if (!rows || rows > kBatchChainRows) return;
-    // short phases while every workgroup runs at once, else the most rows
-    // the device holds
-    const int maxg = std::min(kBatchChainWG, device_cus() / 4);
-    P.rw = rows <= 512 * 256 && maxn <= 512 * maxg ? 2 : 4;
+    if (!rows || rows > kBatchChainRows * P.cus / 256) return;
+    P.rw = batch_chain_rw(rows, maxn, P.cus);
     for (size_t i = 0; i < S.size(); ++i) {
         if (taken[i] || S[i].ci != 0) continue;
         const int rw0 = spmv_kind(S[i].A) <= -2 ? P.rw : 2;
@@ -3440,7 +3456,7 @@ int steps_launch(hipStream_t s, const StepsPlan &P, const char *h, const char *d
         const ChainArgs *q = dch + cg.doff;
         const int *pp = dcp + cg.poff;
         unsigned *ticket = df + cg.foff;
-        const dim3 grid(std::min(cg.wgs, device_cus()));
+        const dim3 grid(std::min(cg.wgs, P.cus));
 #define KB_CHAIN(RW, KIND)                                                                      \
     do {                                                                                        \
         if (cg.mixed)                                                                           \
@@ -4490,6 +4506,7 @@ int trlhip_ctx_create_batched(trlhip_ctx **out, int n, int ncols, int vtype, trl
         // batched: everything from the batch's arenas, nothing to synchronize
         std::lock_guard<std::mutex> lk(b->arena_mu);
         c->batch = b;
+        c->cus = b->cus;
         c->s = b->side;
         c->arena = 1;
         const size_t np = part_need(c->E, ncols);
@@ -4517,6 +4534,7 @@ int trlhip_ctx_create_batched(trlhip_ctx **out, int n, int ncols, int vtype, trl
         *out = c;
         return 0;
     }
+    c->cus = device_cus();
     if (hipStreamCreate(&c->s) != hipSuccess) rc = TRLHIP_EHIP;
     if (!rc && hipMalloc((void **)&c->V, vbytes) != hipSuccess) rc = TRLHIP_ENOMEM;
     const size_t sbytes = sizeof(float) * (size_t)c->ld * (ncols + 1);
@@ -4849,7 +4867,7 @@ static int run_chain(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int 
                      const double *beta, int jnd, int rcol, int K)
 {
     ChainArgs q{};
-    const int rw = chain_rw(A);
+    const int rw = chain_rw(spmv_kind(A), A->n);
     chain_args(q, c, A, rw, first, qa, qb, beta_prev, jnd, rcol, K, c->ch_kept, c->ch_ntot);
     if (c->pend_dst == qa && rcol != c->pend_src) {
         q.x = colp<double>(c, c->pend_src);
@@ -5088,6 +5106,19 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
     out[2] = hr[S_HH];
     out[3] = hr[S_RR2B];
     return 0;
+}
+
+int trlhip_chain_rule(int n, int kind, int nb, int max_blk_nnz, int jnd, int cus, int *wgs)
+{
+    const int rw = chain_rw(kind, n);
+    if (wgs) *wgs = chain_wgs(n, rw);
+    return chain_shape(n, kind, nb, max_blk_nnz, jnd, rw, chain_max_wgs(cus)) ? rw : 0;
+}
+
+int trlhip_batch_chain_rule(long rows, int maxn, int cus, int *maxg)
+{
+    if (maxg) *maxg = batch_chain_wgs(cus);
+    return batch_chain_rw(rows, maxn, cus);
 }
 
 int trlhip_step_chain(trlhip_ctx *c, int steps, int kept, int ntot)
@@ -5435,6 +5466,7 @@ int trlhip_batch_create_on(trlhip_batch **out, trlhip_batch *share)
         delete b;
         return TRLHIP_EHIP;
     }
+    b->cus = device_cus();
     *out = b;
     return 0;
 }
@@ -5621,7 +5653,6 @@ int trlhip_batch_flush(trlhip_batch *b)
 
 namespace {
 constexpr int kNoAllocMaxCols = 256;  // TRLHIP_NOALLOC_MAX_COLS
-constexpr int kMaxDevices = 64;
 // partial rows: kProjGrid per coefficient, 2 coefficients per complex
 // column; then 8 scalars, h (2 per column), the update partials
 constexpr size_t kScrProj = 0;

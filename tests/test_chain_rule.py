@@ -1,0 +1,55 @@
+"""The rules that choose chain kernels and their workgroups, on the CPU."""
+import ctypes
+
+import pytest
+
+from nutrlan_amd import trlan as T
+
+
+def rule(n, kind, cus, nb=None, nnz=1000, jnd=20):
+    wgs = ctypes.c_int()
+    rw = T.lib().trlhip_chain_rule(n, kind, -(-n // 256) if nb is None else nb, nnz, jnd, cus, ctypes.byref(wgs))
+    return rw, wgs.value
+
+
+def batch_rule(rows, maxn, cus):
+    f = T.lib().trlhip_batch_chain_rule
+    f.argtypes = [ctypes.c_long, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+    maxg = ctypes.c_int()
+    return f(rows, maxn, cus, ctypes.byref(maxg)), maxg.value
+
+
+@pytest.mark.parametrize("kind", [-3, -2, -1, 0])
+@pytest.mark.parametrize("cus", [1, 2, 16, 32, 38, 64, 80, 128, 228, 256, 304])
+def test_workgroups_fit_the_device(kind, cus):
+    """All workgroups of a chain wait for each other, so there is at most one
+    per CU, and never more than the flags a context holds."""
+    taken = 0
+    for n in [10, 256, 257, 512, 1024, 1025, 4096, 10000, 20000, 32768, 32769, 50000, 65536, 65537, 98304, 131072,
+              131073, 200000, 262144, 262145, 500000]:
+        rw, wgs = rule(n, kind, cus)
+        if rw:
+            taken += 1
+            assert wgs * 256 * rw >= n and wgs <= min(cus, 256)
+        else:
+            assert -(-n // (512 if kind > -2 else 1024)) > min(cus, 256) or -(-n // 512) > min(cus, 256)
+    assert taken
+
+
+def test_batch_chains_scale_with_the_device():
+    """A chain takes a quarter of the CUs at most, and workgroups of two row
+    waves while the launch's rows fit 512 a CU."""
+    assert batch_rule(131072, 20000, 256) == (2, 64)
+    assert batch_rule(131073, 20000, 256) == (4, 64)
+    assert batch_rule(131072, 32769, 256) == (4, 64)
+    assert batch_rule(20000, 4096, 64) == (2, 16)
+    assert batch_rule(32769, 4096, 64) == (4, 16)
+    assert batch_rule(20000, 8193, 64) == (4, 16)
+    assert batch_rule(1000, 500, 3)[1] == 0
+
+
+def test_shapes_that_keep_the_ordinary_kernels():
+    assert rule(10000, -2, 256, jnd=192)[0] and not rule(10000, -2, 256, jnd=193)[0]
+    assert not rule(262145, -2, 256)[0] and not rule(131073, 0, 256)[0]
+    assert rule(10000, 0, 256, nnz=2048)[0] and not rule(10000, 0, 256, nnz=2049)[0]
+    assert rule(10000, 0, 256, nb=160)[0] and not rule(10000, 0, 256, nb=161)[0]
