@@ -3317,10 +3317,13 @@ void chains_plan(const std::vector<BatchStep> &S, StepsPlan &P, std::vector<char
             if (taken[k] || S[k].ci != 0 || spmv_kind(S[k].A) != cg.kind || (S[k].c->V32 != nullptr) != cg.mixed ||
                 !chain_form(S[k].qa, S[k].jnd, S[k].rcol) || !chain_fits_wg(S[k].c, S[k].A, S[k].jnd, rw0, maxg))
                 continue;
-            // its followers are recorded right after it
+            // its followers are recorded right after it; those past the
+            // kernel's columns are dropped (their go flags stay 0, so the
+            // solver records them again), not left to the phase kernels,
+            // whose own flag the chain does not set
             StepsPlan::Chain ch{S[k], 1};
             taken[k] = 1;
-            for (size_t f = k + 1; f < S.size() && S[f].c == S[k].c && S[f].ci == ch.K; ++f) {
+            for (size_t f = k + 1; f < S.size() && S[f].c == S[k].c && S[f].ci == (int)(f - k); ++f) {
                 taken[f] = 1;
                 if (S[f].jnd <= kChainMaxCols) ++ch.K;
             }

@@ -174,3 +174,23 @@ def test_step_any_column(gpu_lib, kind, size, mixed):
             assert (np.abs(out - want) <= tol * jnd * (1 + scale) ** 2).all(), (out, want)
     c.close()
     A.close()
+
+
+@pytest.mark.parametrize("maxlan", [194, 200, 210])
+def test_chain_past_its_columns_after_phases(gpu_lib, maxlan):
+    """A batch that starts phase by phase and, its larger solves done, goes on
+    in chains, past the columns a chain takes: the steps cut off must not run
+    on what the phase kernels left."""
+    T = gpu_lib
+    n = 3001
+    A = T.Csr(*W.random_sym_csr(n, seed=9))
+    args = (1, 6, maxlan, 1e-8, 1, 450, 6)
+    x0 = W.start_vector(n, seed=3)
+    one = T.solve_csr(A, *args, x0)
+    F, fx = filler(T)
+    fill = [(F, -1, 2, 24, 1e-14, 1, 60, 2, fx)] * 22
+    print(f"n={n} maxlan={maxlan}", flush=True)
+    rc, got, _ = T.solve_batch([(A,) + args + (x0,)] + fill)
+    A.close()
+    assert rc == 0
+    same(one, got[0])
