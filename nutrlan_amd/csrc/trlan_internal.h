@@ -59,13 +59,13 @@ int trlhip_ctx_create_batched(trlhip_ctx **c, int n, int ncols, int vtype, trlhi
  * Gram-Schmidt pass (kept and ntot as lz_orth sees them), and the solver
  * then takes its results from trlhip_step_cgs without a wait of its own. */
 int trlhip_step_chain(trlhip_ctx *c, int steps, int kept, int ntot);
-/* The rules of the chain kernels.  A single solve's step of n rows on a
- * device of `cus` CUs, `kind` the operator's SpMV kernel (-3, -2 stencils, -1
+/* The rules of the chain kernels.  A single solve's step of n rows (mixed:
+ * with an FP32 shadow) on a device of `cus` CUs, `kind` the operator's SpMV kernel (-3, -2 stencils, -1
  * packed CSR, 0 CSR) with nb row blocks of at most max_blk_nnz nonzeros: the
  * row waves of its workgroups, *wgs of them, or 0 where it runs as ordinary
  * kernels.  A batch whose chains hold `rows` rows, maxn at most each: the row
  * waves of its stencils' workgroups, and at most *maxg workgroups a chain. */
-int trlhip_chain_rule(int n, int kind, int nb, int max_blk_nnz, int jnd, int cus, int *wgs);
+int trlhip_chain_rule(int n, int kind, int mixed, int nb, int max_blk_nnz, int jnd, int cus, int *wgs);
 int trlhip_batch_chain_rule(long rows, int maxn, int cus, int *maxg);
 
 /* The reference's basis debug checks on a device basis (trl_debug.c):

@@ -2208,14 +2208,28 @@ bool recproj_ok(const trlhip_ctx *c)
     return c->E == 1 && (long)c->n <= (long)kMaxGrid * kMinRowsUpd;
 }
 
-// Row waves (256 rows each) per workgroup of a chain kernel.  The stencil
-// kernels take 4 above 32,768 rows: a barrier among 64 workgroups costs 2.7
-// us against 1.6 among 32, which outweighs the shorter phases of smaller
-// workgroups (181^2 sites, mixed: 9.2 ms a solve with 4, 9.9 with 2; 100^2
-// sites: 6.5 with 4, 6.4 with 2).  The CSR kinds keep 2: with 4, their
-// prefetched nonzeros no longer fit the 128 registers a thread of 16 waves
-// has (n = 50,001, 17 nonzeros a row: the product takes 30 us against 16).
-int chain_rw(int kind, int n) { return kind <= -2 && n > 32768 ? 4 : 2; }
+// At most a workgroup per CU: they all wait for each other.
+int chain_max_wgs(int cus) { return std::min(kChainMaxWG, cus); }
+int chain_wgs(int n, int rw) { return (n + 256 * rw - 1) / (256 * rw); }
+
+// Row waves (256 rows each) per workgroup of a chain kernel: the phases of
+// workgroups of 2 are shorter, a barrier among half as many of 4 is cheaper.
+// Stencils take 4 where 2 would be more workgroups than CUs (FP64; 2 also
+// keep 32 columns in registers) or than half of them (mixed: no difference
+// beyond what runs differ by up to n = 100,000, 4 better from there).  A
+// solve with 4 against 2, 2-D lattices, FP64: n = 10,000 6.16 and 5.21 ms,
+// 32,761 7.58 and 7.41, 65,536 10.0 and 9.3, 102,400 14.3 and 13.2, 131,044
+// 13.1 and 12.9; mixed: 10,000 6.37 and 5.67, 32,761 7.82 and 8.00, 36,100
+// 7.63 and 7.71, 57,600 11.7 and 11.3, 92,416 10.1 and 10.1, 112,896 19.0 and
+// 19.7, 122,500 15.7 and 16.8.  3-D ones, n = 64,000, 27.6 and 24.4, mixed
+// 26.2 and 25.5.  The CSR kinds keep 2: with 4, their prefetched nonzeros no
+// longer fit the 128 registers a thread of 16 waves has (n = 50,001, 17
+// nonzeros a row: the product takes 30 us against 16).
+int chain_rw(int kind, int n, bool mixed, int cus)
+{
+    const int most = mixed ? chain_max_wgs(cus) / 2 : chain_max_wgs(cus);
+    return kind <= -2 && chain_wgs(n, 2) > most ? 4 : 2;
+}
 
 // Whether a step of a single solve runs as a chain kernel: real solves with
 // a stencil or CSR-stream operator whose workgroups fit kChainMaxWG (n <=
@@ -2226,7 +2240,6 @@ int chain_rw(int kind, int n) { return kind <= -2 && n > 32768 ? 4 : 2; }
 // random rows n = 50,001 69 -> 48 ms (with the faster restarts and columns
 // kept in registers since: 4.6, 5.4 and, for the random rows, 44 ms).
 constexpr int kChainCsrIter = 4;
-int chain_wgs(int n, int rw) { return (n + 256 * rw - 1) / (256 * rw); }
 bool chain_shape(int n, int kind, int nb, int max_blk_nnz, int jnd, int rw, int maxg)
 {
     const int g = chain_wgs(n, rw);
@@ -2238,11 +2251,13 @@ bool chain_fits_wg(const trlhip_ctx *c, const trlhip_csr *A, int jnd, int rw, in
     if (!A || c->E != 1 || c->chain_off || A->lpr || A->pn_on) return false;
     return chain_shape(A->n, spmv_kind(A), A->nb, A->max_blk_nnz, jnd, rw, maxg);
 }
-// At most a workgroup per CU: they all wait for each other.
-int chain_max_wgs(int cus) { return std::min(kChainMaxWG, cus); }
+int chain_rw(const trlhip_ctx *c, const trlhip_csr *A)
+{
+    return chain_rw(spmv_kind(A), A->n, c->V32 != nullptr, c->cus);
+}
 bool chain_fits(const trlhip_ctx *c, const trlhip_csr *A, int jnd)
 {
-    return !c->batch && A && chain_fits_wg(c, A, jnd, chain_rw(spmv_kind(A), A->n), chain_max_wgs(c->cus));
+    return !c->batch && A && chain_fits_wg(c, A, jnd, chain_rw(c, A), chain_max_wgs(c->cus));
 }
 // The form of a step that chain kernels take, the solver's: q_a is the last
 // basis column and r goes to the column after it.  They keep q_a in LDS and,
@@ -4870,7 +4885,7 @@ static int run_chain(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int 
                      const double *beta, int jnd, int rcol, int K)
 {
     ChainArgs q{};
-    const int rw = chain_rw(spmv_kind(A), A->n);
+    const int rw = chain_rw(c, A);
     chain_args(q, c, A, rw, first, qa, qb, beta_prev, jnd, rcol, K, c->ch_kept, c->ch_ntot);
     if (c->pend_dst == qa && rcol != c->pend_src) {
         q.x = colp<double>(c, c->pend_src);
@@ -5111,9 +5126,9 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
     return 0;
 }
 
-int trlhip_chain_rule(int n, int kind, int nb, int max_blk_nnz, int jnd, int cus, int *wgs)
+int trlhip_chain_rule(int n, int kind, int mixed, int nb, int max_blk_nnz, int jnd, int cus, int *wgs)
 {
-    const int rw = chain_rw(kind, n);
+    const int rw = chain_rw(kind, n, mixed != 0, cus);
     if (wgs) *wgs = chain_wgs(n, rw);
     return chain_shape(n, kind, nb, max_blk_nnz, jnd, rw, chain_max_wgs(cus)) ? rw : 0;
 }

@@ -6,9 +6,9 @@ import pytest
 from nutrlan_amd import trlan as T
 
 
-def rule(n, kind, cus, nb=None, nnz=1000, jnd=20):
+def rule(n, kind, cus, nb=None, nnz=1000, jnd=20, mixed=0):
     wgs = ctypes.c_int()
-    rw = T.lib().trlhip_chain_rule(n, kind, -(-n // 256) if nb is None else nb, nnz, jnd, cus, ctypes.byref(wgs))
+    rw = T.lib().trlhip_chain_rule(n, kind, mixed, -(-n // 256) if nb is None else nb, nnz, jnd, cus, ctypes.byref(wgs))
     return rw, wgs.value
 
 
@@ -19,21 +19,30 @@ def batch_rule(rows, maxn, cus):
     return f(rows, maxn, cus, ctypes.byref(maxg)), maxg.value
 
 
+@pytest.mark.parametrize("mixed", [0, 1])
 @pytest.mark.parametrize("kind", [-3, -2, -1, 0])
 @pytest.mark.parametrize("cus", [1, 2, 16, 32, 38, 64, 80, 128, 228, 256, 304])
-def test_workgroups_fit_the_device(kind, cus):
+def test_workgroups_fit_the_device(kind, cus, mixed):
     """All workgroups of a chain wait for each other, so there is at most one
     per CU, and never more than the flags a context holds."""
     taken = 0
     for n in [10, 256, 257, 512, 1024, 1025, 4096, 10000, 20000, 32768, 32769, 50000, 65536, 65537, 98304, 131072,
               131073, 200000, 262144, 262145, 500000]:
-        rw, wgs = rule(n, kind, cus)
+        rw, wgs = rule(n, kind, cus, mixed=mixed)
         if rw:
             taken += 1
             assert wgs * 256 * rw >= n and wgs <= min(cus, 256)
         else:
-            assert -(-n // (512 if kind > -2 else 1024)) > min(cus, 256) or -(-n // 512) > min(cus, 256)
+            assert -(-n // (512 if kind > -2 else 1024)) > min(cus, 256)
     assert taken
+
+
+def test_row_waves():
+    for kind in (-2, -3):
+        assert rule(131072, kind, 256) == (2, 256) and rule(131073, kind, 256) == (4, 129)
+        assert rule(65536, kind, 256, mixed=1) == (2, 128) and rule(65537, kind, 256, mixed=1) == (4, 65)
+        assert rule(20000, kind, 32) == (4, 20) and rule(32769, kind, 32)[0] == 0
+    assert rule(131072, 0, 256, mixed=1) == (2, 256)
 
 
 def test_batch_chains_scale_with_the_device():

@@ -60,6 +60,12 @@ def test_chain_lattice2d(gpu_lib, L, mixed):
     both(gpu_lib, W.anderson2d_csr(L, 6.0, seed=L)[0], mixed, -1, 6, 24, maxmv=120 if L > 200 else 4000)
 
 
+@pytest.mark.parametrize("mixed,L", [(True, 256), (True, 257), (False, 257), (False, 361)])
+def test_chain_lattice2d_row_waves(gpu_lib, L, mixed):
+    """Either side of the line between workgroups of 2 and of 4 row waves."""
+    both(gpu_lib, W.anderson2d_csr(L, 6.0, seed=L)[0], mixed, -1, 6, 24, maxmv=120)
+
+
 @pytest.mark.parametrize("mixed", [False, True])
 @pytest.mark.parametrize("L", [8, 11, 32, 33, 64])
 def test_chain_lattice3d(gpu_lib, L, mixed):
