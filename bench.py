@@ -452,6 +452,7 @@ def batched_anderson2d(args):
     net.close()
 
     # the batched kernels (b_*: one launch steps every solve of a lane)
+    # except in its last, small rounds, which run as chains (b_chain)
     path = ["b_spmv", "b_recur", "b_proj", "b_update"]
     dom = max(path, key=lambda k: stats[k][1])
     launches, ms, byts = stats[dom]
@@ -606,10 +607,10 @@ def single_solve(T, args):
     nec = g["nec"]
 
     # roofline: dominant kernel by time, plus the path aggregate
-    dom = max(("spmv", "recur", "proj", "update", "ritz"), key=lambda k: stats[k][1])
+    dom = max(("spmv", "recur", "proj", "update", "ritz", "chain"), key=lambda k: stats[k][1])
     launches, ms, byts = stats[dom]
     achieved = byts / (ms * 1e-3) / 1e9 if ms > 0 else 0.0
-    pk = ["spmv", "recur", "proj", "update"]
+    pk = ["spmv", "recur", "proj", "update", "chain"]
     pb = sum(stats[k][2] for k in pk)
     pt = sum(stats[k][1] for k in pk)
     path_gbs = pb / (pt * 1e-3) / 1e9 if pt > 0 else 0.0

@@ -297,7 +297,10 @@ enum {
     TRLHIP_K_BPROJ = 8,
     TRLHIP_K_BUPDATE = 9,
     TRLHIP_K_BRITZ = 10,
-    TRLHIP_K_COUNT = 11
+    /* chains of steps in one kernel: a single solve's and a batch's */
+    TRLHIP_K_CHAIN = 11,
+    TRLHIP_K_BCHAIN = 12,
+    TRLHIP_K_COUNT = 13
 };
 
 /* Per-kernel HIP-event timing: on = 0 disables, on = N > 0 times every

@@ -1790,6 +1790,7 @@ struct Timed {
         b = ev_get();
         if (a && b) g_launch_ev = LaunchEvents{a, b};
     }
+    bool on() const { return a && b; }
     ~Timed()
     {
         if (!a && !b) return;
@@ -1811,6 +1812,13 @@ struct Timed {
         g_stats.pending.push_back({a, b, k});
     }
 };
+
+// Bytes of a timed launch that are known only once it has run.
+void stats_add_bytes(int k, double bytes)
+{
+    std::lock_guard<std::mutex> lk(g_stats_mu);
+    g_stats.bytes[k] += bytes;
+}
 
 }  // namespace
 
@@ -1900,6 +1908,7 @@ struct trlhip_ctx {
     unsigned sync_base;
     int gate_parity, chain_off;
     int cus;                          // CUs of its device
+    int chain_timed;                  // the chain kernel its step runs in is timed
     int ch_copy_ok;                   // that follower's fused normalisation was claimed
     int ch_qa[kChainMax], ch_qb[kChainMax], ch_rcol[kChainMax], ch_jnd[kChainMax];
 };
@@ -3263,13 +3272,17 @@ static void chain_args(ChainArgs &q, trlhip_ctx *c, const trlhip_csr *A, int rw,
     q.hchain = c->dres + hres_chain(c->ncols);
 }
 
-// The chain's algorithmic bytes if every step runs.
-static double chain_bytes(const trlhip_ctx *c, const trlhip_csr *A, int jnd, int K)
+// Adds the algorithmic bytes of the steps a timed chain kernel ran.
+static void chain_credit(trlhip_ctx *c, const trlhip_csr *A, int jnd, int K, int kind)
 {
+    if (!c->chain_timed) return;
+    c->chain_timed = 0;
     double bytes = 0.0;
-    for (int k = 0; k < K; ++k)
+    for (int k = 0; k < K; ++k) {
+        if (k > 0 && c->hres[hres_chain(c->ncols) + 7 * (size_t)(k - 1) + 4] != 1.0) break;
         bytes += spmv_bytes(A, 1, 8, 8) + ((c->V32 ? 8.0 : 16.0) * (jnd + k) + 40.0) * c->n;
-    return bytes;
+    }
+    stats_add_bytes(kind, bytes);
 }
 
 // (Grouping the launches group-major instead, so one group's vectors stay
@@ -3295,7 +3308,6 @@ struct StepsPlan {
         int kind, R, wgs;
         bool mixed;
         size_t doff, poff, foff;  // first record, prefix entry, flag word (the ticket)
-        double bytes;
     };
     std::vector<Chain> chains;
     std::vector<ChainGroup> cgroups;
@@ -3404,7 +3416,6 @@ void steps_plan(const std::vector<BatchStep> &steps, size_t ncbuf, StepsPlan &P,
                 const BatchStep &st = P.chains[cg.doff + i].st;
                 const int g = (st.c->n + 256 * rw - 1) / (256 * rw);
                 cg.wgs += g;
-                cg.bytes += chain_bytes(st.c, st.A, st.jnd, P.chains[cg.doff + i].K);
                 flags += 64 + (size_t)((g + 63) & ~63);  // its gate word, its flags
             }
         }
@@ -3470,7 +3481,8 @@ int steps_launch(hipStream_t s, const StepsPlan &P, const char *h, const char *d
     const int *dcp = reinterpret_cast<const int *>(d + P.off_chpre);
     unsigned *df = reinterpret_cast<unsigned *>(const_cast<char *>(d) + P.off_flags);
     for (const StepsPlan::ChainGroup &cg : P.cgroups) {
-        Timed t(TRLHIP_K_MISC, s, cg.bytes);
+        Timed t(TRLHIP_K_BCHAIN, s, 0.0);
+        for (int i = 0; i < cg.R; ++i) P.chains[cg.doff + i].st.c->chain_timed = t.on();
         const ChainArgs *q = dch + cg.doff;
         const int *pp = dcp + cg.poff;
         unsigned *ticket = df + cg.foff;
@@ -4906,7 +4918,8 @@ static int run_chain(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int 
     c->hres[6] = 0.0;
     for (int k = 1; k < K; ++k) c->hres[hres_chain(c->ncols) + 7 * (size_t)(k - 1) + 4] = 0.0;
     {
-        Timed t(TRLHIP_K_MISC, c->s, chain_bytes(c, A, jnd, K));
+        Timed t(TRLHIP_K_CHAIN, c->s, 0.0);
+        c->chain_timed = t.on();
 #define CHAIN_LAUNCH(RW, KIND)                                                                 \
     do {                                                                                       \
         if (c->V32)                                                                            \
@@ -4938,6 +4951,7 @@ static int run_chain(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int 
         return 0;
     }
     if (status != 1.0) return TRLHIP_EHIP;
+    chain_credit(c, A, jnd, K, TRLHIP_K_CHAIN);
     if (q.store_q) c->pend_dst = -1;
     for (int k = 1; k < K; ++k) {
         c->ch_qa[k] = rcol + k - 1;
@@ -5034,6 +5048,7 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
             if (int rc = ctx_wait(c)) return rc;
         }
         if (hr[6] == 3.0) return TRLHIP_EHIP;  // a chain kernel's wait ran out
+        if (hr[6] == 1.0) chain_credit(c, A, jnd, std::max(1, c->ch_n), TRLHIP_K_BCHAIN);
         out[0] = hr[S_ALPHA];
         out[1] = hr[S_RR2];
         out[2] = hr[S_HH];

@@ -22,7 +22,8 @@ LIBPATH = os.path.join(_HERE, "libnutrlan_amd.so")
 TRLHIP_R64, TRLHIP_C128, TRLHIP_R32 = 0, 1, 2
 TRLHIP_STAT_DEVICE = -1201
 KERNELS = ["spmv", "recur", "proj", "update", "ritz", "misc",
-           "b_spmv", "b_recur", "b_proj", "b_update", "b_ritz"]  # b_: batched kernels
+           "b_spmv", "b_recur", "b_proj", "b_update", "b_ritz",  # b_: batched kernels
+           "chain", "b_chain"]  # whole chains of steps
 
 _lib = None
 
@@ -545,6 +546,10 @@ class Ctx:
         self._chk(lib().trlhip_step_cgs(self.h, A.handle if A is not None else None, first, qa,
                                         qb, beta_prev, _ptr(b), jnd, rcol, _ptr(out)), "step_cgs")
         return out
+
+    def step_chain(self, steps, kept, ntot):
+        """Allows the next step up to steps - 1 followers (trlhip_step_chain)."""
+        self._chk(lib().trlhip_step_chain(self.h, steps, kept, ntot), "step_chain")
 
     def ritz(self, lck, jl, k, Y):
         Y = np.asfortranarray(Y, dtype=np.float64)

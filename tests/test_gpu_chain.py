@@ -200,3 +200,44 @@ def test_chain_past_its_columns_after_phases(gpu_lib, maxlan):
     A.close()
     assert rc == 0
     same(one, got[0])
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_chain_statistics(gpu_lib, mixed):
+    """Chain kernels are a class of their own, with the bytes of the steps
+    that ran: a chain over columns that are not orthogonal stops after one."""
+    T = gpu_lib
+    L, ncols = 40, 30
+    n = L * L
+    A = T.Csr(*W.anderson2d_csr(L, 6.0, seed=1)[0], mixed=mixed)
+    c = T.Ctx(n, ncols, mixed=mixed)
+    rng = np.random.default_rng(1)
+    for j in range(ncols):
+        c.set(j, rng.standard_normal(n) / np.sqrt(n))
+
+    def step(steps, jnd):
+        T.stats_enable(True)
+        if steps > 1:
+            c.step_chain(steps, 0, n)
+        c.step_cgs(A, 0, jnd - 1, -1, 0.0, None, jnd, jnd)
+        st = T.stats_get()
+        T.stats_enable(False)
+        assert {k for k, s in st.items() if s[0]} == {"chain"} and st["chain"][0] == 1
+        return st["chain"][2]
+
+    one = step(1, 8)
+    assert one > 0 and step(8, 8) == one
+    # a column more: read twice as stored
+    assert step(1, 9) - one == 2 * (4 if mixed else 8) * n
+    c.close()
+    # a solve: every step in a chain, none as ordinary kernels
+    T.stats_enable(True)
+    T.solve_csr(A, -1, 6, 24, 1e-8, 1, 500, 6, W.start_vector(n, seed=3))
+    st = T.stats_get()
+    T.stats_enable(True)
+    T.solve_batch([(A, -1, 6, 24, 1e-8, 1, 500, 6, W.start_vector(n, seed=3))])
+    bst = T.stats_get()
+    T.stats_enable(False)
+    A.close()
+    assert st["chain"][0] > 10 and st["b_chain"][0] == 0 and st["recur"][0] == 0
+    assert bst["b_chain"][0] > 10 and bst["chain"][0] == 0 and bst["b_update"][0] == 0
