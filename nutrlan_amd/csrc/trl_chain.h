@@ -35,9 +35,9 @@
 // Termination: a chain's workgroups first meet at a gate (chain_gate).
 // Either all of them are running and the chain starts, or -- the device is
 // filled by other work -- the gate closes after a while, nothing has been
-// written and the host runs the step's ordinary kernels.  Past the gate
-// every workgroup is resident, so each barrier ends; its wait is bounded all
-// the same.
+// written and the host runs the step's ordinary kernels (chain_shut).  Past
+// the gate every workgroup is resident, so each barrier ends; its wait is
+// bounded all the same.
 #ifndef TRL_CHAIN_H
 #define TRL_CHAIN_H
 
@@ -146,7 +146,7 @@ __device__ __forceinline__ bool chain_gate(const ChainArgs &q, int b, int *ok_s)
                 const unsigned f = __hip_atomic_load(q.sync + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 in = in && (int)(f - want) >= 0;
             }
-            const bool all = __all(in);
+            const bool all = __all(in) && q.gate_ticks;  // a gate of no ticks never opens
             const bool late = wall_clock64() - t0 > q.gate_ticks;
             if (lane == 0) {
                 if (all || late) {

@@ -59,6 +59,12 @@ int trlhip_ctx_create_batched(trlhip_ctx **c, int n, int ncols, int vtype, trlhi
  * Gram-Schmidt pass (kept and ntot as lz_orth sees them), and the solver
  * then takes its results from trlhip_step_cgs without a wait of its own. */
 int trlhip_step_chain(trlhip_ctx *c, int steps, int kept, int ntot);
+/* How long the context's chains wait at their gate for all their workgroups
+ * to run (0: no gate opens; at most a batch's 200 ms) and how long its steps
+ * run as ordinary kernels once one has closed, in 10 ns; and how many chains
+ * ran and how many gates closed so far. */
+int trlhip_ctx_chain_gate(trlhip_ctx *c, unsigned long long ticks, unsigned long long hold);
+int trlhip_ctx_chain_counts(const trlhip_ctx *c, long *ran, long *closed);
 /* The rules of the chain kernels.  A single solve's step of n rows (mixed:
  * with an FP32 shadow) on a device of `cus` CUs, `kind` the operator's SpMV kernel (-3, -2 stencils, -1
  * packed CSR, 0 CSR) with nb row blocks of at most max_blk_nnz nonzeros: the

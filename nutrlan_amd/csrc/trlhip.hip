@@ -18,6 +18,7 @@
 #include <cfloat>
 #include <cmath>
 #include <atomic>
+#include <chrono>
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -1903,10 +1904,17 @@ struct trlhip_ctx {
     int ch_n, ch_next;                // steps in the chain; next follower to hand out (0: none)
     // chain kernels of a single solve (k_chain): its flags and gate words
     // (after dscal's scalars), the flag value used so far, the gate word in
-    // turn, and whether a gate has closed (the ordinary kernels from then on)
+    // turn
     unsigned *sync;
     unsigned sync_base;
-    int gate_parity, chain_off;
+    int gate_parity;
+    // how long its chains wait at their gate (0: none opens) and are left alone
+    // after one has closed, in 10 ns; that one has, and until when the ordinary
+    // kernels run (chain_retry); chains run and closed
+    unsigned long long gate_ticks, gate_hold;
+    int chain_off;
+    double chain_until;
+    long chain_ran, chain_closed;
     int cus;                          // CUs of its device
     int chain_timed;                  // the chain kernel its step runs in is timed
     int ch_copy_ok;                   // that follower's fused normalisation was claimed
@@ -2268,6 +2276,30 @@ bool chain_fits(const trlhip_ctx *c, const trlhip_csr *A, int jnd)
 {
     return !c->batch && A && chain_fits_wg(c, A, jnd, chain_rw(c, A), chain_max_wgs(c->cus));
 }
+// A gate closes when other work fills the device.  The context's steps then
+// run as ordinary kernels for 16 times the wait, so that waiting costs at most
+// a sixteenth of the time however long that lasts, and a solve that met other
+// work once goes on in chains.
+double host_seconds()
+{
+    return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
+}
+void chain_gate_times(trlhip_ctx *c, unsigned long long ticks)
+{
+    c->gate_ticks = ticks;
+    c->gate_hold = 16 * ticks;
+}
+void chain_shut(trlhip_ctx *c)
+{
+    c->chain_off = 1;
+    c->chain_until = host_seconds() + 1e-8 * (double)c->gate_hold;
+    ++c->chain_closed;
+}
+void chain_retry(trlhip_ctx *c)
+{
+    if (c->chain_off && host_seconds() >= c->chain_until) c->chain_off = 0;
+}
+
 // The form of a step that chain kernels take, the solver's: q_a is the last
 // basis column and r goes to the column after it.  They keep q_a in LDS and,
 // some of them, the columns before it in registers; the step kernels, which
@@ -3458,7 +3490,7 @@ void steps_fill(const std::vector<double> &cbuf, StepsPlan &P, char *h, const ch
             q.store_q = st.fuse;
             q.coef = st.coff >= 0 ? dcbuf + st.coff : nullptr;
             q.gate = df + fl;
-            q.gate_ticks = kBatchGateTicks;
+            q.gate_ticks = st.c->gate_ticks;
             q.sync = df + fl + 64;
             fl += 64 + (size_t)((q.g + 63) & ~63);
             pp[i + 1] = pp[i] + q.g;
@@ -4537,6 +4569,7 @@ int trlhip_ctx_create_batched(trlhip_ctx **out, int n, int ncols, int vtype, trl
         std::lock_guard<std::mutex> lk(b->arena_mu);
         c->batch = b;
         c->cus = b->cus;
+        chain_gate_times(c, kBatchGateTicks);
         c->s = b->side;
         c->arena = 1;
         const size_t np = part_need(c->E, ncols);
@@ -4565,6 +4598,7 @@ int trlhip_ctx_create_batched(trlhip_ctx **out, int n, int ncols, int vtype, trl
         return 0;
     }
     c->cus = device_cus();
+    chain_gate_times(c, kGateTicks);
     if (hipStreamCreate(&c->s) != hipSuccess) rc = TRLHIP_EHIP;
     if (!rc && hipMalloc((void **)&c->V, vbytes) != hipSuccess) rc = TRLHIP_ENOMEM;
     const size_t sbytes = sizeof(float) * (size_t)c->ld * (ncols + 1);
@@ -4891,8 +4925,7 @@ static int run_phases(trlhip_ctx *c, const trlhip_csr *A, int qa, int qb, double
 // Runs a step and up to K - 1 followers of a single real solve as one
 // kernel (k_chain); sets the followers up as a batch's recorded chain does.
 // Returns 1 when the step ran, 0 when it must run as ordinary kernels (the
-// gate closed: the device is filled by other work, so the context keeps to
-// them from then on), or an error.
+// gate closed), or an error.
 static int run_chain(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int qb, double beta_prev,
                      const double *beta, int jnd, int rcol, int K)
 {
@@ -4914,7 +4947,7 @@ static int run_chain(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int 
     q.base = c->sync_base;
     q.gate = c->sync + kChainGate + 32 * c->gate_parity;
     q.gate_next = c->sync + kChainGate + 32 * (1 - c->gate_parity);
-    q.gate_ticks = kGateTicks;
+    q.gate_ticks = c->gate_ticks;
     c->hres[6] = 0.0;
     for (int k = 1; k < K; ++k) c->hres[hres_chain(c->ncols) + 7 * (size_t)(k - 1) + 4] = 0.0;
     {
@@ -4947,10 +4980,11 @@ static int run_chain(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int 
     if (int rc = ctx_wait(c)) return rc;
     const double status = *(const volatile double *)(c->hres + 6);
     if (status == 2.0) {
-        c->chain_off = 1;
+        chain_shut(c);
         return 0;
     }
     if (status != 1.0) return TRLHIP_EHIP;
+    ++c->chain_ran;
     chain_credit(c, A, jnd, K, TRLHIP_K_CHAIN);
     if (q.store_q) c->pend_dst = -1;
     for (int k = 1; k < K; ++k) {
@@ -4992,6 +5026,7 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
         }
         c->ch_next = 0;  // the chain stopped before this step: record it
     }
+    chain_retry(c);
     if (c->batch && A && c->E == 1) {
         // batched: record the step; trlhip_batch_flush runs it with the
         // other contexts' steps
@@ -5031,8 +5066,8 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
         const volatile double *hr = c->hres;
         if (hr[6] == 2.0) {
             // its chain's gate closed before anything was written: the step
-            // alone, as ordinary kernels (this context's from now on)
-            c->chain_off = 1;
+            // alone, as ordinary kernels
+            chain_shut(c);
             c->ch_next = 0;
             st.decide = 0;
             {
@@ -5048,7 +5083,10 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
             if (int rc = ctx_wait(c)) return rc;
         }
         if (hr[6] == 3.0) return TRLHIP_EHIP;  // a chain kernel's wait ran out
-        if (hr[6] == 1.0) chain_credit(c, A, jnd, std::max(1, c->ch_n), TRLHIP_K_BCHAIN);
+        if (hr[6] == 1.0) {
+            ++c->chain_ran;
+            chain_credit(c, A, jnd, std::max(1, c->ch_n), TRLHIP_K_BCHAIN);
+        }
         out[0] = hr[S_ALPHA];
         out[1] = hr[S_RR2];
         out[2] = hr[S_HH];
@@ -5146,6 +5184,22 @@ int trlhip_chain_rule(int n, int kind, int mixed, int nb, int max_blk_nnz, int j
     const int rw = chain_rw(kind, n, mixed != 0, cus);
     if (wgs) *wgs = chain_wgs(n, rw);
     return chain_shape(n, kind, nb, max_blk_nnz, jnd, rw, chain_max_wgs(cus)) ? rw : 0;
+}
+
+int trlhip_ctx_chain_gate(trlhip_ctx *c, unsigned long long ticks, unsigned long long hold)
+{
+    if (!c || ticks > kBatchGateTicks) return TRLHIP_EINVAL;
+    c->gate_ticks = ticks;
+    c->gate_hold = hold;
+    return 0;
+}
+
+int trlhip_ctx_chain_counts(const trlhip_ctx *c, long *ran, long *closed)
+{
+    if (!c || !ran || !closed) return TRLHIP_EINVAL;
+    *ran = c->chain_ran;
+    *closed = c->chain_closed;
+    return 0;
 }
 
 int trlhip_batch_chain_rule(long rows, int maxn, int cus, int *maxg)
