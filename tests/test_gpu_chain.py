@@ -6,7 +6,8 @@ counters bit for bit, at sizes around the kernels' edges (256 rows a wave,
 with several solves on the device at once.
 
 A batch too large for chains runs phase by phase, so each solve is compared
-with itself in a batch beside operators that fill it up."""
+with itself in a batch beside operators that fill it up; the kernel statistics
+say which kernels ran."""
 import threading
 
 import numpy as np
@@ -34,22 +35,38 @@ def filler(T):
     return _fill[0]
 
 
-def both(T, csr, mixed, lohi, ned, maxlan, tol=1e-8, maxmv=4000, seed=3):
+def counted(T, solve):
+    """solve() and the kernel launches of it by class."""
+    T.stats_enable(True)
+    r = solve()
+    st = T.stats_get()
+    T.stats_enable(False)
+    return r, {k: v[0] for k, v in st.items()}
+
+
+def both(T, csr, mixed, lohi, ned, maxlan, tol=1e-8, maxmv=4000, seed=3, dense=False):
+    """dense: a CSR operator with more nonzeros than chains take."""
     n = len(csr[0]) - 1
     A = T.Csr(*csr, mixed=mixed)
     args = (lohi, ned, maxlan, tol, 1, maxmv, ned)
     x0 = W.start_vector(n, seed=seed)
     print(f"n={n} mixed={mixed} stencil={A.stencil} packed={A.packed}", flush=True)
-    one = T.solve_csr(A, *args, x0)
-    rc, small, _ = T.solve_batch([(A,) + args + (x0,)])
+    one, k1 = counted(T, lambda: T.solve_csr(A, *args, x0))
+    (rc, small, _), k2 = counted(T, lambda: T.solve_batch([(A,) + args + (x0,)]))
     assert rc == 0
     # 2 x 11 fillers of 65,025 rows that stop after the same number of steps:
     # each of the batch's two lanes holds over 600,000 rows
     F, fx = filler(T)
-    fill = [(F, -1, 2, maxlan, 1e-14, 1, one["matvec"] + maxlan, 2, fx)] * 11
-    rc, large, _ = T.solve_batch([(A,) + args + (x0,)] + [fill[0]] + fill + fill[:9])
+    fill = [(F, -1, 8, maxlan, 1e-14, 1, one["matvec"] + maxlan, 8, fx)] * 11
+    (rc, large, _), k3 = counted(T, lambda: T.solve_batch([(A,) + args + (x0,)] + [fill[0]] + fill + fill[:9]))
+    stencil = A.stencil[0] > 0
     A.close()
     assert rc == 0
+    assert (k1["chain"] > 0) == (not dense and n <= (262144 if stencil else 131072)), k1
+    assert (k2["b_chain"] > 0) == (not dense and n <= (65536 if stencil else 32768)), k2
+    # fillers past a chain's columns are not among the rows that keep the
+    # batch from chains, so the last steps of such a cycle may be one
+    assert 10 * k3["b_chain"] <= (k2["b_chain"] if maxlan > 192 else 0) and k3["b_update"] > 0, k3
     same(one, small[0])
     same(one, large[0])
 
@@ -82,7 +99,7 @@ def test_chain_packed(gpu_lib, n):
 @pytest.mark.parametrize("n,degree", [(300, 16.0), (1023, 3.0), (4099, 16.0), (20001, 40.0), (131072, 4.0),
                                       (131073, 4.0)])
 def test_chain_random_rows(gpu_lib, n, degree, mixed):
-    both(gpu_lib, W.random_sym_csr(n, degree=degree, seed=n), mixed, 1, 10, 60, maxmv=130)
+    both(gpu_lib, W.random_sym_csr(n, degree=degree, seed=n), mixed, 1, 10, 60, maxmv=130, dense=degree == 40.0)
 
 
 def test_chain_wide_basis(gpu_lib):
@@ -196,9 +213,9 @@ def test_chain_past_its_columns_after_phases(gpu_lib, maxlan):
     F, fx = filler(T)
     fill = [(F, -1, 2, 24, 1e-14, 1, 60, 2, fx)] * 22
     print(f"n={n} maxlan={maxlan}", flush=True)
-    rc, got, _ = T.solve_batch([(A,) + args + (x0,)] + fill)
+    (rc, got, _), k = counted(T, lambda: T.solve_batch([(A,) + args + (x0,)] + fill))
     A.close()
-    assert rc == 0
+    assert rc == 0 and k["b_chain"] > 0 and k["b_update"] > 0
     same(one, got[0])
 
 
@@ -231,13 +248,8 @@ def test_chain_statistics(gpu_lib, mixed):
     assert step(1, 9) - one == 2 * (4 if mixed else 8) * n
     c.close()
     # a solve: every step in a chain, none as ordinary kernels
-    T.stats_enable(True)
-    T.solve_csr(A, -1, 6, 24, 1e-8, 1, 500, 6, W.start_vector(n, seed=3))
-    st = T.stats_get()
-    T.stats_enable(True)
-    T.solve_batch([(A, -1, 6, 24, 1e-8, 1, 500, 6, W.start_vector(n, seed=3))])
-    bst = T.stats_get()
-    T.stats_enable(False)
+    args = (A, -1, 6, 24, 1e-8, 1, 500, 6, W.start_vector(n, seed=3))
+    st, bst = counted(T, lambda: T.solve_csr(*args))[1], counted(T, lambda: T.solve_batch([args]))[1]
     A.close()
-    assert st["chain"][0] > 10 and st["b_chain"][0] == 0 and st["recur"][0] == 0
-    assert bst["b_chain"][0] > 10 and bst["chain"][0] == 0 and bst["b_update"][0] == 0
+    assert st["chain"] > 10 and st["b_chain"] == 0 and st["recur"] == 0
+    assert bst["b_chain"] > 10 and bst["chain"] == 0 and bst["b_update"] == 0
