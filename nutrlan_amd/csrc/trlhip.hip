@@ -1313,13 +1313,15 @@ __global__ __launch_bounds__(kBlock) void k_update(
 // the columns over four groups of 256 threads, by the running sum of
 // update_rows4 a column goes to (c mod 4; after the last full group of 8 all
 // to the first); complex bases give each group one of a thread's four rows.
-// The sums and their order are k_update's, so are the bits.  For row counts
-// whose blocks leave most of the device idle it puts four times the loads in
-// flight.  Whole passes (trlhip_cgs_pass_noalloc) before and after: complex n
-// = 60,000, m = 60 93 -> 55 us, FP64 n = 100,000, m = 80 81 -> 53, n =
-// 260,000, m = 30 66 -> 52, FP32 n = 200,000, m = 60 74 -> 50 (some 13 us of
-// each are the one copy back instead of two); the 48^3 complex lattice 132 ->
-// 104 ms a solve.  Above kWideRows the 256-thread blocks fill the device.
+// The sums and their order are k_update's, and of real bases the bits (which
+// of a complex product's two terms is rounded first is the compiler's choice
+// in each kernel).  For row counts whose blocks leave most of the device idle
+// it puts four times the loads in flight.  Whole passes
+// (trlhip_cgs_pass_noalloc) before and after: complex n = 60,000, m = 60 93 ->
+// 55 us, FP64 n = 100,000, m = 80 81 -> 53, n = 260,000, m = 30 66 -> 52, FP32
+// n = 200,000, m = 60 74 -> 50 (some 13 us of each are the one copy back
+// instead of two); the 48^3 complex lattice 132 -> 104 ms a solve.  Above
+// kWideRows the 256-thread blocks fill the device.
 constexpr int kWide = 4 * kBlock;
 
 // Four rows of a column (ld4; ld4u from any row) and one (ld1) for

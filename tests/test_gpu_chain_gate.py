@@ -153,3 +153,26 @@ def test_gate_closed_for_a_while(gpu_lib):
     assert counts(T, c)[0] == 1
     c.close()
     A.close()
+
+
+@pytest.mark.parametrize("size,complex_", [(12, True), (31, True), (65, True), (66, False)])
+def test_queued_steps(gpu_lib, size, complex_):
+    """Complex and larger solves queue their steps phase by phase: the bits of
+    the same steps taken one at a time."""
+    T = gpu_lib
+    csr = W.anderson3d_csr(size, seed=size) if complex_ else W.laplace3d_csr(size, seed=size)
+    n = len(csr[0]) - 1
+    A = T.Csr(*csr, complex_=complex_)
+    x0 = W.start_vector(n, seed=1, complex_=complex_)
+    m = 17
+    coef = np.random.default_rng(2).standard_normal(m) * 0.1
+    got = []
+    for steps in (1, 6):
+        print(f"n={n} complex={complex_} steps={steps}", flush=True)
+        c = T.Ctx(n, m + 8, complex_=complex_)
+        got.append(lanczos(c, A, n, m, steps, x0 / np.linalg.norm(x0), coef))
+        assert counts(T, c) == (0, 0)
+        c.close()
+    A.close()
+    assert np.array_equal(got[0][0], got[1][0])
+    assert np.array_equal(got[0][1], got[1][1])
