@@ -66,6 +66,7 @@ struct ChainArgs {
     unsigned *gate;         // this launch's gate word (zero)
     unsigned *gate_next;    // the next launch's, cleared at the end, or null
     unsigned long long gate_ticks;
+    unsigned *shut;         // a batch's launch: set once one of its gates has closed, else null
 };
 
 __device__ __forceinline__ double ld_agent(const double *p)
@@ -128,7 +129,9 @@ __device__ __forceinline__ bool chain_barrier(const ChainArgs &q, int b, unsigne
 
 // The gate: true in every workgroup when all g are running, false in every
 // workgroup when one of them gave up waiting first (the gate word is set
-// once: 1 open, 2 closed).
+// once: 1 open, 2 closed).  Once a chain of a batch's launch has waited in
+// vain the others do not wait: where few workgroups find a place, each chain
+// would spend the whole time anew.
 __device__ __forceinline__ bool chain_gate(const ChainArgs &q, int b, int *ok_s)
 {
     if (q.g == 1) return true;
@@ -147,14 +150,18 @@ __device__ __forceinline__ bool chain_gate(const ChainArgs &q, int b, int *ok_s)
                 in = in && (int)(f - want) >= 0;
             }
             const bool all = __all(in) && q.gate_ticks;  // a gate of no ticks never opens
-            const bool late = wall_clock64() - t0 > q.gate_ticks;
             if (lane == 0) {
+                const bool late =
+                    wall_clock64() - t0 > q.gate_ticks ||
+                    (q.shut && __hip_atomic_load(q.shut, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
                 if (all || late) {
                     unsigned seen = 0;
                     if (__hip_atomic_compare_exchange_strong(gate, &seen, all ? 1u : 2u, __ATOMIC_RELAXED,
                                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
                         seen = all ? 1u : 2u;
                     st = seen;
+                    if (st == 2 && q.shut)
+                        __hip_atomic_store(q.shut, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 } else {
                     st = __hip_atomic_load(gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }

@@ -2317,6 +2317,7 @@ bool chain_form(int qa, int jnd, int rcol) { return qa == jnd - 1 && rcol == jnd
 // 56.5, 39.9, 39.8, 37.8; 90 of 60-180 84.8, 77.5, 77.6, 79.6; 192 of 64-256,
 // mixed, 183, 170, 170, 174 (whose later rounds fit).
 constexpr long kBatchChainRows = 600000;
+constexpr int kChainShut = 32;     // the launch's shut word: in the first group's ticket block
 constexpr int kBatchChainWG = 64;  // workgroups of one solve at most, and a quarter of the CUs
 
 // A chain of a batch has at most maxg workgroups, of two row waves while all
@@ -3493,6 +3494,7 @@ void steps_fill(const std::vector<double> &cbuf, StepsPlan &P, char *h, const ch
             q.coef = st.coff >= 0 ? dcbuf + st.coff : nullptr;
             q.gate = df + fl;
             q.gate_ticks = st.c->gate_ticks;
+            q.shut = df + kChainShut;
             q.sync = df + fl + 64;
             fl += 64 + (size_t)((q.g + 63) & ~63);
             pp[i + 1] = pp[i] + q.g;

@@ -18,7 +18,10 @@ YIELD = ctypes.CFUNCTYPE(None, ctypes.c_void_p)
 
 
 class Batch:
-    """A batch of one context: what the context waits for runs at once."""
+    """A batch whose contexts are driven by one thread: what a context waits
+    for runs at once, with whatever `before` records first."""
+
+    before = None
 
     def __init__(self, T, n, ncols, mixed):
         L, P = T.lib(), ctypes.c_void_p
@@ -26,24 +29,33 @@ class Batch:
                            ("trlhip_batch_flush", [P]), ("trlhip_batch_destroy", [P]),
                            ("trlhip_ctx_create_batched", [P, ctypes.c_int, ctypes.c_int, ctypes.c_int, P])]:
             getattr(L, name).argtypes = args
-        self.L, self.b, self.flushes = L, P(), 0
+        self.L, self.b = L, P()
         assert L.trlhip_batch_create(ctypes.byref(self.b)) == 0
 
         def run(_):
-            self.flushes += 1
+            f, self.before = self.before, None
+            if f:
+                f()
             L.trlhip_batch_flush(self.b)
 
         self.cb = YIELD(run)
         L.trlhip_batch_set_yield(self.b, self.cb, None)
-        self.ctx = T.Ctx(1, 1)  # its bound functions, with the batch's handle
-        self.ctx.close()
-        h = P()
-        vt = T.TRLHIP_R32 if mixed else T.TRLHIP_R64
-        assert L.trlhip_ctx_create_batched(ctypes.byref(h), n, ncols, vt, self.b) == 0
-        self.ctx.h, self.ctx.n, self.ctx.ncols = h, n, ncols
+        self.T, self.all = T, []
+        self.ctx = self.add(n, ncols, mixed)
+
+    def add(self, n, ncols, mixed):
+        c = self.T.Ctx(1, 1)  # its bound functions, with the batch's handle
+        c.close()
+        h = ctypes.c_void_p()
+        vt = self.T.TRLHIP_R32 if mixed else self.T.TRLHIP_R64
+        assert self.L.trlhip_ctx_create_batched(ctypes.byref(h), n, ncols, vt, self.b) == 0
+        c.h, c.n, c.ncols = h, n, ncols
+        self.all.append(c)
+        return c
 
     def close(self):
-        self.ctx.close()
+        for c in self.all:
+            c.close()
         self.L.trlhip_batch_destroy(self.b)
 
 
@@ -153,6 +165,44 @@ def test_gate_closed_for_a_while(gpu_lib):
     assert counts(T, c)[0] == 1
     c.close()
     A.close()
+
+
+@pytest.mark.parametrize("closed", [0, 1])
+def test_closed_gate_beside_others(gpu_lib, closed):
+    """One of two chains of a launch has a gate that never opens: once it has
+    closed the other need not wait for its own, and either way both steps have
+    the bits they have alone."""
+    T = gpu_lib
+    sizes = (45, 60)
+    ops = [T.Csr(*W.anderson2d_csr(L, 6.0, seed=L)[0]) for L in sizes]
+    x0 = [W.start_vector(L * L, seed=L) for L in sizes]
+    x0 = [x / np.linalg.norm(x) for x in x0]
+    want = []
+    for A, x in zip(ops, x0):
+        c = T.Ctx(len(x), 6)
+        c.set(0, x)
+        want.append((c.step_cgs(A, 1, 0, -1, 0.0, np.zeros(0), 1, 1), c.get(1)))
+        c.close()
+    b = Batch(T, len(x0[0]), 6, False)
+    c = [b.ctx, b.add(len(x0[1]), 6, False)]
+    for k in (0, 1):
+        c[k].set(0, x0[k])
+    gate(T, c[closed], 0, 100000000)
+    print(f"closed={closed}", flush=True)
+    got = [None, None]
+
+    def step(k):
+        got[k] = c[k].step_cgs(ops[k], 1, 0, -1, 0.0, np.zeros(0), 1, 1)
+
+    b.before = lambda: step(1)  # recorded beside the first one's step
+    step(0)
+    assert counts(T, c[closed]) == (0, 1)
+    assert sum(counts(T, c[1 - closed])) == 1
+    for k in (0, 1):
+        assert np.array_equal(got[k], want[k][0]) and np.array_equal(c[k].get(1), want[k][1])
+    b.close()
+    for A in ops:
+        A.close()
 
 
 @pytest.mark.parametrize("size,complex_", [(12, True), (31, True), (65, True), (66, False)])
