@@ -66,12 +66,17 @@ int trlhip_step_chain(trlhip_ctx *c, int steps, int kept, int ntot);
 int trlhip_ctx_chain_gate(trlhip_ctx *c, unsigned long long ticks, unsigned long long hold);
 int trlhip_ctx_chain_counts(const trlhip_ctx *c, long *ran, long *closed);
 /* The rules of the chain kernels.  A single solve's step of n rows (mixed:
- * with an FP32 shadow) on a device of `cus` CUs, `kind` the operator's SpMV kernel (-3, -2 stencils, -1
+ * with an FP32 shadow) on a device of `cus` CUs where `active` solves are at
+ * work, `kind` the operator's SpMV kernel (-3, -2 stencils, -1
  * packed CSR, 0 CSR) with nb row blocks of at most max_blk_nnz nonzeros: the
  * row waves of its workgroups, *wgs of them, or 0 where it runs as ordinary
  * kernels.  A batch whose chains hold `rows` rows, maxn at most each: the row
  * waves of its stencils' workgroups, and at most *maxg workgroups a chain. */
-int trlhip_chain_rule(int n, int kind, int mixed, int nb, int max_blk_nnz, int jnd, int cus, int *wgs);
+int trlhip_chain_rule(int n, int kind, int mixed, int nb, int max_blk_nnz, int jnd, int cus, int active,
+                      int *wgs);
+/* Contexts of single solves in a step on device `dev` and workgroups of their
+ * chains: both 0 when no call is in progress. */
+int trlhip_device_load(int dev, int *steps, int *wgs);
 int trlhip_batch_chain_rule(long rows, int maxn, int cus, int *maxg);
 
 /* The reference's basis debug checks on a device basis (trl_debug.c):

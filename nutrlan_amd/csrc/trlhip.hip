@@ -1917,7 +1917,8 @@ struct trlhip_ctx {
     int chain_off;
     double chain_until;
     long chain_ran, chain_closed;
-    int cus;                          // CUs of its device
+    int cus, dev;                     // CUs of its device, and its entry of g_load
+    unsigned serial;                  // its own number among all contexts, from 1
     int chain_timed;                  // the chain kernel its step runs in is timed
     int ch_copy_ok;                   // that follower's fused normalisation was claimed
     int ch_qa[kChainMax], ch_qb[kChainMax], ch_rcol[kChainMax], ch_jnd[kChainMax];
@@ -2227,6 +2228,33 @@ bool recproj_ok(const trlhip_ctx *c)
     return c->E == 1 && (long)c->n <= (long)kMaxGrid * kMinRowsUpd;
 }
 
+constexpr int kMaxDevices = 64;
+
+double host_seconds()
+{
+    return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
+}
+
+// CUs of a device, queried once for each.
+int device_cus(int dev)
+{
+    static std::atomic<int> cus[kMaxDevices];
+    int n = 0;
+    if (dev < 0) return 1;
+    if (dev < kMaxDevices) n = cus[dev].load(std::memory_order_relaxed);
+    if (!n) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 1;
+        if (dev < kMaxDevices) cus[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
+
+int current_device()
+{
+    int dev = -1;
+    return hipGetDevice(&dev) == hipSuccess ? dev : -1;
+}
+
 // At most a workgroup per CU: they all wait for each other.
 int chain_max_wgs(int cus) { return std::min(kChainMaxWG, cus); }
 int chain_wgs(int n, int rw) { return (n + 256 * rw - 1) / (256 * rw); }
@@ -2270,22 +2298,84 @@ bool chain_fits_wg(const trlhip_ctx *c, const trlhip_csr *A, int jnd, int rw, in
     if (!A || c->E != 1 || c->chain_off || A->lpr || A->pn_on) return false;
     return chain_shape(A->n, spmv_kind(A), A->nb, A->max_blk_nnz, jnd, rw, maxg);
 }
-int chain_rw(const trlhip_ctx *c, const trlhip_csr *A)
+// The row waves of a chain of n rows beside `active` - 1 other solves, 0: no
+// chain.  Beside others a chain takes its share of the CUs, if need be with 4
+// row waves, and no more than a quarter of them beyond that.
+int chain_pick(int n, int kind, bool mixed, int nb, int max_blk_nnz, int jnd, int cus, int active)
 {
-    return chain_rw(spmv_kind(A), A->n, c->V32 != nullptr, c->cus);
+    int rw = chain_rw(kind, n, mixed, cus), maxg = chain_max_wgs(cus);
+    if (active > 1) {
+        maxg = std::min(maxg, cus / active);
+        if (kind <= -2 && chain_wgs(n, rw) > maxg) rw = 4;
+        maxg = std::max(maxg, std::min(kChainMaxWG, cus / 4));
+    }
+    return chain_shape(n, kind, nb, max_blk_nnz, jnd, rw, maxg) ? rw : 0;
 }
-bool chain_fits(const trlhip_ctx *c, const trlhip_csr *A, int jnd)
+
+// What single solves have on a device: contexts in a step, workgroups of
+// their chains, and the context that took the last step and when it was
+// another's turn.  A chain's workgroup has a CU to itself for the whole chain,
+// so chains that do not all fit would wait at their gates for each other, and
+// a chain of most of the device keeps the others' short kernels waiting.
+// Threads solving 2-D lattices at once, ms a solve, without chains, with
+// chains that know nothing of each other, and so: 8 of 100^2 4.4, 3.0, 3.0; 2
+// of 250^2 12.9, 9.4, 8.6, 16 6.8, 6.0, 5.9; 8 of 350^2 8.8, 9.1, 8.0; 2 of
+// 500^2 17.7, 20.7, 17.0, 8 14.0, 17.3, 14.5.
+struct DeviceLoad {
+    std::atomic<int> steps{0}, wgs{0};
+    std::atomic<unsigned> last{0};
+    std::atomic<double> turned{0.0};
+};
+DeviceLoad g_load[kMaxDevices + 1];  // the last: devices past the table
+
+// A context's step on its device, and its chain's workgroups.
+constexpr double kTurnSeconds = 2e-3;  // other solves' host work between steps is shorter
+struct StepOnDevice {
+    DeviceLoad &d;
+    int held = 0, active;
+    explicit StepOnDevice(const trlhip_ctx *c) : d(g_load[c->dev]), active(d.steps.fetch_add(1) + 1)
+    {
+        const double now = host_seconds();
+        const unsigned was = d.last.exchange(c->serial);
+        if (was && was != c->serial) d.turned.store(now);
+        if (active == 1 && now - d.turned.load() < kTurnSeconds) active = 2;
+    }
+    ~StepOnDevice()
+    {
+        if (held) d.wgs.fetch_sub(held);
+        d.steps.fetch_sub(1);
+    }
+    bool take(int wgs, int cus)
+    {
+        if (d.wgs.fetch_add(wgs) + wgs > cus) {
+            d.wgs.fetch_sub(wgs);
+            return false;
+        }
+        held = wgs;
+        return true;
+    }
+    void give()
+    {
+        d.wgs.fetch_sub(held);
+        held = 0;
+    }
+};
+// A context that ends has no more turns.
+void left_device(const trlhip_ctx *c)
 {
-    return !c->batch && A && chain_fits_wg(c, A, jnd, chain_rw(c, A), chain_max_wgs(c->cus));
+    unsigned me = c->serial;
+    (void)g_load[c->dev].last.compare_exchange_strong(me, 0u);
 }
+int chain_pick(const trlhip_ctx *c, const trlhip_csr *A, int jnd, int active)
+{
+    if (!A || c->batch || c->E != 1 || c->chain_off || A->lpr || A->pn_on) return 0;
+    return chain_pick(A->n, spmv_kind(A), c->V32 != nullptr, A->nb, A->max_blk_nnz, jnd, c->cus, active);
+}
+
 // A gate closes when other work fills the device.  The context's steps then
 // run as ordinary kernels for 16 times the wait, so that waiting costs at most
 // a sixteenth of the time however long that lasts, and a solve that met other
 // work once goes on in chains.
-double host_seconds()
-{
-    return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
-}
 void chain_gate_times(trlhip_ctx *c, unsigned long long ticks)
 {
     c->gate_ticks = ticks;
@@ -2326,21 +2416,6 @@ int batch_chain_wgs(int cus) { return std::min(kBatchChainWG, cus / 4); }
 int batch_chain_rw(long rows, int maxn, int cus)
 {
     return rows <= 512L * cus && maxn <= 512 * batch_chain_wgs(cus) ? 2 : 4;
-}
-
-// CUs of the current device, queried once for each device.
-constexpr int kMaxDevices = 64;
-int device_cus()
-{
-    static std::atomic<int> cus[kMaxDevices];
-    int dev = -1, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 1;
-    if (dev < kMaxDevices) n = cus[dev].load(std::memory_order_relaxed);
-    if (!n) {
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 1;
-        if (dev < kMaxDevices) cus[dev].store(n, std::memory_order_relaxed);
-    }
-    return n;
 }
 
 // Workgroups of the stencil SpMV: kStRB row blocks each (one alpha partial
@@ -4525,6 +4600,7 @@ int trlhip_ctx_destroy(trlhip_ctx *c)
         free(c);
         return 0;
     }
+    left_device(c);
     if (c->s) (void)hipStreamSynchronize(c->s);
     if (c->V) (void)hipFree(c->V);
     if (c->V32) (void)hipFree(c->V32);
@@ -4601,7 +4677,12 @@ int trlhip_ctx_create_batched(trlhip_ctx **out, int n, int ncols, int vtype, trl
         *out = c;
         return 0;
     }
-    c->cus = device_cus();
+    const int dev = current_device();
+    c->cus = device_cus(dev);
+    c->dev = dev >= 0 && dev < kMaxDevices ? dev : kMaxDevices;
+    static std::atomic<unsigned> serial{0};
+    while (!(c->serial = serial.fetch_add(1) + 1)) {
+    }
     chain_gate_times(c, kGateTicks);
     if (hipStreamCreate(&c->s) != hipSuccess) rc = TRLHIP_EHIP;
     if (!rc && hipMalloc((void **)&c->V, vbytes) != hipSuccess) rc = TRLHIP_ENOMEM;
@@ -4930,11 +5011,10 @@ static int run_phases(trlhip_ctx *c, const trlhip_csr *A, int qa, int qb, double
 // kernel (k_chain); sets the followers up as a batch's recorded chain does.
 // Returns 1 when the step ran, 0 when it must run as ordinary kernels (the
 // gate closed), or an error.
-static int run_chain(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int qb, double beta_prev,
+static int run_chain(trlhip_ctx *c, const trlhip_csr *A, int rw, int first, int qa, int qb, double beta_prev,
                      const double *beta, int jnd, int rcol, int K)
 {
     ChainArgs q{};
-    const int rw = chain_rw(c, A);
     chain_args(q, c, A, rw, first, qa, qb, beta_prev, jnd, rcol, K, c->ch_kept, c->ch_ntot);
     if (c->pend_dst == qa && rcol != c->pend_src) {
         q.x = colp<double>(c, c->pend_src);
@@ -5101,9 +5181,12 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
     int K = first ? 1 : std::max(1, std::min(c->ch_budget, kChainMax));
     c->ch_budget = 0;
     while (K > 1 && (!valid_col(c, rcol + K - 1) || jnd + K - 1 > c->ncols)) --K;
-    if (chain_form(qa, jnd, rcol) && chain_fits(c, A, jnd)) {
+    StepOnDevice on(c);
+    const int rw = chain_form(qa, jnd, rcol) ? chain_pick(c, A, jnd, on.active) : 0;
+    if (rw && on.take(chain_wgs(c->n, rw), c->cus)) {
         while (K > 1 && jnd + K - 1 > kChainMaxCols) --K;
-        const int ran = run_chain(c, A, first, qa, qb, beta_prev, beta, jnd, rcol, K);
+        const int ran = run_chain(c, A, rw, first, qa, qb, beta_prev, beta, jnd, rcol, K);
+        on.give();
         if (ran < 0) return ran;
         if (ran) {
             const volatile double *hr = c->hres;
@@ -5114,7 +5197,11 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
             return 0;
         }
     }
-    if (K > 1 && phases_fit(c, A)) {
+    // beside other solves a wait after every step lets their kernels in: 8
+    // threads, 350^2 sites, 8.0 ms a solve against 8.6 with queued steps, 500^2
+    // 13.9 against 14.7; complex ones with one other still gain (20^3 sites
+    // 10.8 against 11.2)
+    if (K > 1 && on.active <= c->E && phases_fit(c, A)) {
         if (int rc = run_phases(c, A, qa, qb, beta_prev, jnd, rcol, std::min(K, kPhaseChain))) return rc;
         const volatile double *hr = c->hres;
         out[0] = hr[S_ALPHA];
@@ -5183,11 +5270,12 @@ int trlhip_step_cgs(trlhip_ctx *c, const trlhip_csr *A, int first, int qa, int q
     return 0;
 }
 
-int trlhip_chain_rule(int n, int kind, int mixed, int nb, int max_blk_nnz, int jnd, int cus, int *wgs)
+int trlhip_chain_rule(int n, int kind, int mixed, int nb, int max_blk_nnz, int jnd, int cus, int active,
+                      int *wgs)
 {
-    const int rw = chain_rw(kind, n, mixed != 0, cus);
-    if (wgs) *wgs = chain_wgs(n, rw);
-    return chain_shape(n, kind, nb, max_blk_nnz, jnd, rw, chain_max_wgs(cus)) ? rw : 0;
+    const int rw = chain_pick(n, kind, mixed != 0, nb, max_blk_nnz, jnd, cus, active);
+    if (wgs) *wgs = rw ? chain_wgs(n, rw) : 0;
+    return rw;
 }
 
 int trlhip_ctx_chain_gate(trlhip_ctx *c, unsigned long long ticks, unsigned long long hold)
@@ -5203,6 +5291,14 @@ int trlhip_ctx_chain_counts(const trlhip_ctx *c, long *ran, long *closed)
     if (!c || !ran || !closed) return TRLHIP_EINVAL;
     *ran = c->chain_ran;
     *closed = c->chain_closed;
+    return 0;
+}
+
+int trlhip_device_load(int dev, int *steps, int *wgs)
+{
+    if (dev < 0 || dev >= kMaxDevices || !steps || !wgs) return TRLHIP_EINVAL;
+    *steps = g_load[dev].steps.load();
+    *wgs = g_load[dev].wgs.load();
     return 0;
 }
 
@@ -5557,7 +5653,7 @@ int trlhip_batch_create_on(trlhip_batch **out, trlhip_batch *share)
         delete b;
         return TRLHIP_EHIP;
     }
-    b->cus = device_cus();
+    b->cus = device_cus(current_device());
     *out = b;
     return 0;
 }

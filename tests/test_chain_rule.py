@@ -6,9 +6,10 @@ import pytest
 from nutrlan_amd import trlan as T
 
 
-def rule(n, kind, cus, nb=None, nnz=1000, jnd=20, mixed=0):
+def rule(n, kind, cus, nb=None, nnz=1000, jnd=20, mixed=0, active=1):
     wgs = ctypes.c_int()
-    rw = T.lib().trlhip_chain_rule(n, kind, mixed, -(-n // 256) if nb is None else nb, nnz, jnd, cus, ctypes.byref(wgs))
+    rw = T.lib().trlhip_chain_rule(n, kind, mixed, -(-n // 256) if nb is None else nb, nnz, jnd, cus, active,
+                                   ctypes.byref(wgs))
     return rw, wgs.value
 
 
@@ -32,6 +33,7 @@ def test_workgroups_fit_the_device(kind, cus, mixed):
         if rw:
             taken += 1
             assert wgs * 256 * rw >= n and wgs <= min(cus, 256)
+            assert rule(n, kind, cus, mixed=mixed, active=1) == (rw, wgs)
         else:
             assert -(-n // (512 if kind > -2 else 1024)) > min(cus, 256)
     assert taken
@@ -43,6 +45,28 @@ def test_row_waves():
         assert rule(65536, kind, 256, mixed=1) == (2, 128) and rule(65537, kind, 256, mixed=1) == (4, 65)
         assert rule(20000, kind, 32) == (4, 20) and rule(32769, kind, 32)[0] == 0
     assert rule(131072, 0, 256, mixed=1) == (2, 256)
+
+
+@pytest.mark.parametrize("mixed", [0, 1])
+def test_share_beside_others(mixed):
+    """Beside others a chain takes its share of the CUs, 4 row waves if it
+    needs them, or up to a quarter of the CUs."""
+    assert rule(62500, -2, 256, mixed=mixed) == (2, 123)
+    assert rule(62500, -2, 256, mixed=mixed, active=2) == (2, 123)
+    assert rule(62500, -2, 256, mixed=mixed, active=3) == (4, 62)
+    assert rule(62500, -2, 256, mixed=mixed, active=16) == (4, 62)
+    assert rule(65537, -2, 256, mixed=mixed, active=16)[0] == 0
+    assert rule(122500, -2, 256, mixed=mixed, active=2) == (4, 120)
+    assert rule(122500, -2, 256, mixed=mixed, active=3)[0] == 0
+    assert rule(10000, -2, 256, mixed=mixed, active=8) == (2, 20)
+    assert rule(10000, -2, 256, mixed=mixed, active=16) == (4, 10)
+    assert rule(32768, 0, 256, mixed=mixed, active=16) == (2, 64)
+    assert rule(32769, 0, 256, mixed=mixed, active=4)[0] == 0
+    for cus in (8, 32, 256):
+        for active in (2, 3, 5, 9, 100):
+            for n in (300, 5000, 20000, 40000, 100000, 200000):
+                rw, wgs = rule(n, -2, cus, mixed=mixed, active=active)
+                assert wgs <= max(cus // active, cus // 4)
 
 
 def test_batch_chains_scale_with_the_device():

@@ -8,6 +8,7 @@ with several solves on the device at once.
 A batch too large for chains runs phase by phase, so each solve is compared
 with itself in a batch beside operators that fill it up; the kernel statistics
 say which kernels ran."""
+import ctypes
 import threading
 
 import numpy as np
@@ -149,6 +150,9 @@ def test_chain_concurrent_solves(gpu_lib):
         t.start()
     for t in th:
         t.join()
+    steps, wgs = ctypes.c_int(-1), ctypes.c_int(-1)
+    assert T.lib().trlhip_device_load(0, ctypes.byref(steps), ctypes.byref(wgs)) == 0
+    assert (steps.value, wgs.value) == (0, 0)  # what they had taken is given back
     for A in ops:
         A.close()
     for a, b in zip(alone, got):
