@@ -4985,7 +4985,7 @@ static bool phases_fit(const trlhip_ctx *c, const trlhip_csr *A)
 // waits once per chain instead of once per step.
 static int run_phases(trlhip_ctx *c, const trlhip_csr *A, int qa, int qb, double beta_prev, int jnd, int rcol,
                       int K)
-{
+try {
     BatchStep st{c, A, 0, qa, qb, rcol, jnd, beta_prev, 0, 1.0, -1, 0, 0, 1, c->ch_kept, c->ch_ntot};
     if (c->pend_dst == qa && rcol != c->pend_src) {
         st.fuse = 1;
@@ -5005,6 +5005,8 @@ static int run_phases(trlhip_ctx *c, const trlhip_csr *A, int qa, int qb, double
     TRY(hipMemcpyAsync(c->dops, c->hops, P.total, hipMemcpyHostToDevice, c->s));
     if (int rc = steps_launch(c->s, P, c->hops, c->dops)) return rc;
     return ctx_wait(c);
+} catch (const std::bad_alloc &) {
+    return TRLHIP_ENOMEM;
 }
 
 // Runs a step and up to K - 1 followers of a single real solve as one
