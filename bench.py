@@ -50,27 +50,32 @@ def kernel_names(T, path, A=None):
     """Device kernel(s) behind each timed kernel class of a solver path, as
     rocprofv3 names the dispatches (the projection's columns per block come
     from the library's current tile setting; the SpMV from operator A's
-    format: column panels run two kernels per product, joined by '+')."""
+    format: column panels run two kernels per product, joined by '+', and
+    their steps one at a time).  Other solves queue their steps (kb_*, complex
+    kbz_*); only a cycle's first step runs as the k_* kernels."""
     cb64, cb32 = T.proj_tiles_get()
+    n = A.n if A is not None else 1 << 30
+    wide = n <= 262144  # updates of 1024-thread blocks
     if path == "complex":
-        return {"proj": "k_proj<double, double, 2, 4, 4>", "update": "k_update<double, double, 2, 4>",
-                "spmv": "k_spmv<double, double, 2, true>"}
+        return {"proj": "kbz_proj", "update": "kb_update_wide<double, 2>" if wide else "kbz_update",
+                "spmv": "kbz_spmv"}
     vs, cb = ("float", cb32) if path == "mixed" else ("double", cb64)
     # real operators up to 2^20 rows: the recurrence runs fused with the
-    # first projection (k_recproj, over the FP32 shadow or the FP64 basis),
-    # timed as the projection
-    fused = A is not None and A.n <= 1 << 20
-    spmv = "k_spmv<double, double, 1, true>"
+    # first projection (over the FP32 shadow or the FP64 basis), timed as the
+    # projection
+    fused = n <= 1 << 20
     if A is not None and A.paneled:
-        spmv = "k_spmv_panel<true>+k_spmv_panel_rows<true>"
-    elif A is not None and A.stencil[0]:
-        # up to 2048 row blocks of at most 256 rows: four row blocks per workgroup
-        D, L = A.stencil
-        spmv = f"k_spmv_st_rb<{D}, 4>" if L ** D <= 2048 * 256 else f"k_spmv_st<{D}, true>"
-    elif A is not None and A.packed:
-        spmv = "k_spmv_pk<true>"
-    return {"proj": f"k_recproj<{cb}, {vs}>" if fused else f"k_proj<{vs}, double, 1, {cb}, 4>",
-            "update": f"k_update<{vs}, double, 1, 4>", "spmv": spmv}
+        return {"proj": f"k_recproj<{cb}, {vs}>" if fused else f"k_proj<{vs}, double, 1, {cb}, 4>",
+                "update": f"k_update_wide<{vs}, 1>" if wide else f"k_update<{vs}, double, 1, 4, false>",
+                "spmv": "k_spmv_panel<true>+k_spmv_panel_rows<true>"}
+    D = A.stencil[0] if A is not None else 0
+    packed = A is not None and A.packed
+    spmv = f"kb_spmv_st<{D}>" if D else "kb_spmv_pk" if packed else "kb_spmv_stream"
+    kind = -D if D else -1 if packed else 0
+    rw = T.lib().trlhip_chain_rule(n, kind, int(path == "mixed"), 1, 1, 1, 256, 1, None)
+    names = {"proj": f"kb_recproj<{cb}, {vs}>" if fused else f"kb_proj<{vs}, {cb}>",
+             "update": f"kb_update_wide<{vs}, 1>" if wide else f"kb_update<{vs}>", "spmv": spmv}
+    return dict(names, chain=f"k_chain<{rw}, {kind}, {vs}>") if rw else names
 
 
 def calibration_copy(T, n):
