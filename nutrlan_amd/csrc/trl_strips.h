@@ -107,7 +107,8 @@ inline int dw_rows(int nimg, int h, int w)
 
 inline Geo geo_of(int nimg, int h, int w, int rows)
 {
-    return Geo{nimg, h, w, (long)nimg * h * w, rows, strip_images(h, w), conv_tasks(nimg, h, w, rows), dw_rows(nimg, h, w)};
+    return Geo{nimg, h, w, (long)nimg * h * w, rows, strip_images(h, w), conv_tasks(nimg, h, w, rows),
+               dw_rows(nimg, h, w)};
 }
 
 struct DwStrip {

@@ -2399,13 +2399,13 @@ void chain_retry(trlhip_ctx *c)
 bool chain_form(int qa, int jnd, int rcol) { return qa == jnd - 1 && rcol == jnd; }
 
 // A batch's launch runs its steps as chains (kb_chain) while the solves that
-// fit hold at most kBatchChainRows rows together (on 256 CUs).  The device holds 262,144
-// rows of a chain kernel at once (1024 a workgroup, one workgroup per CU) and
-// steps them in about 14 us; the phase kernels take 25 us and 40 more per
-// million rows.  Batches with the limit at 0, 300,000, 600,000 and 1,500,000:
-// 40 lattices of 48-160 61.2, 44.1, 44.8, 44.5 ms; 16 of 100-220, mixed,
-// 56.5, 39.9, 39.8, 37.8; 90 of 60-180 84.8, 77.5, 77.6, 79.6; 192 of 64-256,
-// mixed, 183, 170, 170, 174 (whose later rounds fit).
+// fit hold at most kBatchChainRows rows together (on 256 CUs).  The device
+// holds 262,144 rows of a chain kernel at once (1024 a workgroup, one
+// workgroup per CU) and steps them in about 14 us; the phase kernels take 25
+// us and 40 more per million rows.  Batches with the limit at 0, 300,000,
+// 600,000 and 1,500,000: 40 lattices of 48-160 61.2, 44.1, 44.8, 44.5 ms; 16
+// of 100-220, mixed, 56.5, 39.9, 39.8, 37.8; 90 of 60-180 84.8, 77.5, 77.6,
+// 79.6; 192 of 64-256, mixed, 183, 170, 170, 174 (whose later rounds fit).
 constexpr long kBatchChainRows = 600000;
 constexpr int kChainShut = 32;     // the launch's shut word: in the first group's ticket block
 constexpr int kBatchChainWG = 64;  // workgroups of one solve at most, and a quarter of the CUs

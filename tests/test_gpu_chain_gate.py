@@ -226,3 +226,26 @@ def test_queued_steps(gpu_lib, size, complex_):
     A.close()
     assert np.array_equal(got[0][0], got[1][0])
     assert np.array_equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("lpr", [2, 4, 8, 16, 32])
+def test_queued_steps_vector_csr(gpu_lib, lpr, mixed):
+    """The same for operators set to the vector-CSR kernel, which no chain
+    takes."""
+    T = gpu_lib
+    n, m = 3001, 17
+    A = T.Csr(*W.random_sym_csr(n, seed=n), mixed=mixed)
+    A.set_spmv(lpr)
+    x0 = W.start_vector(n, seed=1)
+    coef = np.random.default_rng(2).standard_normal(m) * 0.1
+    got = []
+    for steps in (1, 6):
+        print(f"lpr={lpr} mixed={mixed} steps={steps}", flush=True)
+        c = T.Ctx(n, m + 8, mixed=mixed)
+        got.append(lanczos(c, A, n, m, steps, x0 / np.linalg.norm(x0), coef))
+        assert counts(T, c) == (0, 0)
+        c.close()
+    A.close()
+    assert np.array_equal(got[0][0], got[1][0])
+    assert np.array_equal(got[0][1], got[1][1])
