@@ -486,15 +486,13 @@ __global__ __launch_bounds__(NB) void k_bwd32(Geo g, const bf16_t *__restrict__ 
 // 650 us each (now 17).
 constexpr int kTr = 18;               // dwords per channel: 36 pixels
 static_assert(kDwWaves == kDwBlocks * (NB / 64), "waves of the gradient kernels");
-// Partials of the four layers: a row per block (layers 3 and 2), per wave
-// (4 and 1), and where each starts.  They are FP64: the sum over the waves'
-// FP32 accumulators is rounded once, at its end.  Blocks without a strip are
-// not launched.
+// Partials of the four layers, a row per block, and where each starts.  They
+// are FP64: the sum over the waves' FP32 accumulators is rounded once, at its
+// end.  Blocks without a strip are not launched.
 constexpr int kRowMid = C * T * C + C, kRowEdge = C * T + C;
 constexpr long kPart3 = 0, kPart2 = kPart3 + (long)kDwBlocks * kRowMid,
                kPart4 = kPart2 + (long)kDwBlocks * kRowMid,
-               kPart1 = kPart4 + (long)kDwBlocks * (NB / 64) * kRowEdge,
-               kPartCount = kPart1 + (long)kDwBlocks * (NB / 64) * kRowEdge;
+               kPart1 = kPart4 + (long)kDwBlocks * kRowEdge, kPartCount = kPart1 + (long)kDwBlocks * kRowEdge;
 
 // Column x0 + p of a row of w, periodic one pixel beyond either end; further
 // out (a ragged strip's unused pixels) any column.
@@ -531,7 +529,7 @@ __device__ __forceinline__ bf16x8 frag(const uint32_t d[4])
 // channel and shifts them by one for the left and right taps.  The block's
 // partial (co, t, ci) and bias sums (a product with ones), its four waves
 // added in FP64, go to part[blockIdx] in FP64 (38 MB for 256 blocks, against
-// 19 in FP32: 128 images of 64 x 64 475 -> 483 us a forward and backward).
+// 19 in FP32, 0.8 us of the kernel's 18.8 at 64 images of 64 x 64).
 __global__ __launch_bounds__(NB) void k_dw32(Geo g, const bf16_t *__restrict__ dy,
                                              const bf16_t *__restrict__ x, double *__restrict__ part)
 {
@@ -689,8 +687,8 @@ __global__ __launch_bounds__(NB) void k_dw32(Geo g, const bf16_t *__restrict__ d
 //   (column 9: ones).
 // Layer 4 (LAST): v = a3, u = dO:
 //   dW4[t][ci] = sum_p a3[p][ci] dO[nbr(p,-t)], db4 = sum_p dO[p] in FP32.
-// The wave's partial goes to part[4 blockIdx + wave], C T + C values in the
-// parameters' order.
+// The block's partial, its four waves added in FP64, goes to part[blockIdx],
+// C T + C values in the parameters' order.
 template <bool LAST>
 __global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict__ v,
                                                 const float *__restrict__ u, double *__restrict__ part)
@@ -756,19 +754,27 @@ __global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict_
             __builtin_amdgcn_wave_barrier();
         }
     }
-    double *out = part + ((long)blockIdx.x * (NB / 64) + wv) * NV;
+    static_assert(sizeof(lds[0]) >= NV * sizeof(float), "a wave's sums in its part of the LDS");
+    uint32_t *out = lds[wv];
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int ch = 16 * mt + 4 * kq + i;
-            if (m < T) out[LAST ? m * C + ch : ch * T + m] = acc[mt][i];
-            if (!LAST && m == T) out[C * T + ch] = acc[mt][i];
+            if (m < T) out[LAST ? m * C + ch : ch * T + m] = __float_as_uint(acc[mt][i]);
+            if (!LAST && m == T) out[C * T + ch] = __float_as_uint(acc[mt][i]);
         }
     if (LAST) {
         bsum += __shfl_xor(bsum, 16);
         bsum += __shfl_xor(bsum, 32);
-        if (lane == 4) out[C * T] = bsum;
+        if (lane == 4) out[C * T] = __float_as_uint(bsum);
+    }
+    __syncthreads();
+    for (int j = threadIdx.x; j < (LAST ? C * T + 1 : NV); j += NB) {
+        double t = 0.0;
+#pragma unroll
+        for (int w = 0; w < NB / 64; ++w) t += __uint_as_float(lds[w][j]);
+        part[(long)blockIdx.x * NV + j] = t;
     }
 }
 
@@ -776,11 +782,12 @@ __global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict_
 // launch: a block takes 32 columns of a layer, its 32 groups of threads every
 // 32nd row, all their loads in flight, and the groups' sums are added in
 // order.  (A launch per layer: 24 us and the gaps between them, of 340 for 64
-// images of 64 x 64; 38 MB with 16 groups of 64 columns: 14 us, now 10.3.)
+// images of 64 x 64; 39 MB with 16 groups of 64 columns, and a row per wave of
+// the first and last layers: 14.0 us, now 7.1.)
 constexpr int kRedGroups = 32, kRedCols = 32;
 struct RedSeg {
     long part;
-    int rows, len, stride, out, blk0;  // rows a block of the gradient kernel leaves
+    int len, stride, out, blk0;
 };
 struct RedArgs {
     RedSeg s[4];
@@ -789,10 +796,10 @@ struct RedArgs {
 constexpr RedArgs red_args()
 {
     RedArgs a{};
-    a.s[0] = {kPart3, 1, kRowMid, kRowMid, OW3, 0};
-    a.s[1] = {kPart2, 1, kRowMid, kRowMid, OW2, 0};
-    a.s[2] = {kPart4, NB / 64, C * T + 1, kRowEdge, OW4, 0};  // layer 4 has one bias
-    a.s[3] = {kPart1, NB / 64, kRowEdge, kRowEdge, OW1, 0};
+    a.s[0] = {kPart3, kRowMid, kRowMid, OW3, 0};
+    a.s[1] = {kPart2, kRowMid, kRowMid, OW2, 0};
+    a.s[2] = {kPart4, C * T + 1, kRowEdge, OW4, 0};  // layer 4 has one bias
+    a.s[3] = {kPart1, kRowEdge, kRowEdge, OW1, 0};
     for (int i = 0; i < 4; ++i) {
         a.s[i].blk0 = a.blocks;
         a.blocks += (a.s[i].len + kRedCols - 1) / kRedCols;
@@ -814,7 +821,7 @@ __global__ __launch_bounds__(kRedCols * kRedGroups) void k_reduce(const double *
     if (j < q.len) {
         const double *p = part + q.part + j;
 #pragma unroll 8
-        for (int b = gr; b < q.rows * dwb; b += kRedGroups) s += p[(long)b * q.stride];
+        for (int b = gr; b < dwb; b += kRedGroups) s += p[(long)b * q.stride];
     }
     sm[gr][c] = s;
     __syncthreads();
