@@ -7,9 +7,12 @@ struct Geo {
     int nimg, h, w;
     long np;   // pixels
     // a convolution's wave: the rows it walks (conv_rows), the images side by
-    // side (strip_images); how many there are
-    int rows, ni;
+    // side (strip_images); strips across, waves for these images, all waves.
+    // Formed on the host: divisions in the kernels' first microsecond show at
+    // a few images
+    int rows, ni, ns, per;
     long tasks;
+    unsigned recip;  // a lane's image is lane * recip >> 16
     int dwr;   // rows of a weight-gradient strip (dw_rows)
 };
 
@@ -33,6 +36,12 @@ inline long conv_tasks(int nimg, int h, int w, int rows)
     return (long)((nimg + ni - 1) / ni) * strips_of(w) * segs_of(h, rows);
 }
 
+// task / per, in 32 bits where it fits.
+__host__ __device__ inline int group_of_task(long task, int per)
+{
+    return task <= 0x7fffffffL ? (int)task / per : (int)(task / per);
+}
+
 // A lane's part of a wave's strip: pixel (y, its column) is base + y w + x,
 // its neighbours' columns (periodic) are xc.  Its image's offset from the
 // wave's first is part of x and xc, so that base stays the wave's.
@@ -45,13 +54,13 @@ struct Strip {
 __host__ __device__ inline bool strip_of(const Geo &g, long task, int lane, Strip &s)
 {
     if (task >= g.tasks) return false;
-    const int ns = strips_of(g.w), per = ns * segs_of(g.h, g.rows), ni = g.ni;
-    const int grp = (int)(task / per), r = (int)(task - (long)grp * per);
+    const int ns = g.ns, ni = g.ni;
+    const int grp = group_of_task(task, g.per), r = (int)(task - (long)grp * g.per);
     const int seg = r / ns, strip = r - seg * ns;
     int x = strip * kStrip + lane, off = 0;
     s.ok = x < g.w;
     if (ni > 1) {
-        const int i = lane / g.w, last = g.nimg - 1 - grp * ni;
+        const int i = (int)(lane * g.recip >> 16), last = g.nimg - 1 - grp * ni;
         x = lane - i * g.w;
         s.ok = i < ni && i <= last;
         off = (i < last ? i : last) * g.h * g.w;
@@ -82,10 +91,10 @@ __host__ __device__ inline long dw_tasks(const Geo &g)
 
 // Strip height.  A strip of r rows loads r + 2 rows of inputs, but a wave's
 // FP32 sums are to run over no more pixels than an even split gives them (32
-// up to 1,024 strips of one row), but for an eighth: of the heights that keep
+// up to 1,024 strips of one row), but for a quarter: of the heights that keep
 // to that, the one with the fewest rows to load for the busiest wave.  Forward
 // and backward of 1, 8 and 32 images of 64 x 64 with 8-row strips throughout:
-// 211, 200 and 256 us, so 174, 171 and 240 (more waves).
+// 211, 200 and 256 us, so 175, 168 and 236 (more waves).
 __host__ __device__ inline long dw_wave_strips(int nimg, int h, int w, int r)
 {
     return ((long)nimg * dw_strips(w) * dw_segs(h, r) + kDwWaves - 1) / kDwWaves;
@@ -97,7 +106,7 @@ inline int dw_rows(int nimg, int h, int w)
     long least = 3 * even;
     for (int r = 2; r <= kDwRows && r <= h; ++r) {
         const long n = dw_wave_strips(nimg, h, w, r);
-        if (n * r <= even + even / 8 && n * (r + 2) < least) {
+        if (n * r <= even + even / 4 && n * (r + 2) < least) {
             least = n * (r + 2);
             best = r;
         }
@@ -107,8 +116,9 @@ inline int dw_rows(int nimg, int h, int w)
 
 inline Geo geo_of(int nimg, int h, int w, int rows)
 {
-    return Geo{nimg, h, w, (long)nimg * h * w, rows, strip_images(h, w), conv_tasks(nimg, h, w, rows),
-               dw_rows(nimg, h, w)};
+    const int ns = strips_of(w);
+    return Geo{nimg, h, w, (long)nimg * h * w, rows, strip_images(h, w), ns, ns * segs_of(h, rows),
+               conv_tasks(nimg, h, w, rows), 65536u / (unsigned)w + 1u, dw_rows(nimg, h, w)};
 }
 
 struct DwStrip {
@@ -119,7 +129,7 @@ struct DwStrip {
 __host__ __device__ inline DwStrip dw_strip(const Geo &g, long task)
 {
     const int ns = dw_strips(g.w), sw = dw_width(g.w), per = ns * dw_segs(g.h, g.dwr);
-    const int img = (int)(task / per), r = (int)(task - (long)img * per);
+    const int img = group_of_task(task, per), r = (int)(task - (long)img * per);
     const int seg = r / ns;
     DwStrip s;
     s.base = (long)img * g.h * g.w;
