@@ -686,7 +686,8 @@ __global__ __launch_bounds__(NB) void k_dw32(Geo g, const bf16_t *__restrict__ d
 //   dW1[co][t] = sum_p dA1[p][co] x[nbr(p,t)], db1[co] = sum_p dA1[p][co]
 //   (column 9: ones).
 // Layer 4 (LAST): v = a3, u = dO:
-//   dW4[t][ci] = sum_p a3[p][ci] dO[nbr(p,-t)], db4 = sum_p dO[p] in FP32.
+//   dW4[t][ci] = sum_p a3[p][ci] dO[nbr(p,-t)], db4 = sum_p dO[p] in FP64
+//   (dO's values nearly cancel).
 // The block's partial, its four waves added in FP64, goes to part[blockIdx],
 // C T + C values in the parameters' order.
 template <bool LAST>
@@ -695,6 +696,7 @@ __global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict_
 {
     constexpr int NV = C * T + C;
     __shared__ __align__(16) uint32_t lds[NB / 64][C * kTr];
+    __shared__ double bs[NB / 64];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int m = lane & 15, kq = lane >> 4;
     const int pp = lane >> 2, cg = lane & 3;
@@ -703,7 +705,7 @@ __global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict_
     uint32_t *tv = lds[wv];
     const f4 zero = {0.f, 0.f, 0.f, 0.f};
     f4 acc[2] = {zero, zero};
-    float bsum = 0.f;
+    double bsum = 0.0;
     const uint4 z4 = {0, 0, 0, 0};
     const long nt_ = dw_tasks(g);
     for (long task = (long)blockIdx.x * (NB / 64) + wv; task < nt_; task += (long)gridDim.x * (NB / 64)) {
@@ -767,13 +769,13 @@ __global__ __launch_bounds__(NB) void k_dw_edge(Geo g, const bf16_t *__restrict_
     if (LAST) {
         bsum += __shfl_xor(bsum, 16);
         bsum += __shfl_xor(bsum, 32);
-        if (lane == 4) out[C * T] = __float_as_uint(bsum);
+        if (lane == 4) bs[wv] = bsum;
     }
     __syncthreads();
     for (int j = threadIdx.x; j < (LAST ? C * T + 1 : NV); j += NB) {
         double t = 0.0;
 #pragma unroll
-        for (int w = 0; w < NB / 64; ++w) t += __uint_as_float(lds[w][j]);
+        for (int w = 0; w < NB / 64; ++w) t += LAST && j == C * T ? bs[w] : (double)__uint_as_float(lds[w][j]);
         part[(long)blockIdx.x * NV + j] = t;
     }
 }

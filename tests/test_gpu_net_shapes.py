@@ -91,3 +91,22 @@ def test_narrow_images(gpu_lib, shape):
     for i in range(len(x)):
         assert np.array_equal(net.forward(x[i:i + 1])[0], y[i]), i
     net.close()
+
+
+@pytest.mark.parametrize("shape", [(1, 8, 8), (1, 20, 20), (6, 6, 5), (3, 50, 71), (1, 64, 64), (40, 64, 33)])
+def test_last_bias_gradient(gpu_lib, shape):
+    """The last layer's bias sums loss gradients that nearly cancel, in FP64:
+    the result is rounded once (2^-24), and one in 10^3 of the summands may
+    differ by a rounding from those formed here."""
+    for k in range(4):
+        net = learned.load_net()
+        rng = np.random.default_rng(100 * shape[0] + k)
+        x = rng.uniform(-1, 1, shape).astype(np.float32)
+        t = np.abs(rng.standard_normal(shape)).astype(np.float32)
+        o, tg = net.forward(x).astype(np.float64), t.astype(np.float64)
+        ot, oo, tt = [(u * v).sum((1, 2), keepdims=True) for u, v in ((o, tg), (o, o), (tg, tg))]
+        c = ot * ot / (oo * tt)
+        do = (2.0 / len(x) * (c * o / oo - ot * tg / (oo * tt))).astype(np.float32).astype(np.float64)
+        g = net.loss_grad(x, t)[1][-1]
+        assert abs(g - do.sum()) <= 2.0 ** -24 * (abs(do.sum()) + 1e-3 * np.abs(do).sum()), (k, g, do.sum())
+        net.close()
